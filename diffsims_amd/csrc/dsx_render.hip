@@ -775,8 +775,6 @@ constexpr int kPlanPerLane = 8;
 constexpr int kPlanMax = kPlanPerLane * kWave;  // listed spots per pattern
 constexpr int kPlanMaxSide = 1024;              // 10-bit pixel coordinates in the sort key
 constexpr int kBandThreads = 256;
-constexpr int kBandVec = 2;                              // float4 stores per thread
-constexpr int kBandPix = 4 * kBandVec * kBandThreads;    // pixels per band
 // patterns per plan/writer round: the plan's hand-over for 16,384 patterns
 // stays in the last-level cache while the writer reads it (render stage of
 // 200,000 library patterns: 8.50 ms with 16,384, 8.57 with 12,288 or 32,768,
@@ -1145,9 +1143,26 @@ __global__ __launch_bounds__(kPlanThreads) void render_plan_kernel(BandArgs b) {
   }
 }
 
-template <int kR>
+// Pixels per band: 2,048 (two 16-byte stores per thread) up to R = 5, 4,096
+// for wider taps.  A band of B rows splats the spots of B + 2R rows, so wide
+// taps make the splat's VALU work, not the stores, bound small bands.
+// Render stage of 12,000 x 232 x 200, 235 spots each, with 2,048 / 4,096
+// pixels: R = 4 402 / 461 us, R = 5 458 / 468, R = 6 589 / 472, R = 7
+// 672 / 533, R = 8 782 / 618.
+__host__ __device__ constexpr int band_vec(int R) { return R <= 5 ? 2 : 4; }
+__host__ __device__ constexpr int band_pix(int R) { return 4 * band_vec(R) * kBandThreads; }
+
+// kAligned: every row is a whole number of 16-byte vectors.  Otherwise the
+// band's pixels sit in LDS at the offset their first pixel has within its
+// 16-byte vector in memory (`shift`), so the vectors of both line up and only
+// the band's first and last vector can be partial (one kernel for both cost
+// the library's aligned patterns 6 %: 487 -> 519 us per round of 16,384).
+// Odd widths went through render_kernel before (12,000 x 231 x 201, R = 7:
+// 730 us there; 62 us plan and 425 us writer here, 5.3 TB/s).
+template <int kR, bool kAligned>
 __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
-  __shared__ __align__(16) racc_t s_acc[kBandPix];
+  constexpr int kVec = band_vec(kR), kPix = band_pix(kR);
+  __shared__ __align__(16) racc_t s_acc[kPix + (kAligned ? 0 : 4)];
   __shared__ int2 s_ent[kPlanMax];
   __shared__ float s_tp[kR + 1];
   const RenderArgs &a = b.r;
@@ -1165,7 +1180,10 @@ __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
   const int H = a.H, W = a.W;
   const int y0 = bb * b.band_rows;
   const int y1 = min(H, y0 + b.band_rows) - 1;  // last row of the band
-  const int nvec = (y1 - y0 + 1) * W / 4;
+  float *first = a.out + static_cast<size_t>(p) * H * W + static_cast<size_t>(y0) * W;
+  const int shift = kAligned ? 0 : static_cast<int>(reinterpret_cast<uintptr_t>(first) >> 2) & 3;
+  const int last = shift + (y1 - y0 + 1) * W;  // LDS words [shift, last) are the band
+  const int nvec = kAligned ? last / 4 : (last + 3) / 4;
   // one scalar round: the pattern's header and the band's window of the
   // row-sorted list (rows y0 - R .. y1 + R)
   const int *rec = b.rec + static_cast<size_t>(pl) * b.rec_ints;
@@ -1193,7 +1211,7 @@ __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
                                              : reflect_weight3(x, xi, W, R, s_tp);
     const float iws = __int_as_float(en.y) * wx * scale;
     const int ya = max(yi - R, y0), yb = min(yi + R, y1);
-    racc_t *col = s_acc + (x - y0 * W);
+    racc_t *col = s_acc + (x - y0 * W + shift);
     if (yi >= R && yi + R < H) {
 #pragma unroll
       for (int dd = -R; dd <= R; ++dd) {
@@ -1205,17 +1223,27 @@ __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
     }
   }
   lds_sync();
-  float4 *dst = reinterpret_cast<float4 *>(a.out + static_cast<size_t>(p) * H * W + static_cast<size_t>(y0) * W);
+  float *dst = first - shift;  // words outside [shift, last) are not touched
+  auto store = [&](int v) {
+    const int4 u = reinterpret_cast<const int4 *>(s_acc)[v];
+    const float4 o = make_float4(static_cast<float>(u.x) * out_scale, static_cast<float>(u.y) * out_scale,
+                                 static_cast<float>(u.z) * out_scale, static_cast<float>(u.w) * out_scale);
+    if (kAligned || (4 * v >= shift && 4 * v + 4 <= last)) {
+      store_nt(o, reinterpret_cast<float4 *>(dst) + v);
+    } else {
+      const float f[4] = {o.x, o.y, o.z, o.w};
 #pragma unroll
-  for (int k = 0; k < kBandVec; ++k) {
-    const int v = tid + k * kBandThreads;
-    if (v < nvec) {
-      const int4 u = reinterpret_cast<const int4 *>(s_acc)[v];
-      store_nt(make_float4(static_cast<float>(u.x) * out_scale, static_cast<float>(u.y) * out_scale,
-                           static_cast<float>(u.z) * out_scale, static_cast<float>(u.w) * out_scale),
-               dst + v);
+      for (int k = 0; k < 4; ++k)
+        if (4 * v + k >= shift && 4 * v + k < last) dst[4 * v + k] = f[k];
     }
+  };
+#pragma unroll
+  for (int k = 0; k < kVec; ++k) {
+    const int v = tid + k * kBandThreads;
+    if (v < nvec) store(v);
   }
+  // a shifted band of kPix pixels has one vector more
+  if (!kAligned && tid == 0 && nvec > kVec * kBandThreads) store(kVec * kBandThreads);
 }
 
 // ---------------------------------------------------------------------------
@@ -2079,17 +2107,17 @@ static int render_common(int mode, const float *spot_d, const int *count_d, int 
 
 // ---- band renderer: host side ----------------------------------------------
 
-static void band_shape(int H, int W, int &band_rows, int &nb) {
-  band_rows = std::max(1, std::min(H, kBandPix / std::max(1, W)));
+static void band_shape(int R, int H, int W, int &band_rows, int &nb) {
+  band_rows = std::max(1, std::min(H, band_pix(R) / std::max(1, W)));
   nb = (H + band_rows - 1) / band_rows;
 }
 
 // Shapes the plan and the band writer take: tap radius 1..8 below both
-// pattern sides, rows of whole float4 vectors, sides of at most 1024 pixels
-// (10-bit coordinates in the plan's sort key), tile bounds in the plan's LDS.
+// pattern sides, sides of at most 1024 pixels (10-bit coordinates in the
+// plan's sort key), tile bounds in the plan's LDS.
 static bool band_fits(const RenderArgs &a) {
   const int n_tiles = ((a.W + kTile - 1) / kTile) * ((a.H + kTile - 1) / kTile);
-  return a.R >= 1 && a.R <= 8 && a.R < std::min(a.H, a.W) && (a.W & 3) == 0 &&
+  return a.R >= 1 && a.R <= 8 && a.R < std::min(a.H, a.W) &&
          a.W <= kPlanMaxSide && a.H <= kPlanMaxSide && n_tiles <= kMaxTiles;
 }
 
@@ -2100,7 +2128,7 @@ static int band_rec_ints(int nb) { return (4 + 2 * nb + 3) & ~3; }
 // rounds) | per pattern of a round: header and each band's window | row-sorted spots.
 static long long band_workspace_ints(int n, int H, int W) {
   int br, nb;
-  band_shape(H, W, br, nb);
+  band_shape(1, H, W, br, nb);  // the narrowest bands
   const long long chunk = std::min(std::max(n, 1), kBandChunk);
   return band_list_ints(std::max(n, 1)) + chunk * band_rec_ints(nb) + chunk * kPlanMax * 2;
 }
@@ -2114,7 +2142,10 @@ static void launch_bands_r(const BandArgs &b, size_t plan_lds, hipStream_t st) {
   const int plan_blocks = (b.m + 8 * kPlanWaves - 1) / (8 * kPlanWaves) * 8;
   hipLaunchKernelGGL(render_plan_kernel<kR>, dim3(plan_blocks), dim3(kPlanThreads), plan_lds, st, b);
   const unsigned band_blocks = static_cast<unsigned>((b.m + 7) / 8) * 8u * static_cast<unsigned>(b.nb);
-  hipLaunchKernelGGL(render_band_kernel<kR>, dim3(band_blocks), dim3(kBandThreads), 0, st, b);
+  if ((b.r.W & 3) == 0 && (reinterpret_cast<uintptr_t>(b.r.out) & 15) == 0)
+    hipLaunchKernelGGL((render_band_kernel<kR, true>), dim3(band_blocks), dim3(kBandThreads), 0, st, b);
+  else
+    hipLaunchKernelGGL((render_band_kernel<kR, false>), dim3(band_blocks), dim3(kBandThreads), 0, st, b);
 }
 
 }  // namespace dsx
@@ -2198,15 +2229,18 @@ extern "C" int dsx_render_fast_bands(const float *spot_d, const int *count_d, in
   a.out = out_d;
   a.status = status_d;
   hipStream_t s = as_stream(stream);
-  if (!band_fits(a)) return launch_splat(kModeFast, a, bpc, s, name);
   const long long need = band_workspace_ints(n, a.H, a.W);
+  // widths that are not a multiple of 4 may come without a workspace (they
+  // needed none when only render_kernel took them)
+  const bool no_work = (a.W & 3) != 0 && (!work_d || work_ints < need);
+  if (!band_fits(a) || no_work) return launch_splat(kModeFast, a, bpc, s, name);
   if (!work_d || work_ints < need) {
     set_error("%s: workspace of %lld ints is smaller than %lld", name, work_ints, need);
     return DSX_EINVAL;
   }
   BandArgs b;
   b.r = a;
-  band_shape(a.H, a.W, b.band_rows, b.nb);
+  band_shape(a.R, a.H, a.W, b.band_rows, b.nb);
   b.ntx = (a.W + kTile - 1) / kTile;
   b.n_tiles = b.ntx * ((a.H + kTile - 1) / kTile);
   b.wave_ints = plan_wave_ints(a.H, b.n_tiles);

@@ -287,11 +287,11 @@ int dsx_render_fast(const float *spot_d, const int *count_d, int cap, int n,
  * detector_functions.py:293-300) — in two kernels: a plan kernel (one wave per
  * pattern: pixels, last write wins, the exact maximum) hands each band of
  * rows its spots through work_d, then a one-shot grid writes every band
- * (two 16-byte stores per thread).  Patterns the plan cannot hold are rendered
- * by dsx_render_fast's kernel in the same call.  Shapes outside the band
- * path (tap radius above 8 or not below both sides, width not a multiple of 4
- * or above 1024, height above 1024) run dsx_render_fast's kernel alone and
- * leave work_d unused.
+ * (two or four 16-byte stores per thread).  Patterns the plan cannot hold are
+ * rendered by dsx_render_fast's kernel in the same call.  Shapes outside the
+ * band path (tap radius above 8 or not below both sides, a side above 1024)
+ * run dsx_render_fast's kernel alone and leave work_d unused, as do widths
+ * that are not a multiple of 4 when work_d is NULL or too small.
  *   work_d : dsx_render_fast_bands_workspace_ints(n, height, width) ints
  *            (patterns are taken in rounds of at most 16,384, which reuse
  *            it in stream order); overlapping

@@ -182,11 +182,53 @@ def test_rounds_of_patterns():
 
 @pytest.mark.parametrize("shape,sigma", [((128, 128), 3.0), ((128, 130), 1.0)])
 def test_shapes_outside_the_band_path(shape, sigma):
-    # tap radius 12, and a width that is not a multiple of 4: the splat kernel alone
+    # tap radius 12: the splat kernel alone; a width that is not a multiple of 4
     print(f"bands: 50 x {shape}, sigma {sigma}", flush=True)
     spots, cnt = _spot_lists(50, 64, shape[0], shape[1], 40, seed=7)
     ref, out, st_ref, st, _ = _render_both(spots, cnt, 64, shape, sigma)
     _assert_same(ref, out, st_ref, st)
+
+
+@pytest.mark.parametrize("shape,sigma", [((37, 33), 0.3), ((61, 101), 1.25), ((231, 201), 1.7),
+                                         ((19, 1021), 2.0), ((300, 1023), 1.0), ((64, 513), 1.0)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_odd_widths_and_unaligned_output(shape, sigma, offset):
+    # rows that are not whole 16-byte vectors, and an output that starts
+    # between two of them: every pixel of the output and nothing beside it
+    import torch
+    from diffsims_amd import engine
+    H, W = shape
+    n, R = 41, int(4 * sigma + 0.5)
+    print(f"bands: {n} x {H}x{W}, sigma {sigma}, output offset {offset}", flush=True)
+    spots, cnt = _spot_lists(n, 96, H, W, 60, seed=W, edge=0.2, dup=0.05, R=R)
+    ref, out, st_ref, st, _ = _render_both(spots, cnt, 96, shape, sigma)
+    _assert_same(ref, out, st_ref, st)
+    lib, L = _lib()
+    p = engine.render_params(shape, sigma, 1.0)
+    buf = torch.full((n * H * W + 8,), -3.0, dtype=torch.float32, device="cuda")
+    view = buf[offset:offset + n * H * W]
+    ws = int(L.dsx_render_fast_bands_workspace_ints(n, H, W))
+    work = torch.empty(ws, dtype=torch.int32, device="cuda")
+    lib.check(L.dsx_render_fast_bands(lib.ptr(spots), lib.ptr(cnt), 96, n, ctypes.byref(p),
+                                      lib.ptr(work), ws, lib.ptr(view), lib.ptr(st),
+                                      lib.stream_handle(spots.device)), "dsx_render_fast_bands")
+    assert torch.equal(view.view(n, H, W), ref)
+    assert bool((buf[:offset] == -3.0).all()) and bool((buf[offset + n * H * W:] == -3.0).all())
+
+
+def test_odd_width_without_workspace():
+    # such widths need no workspace (the splat kernel alone renders them then)
+    import torch
+    from diffsims_amd import engine
+    lib, L = _lib()
+    spots, cnt = _spot_lists(20, 64, 60, 61, 40, seed=9)
+    p = engine.render_params((60, 61), 1.0, 1.0)
+    ref, _, _, st, _ = _render_both(spots, cnt, 64, (60, 61), 1.0)
+    out = torch.full_like(ref, float("nan"))
+    lib.check(L.dsx_render_fast_bands(lib.ptr(spots), lib.ptr(cnt), 64, 20, ctypes.byref(p), None,
+                                      0, lib.ptr(out), lib.ptr(st),
+                                      lib.stream_handle(spots.device)), "dsx_render_fast_bands")
+    assert torch.equal(out, ref)
 
 
 def test_workspace_query_and_rejection():
