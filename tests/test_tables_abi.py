@@ -29,7 +29,8 @@ def test_table_sizes_and_known_values():
                                          0.2356, 16.5591, 0.0914, 43.2743])
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference sources not present")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "diffsims")),
+                    reason="reference sources not present")
 @pytest.mark.parametrize("name, rel", [("lobato", "diffsims/utils/lobato_scattering_params.py"),
                                        ("xtables", "diffsims/utils/atomic_scattering_params.py")])
 def test_tables_match_reference_text(name, rel):
