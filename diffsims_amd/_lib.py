@@ -94,6 +94,9 @@ EXPORTED = (
     "dsx_render_fast_large",
     "dsx_render_fast_bands_workspace_ints",
     "dsx_render_fast_bands",
+    "dsx_render_fast_long_fits",
+    "dsx_render_fast_long_workspace_ints",
+    "dsx_render_fast_long",
     "dsx_euler_to_rt",
     "dsx_euler_to_rt_backward",
 )
@@ -212,6 +215,10 @@ _SIGS = {
     "dsx_render_fast_bands_workspace_ints": (ctypes.c_longlong, [_I, _I, _I]),
     "dsx_render_fast_bands": (_I, [_P, _P, _I, _I, ctypes.POINTER(RenderParams), _P,
                                    ctypes.c_longlong, _P, _P, _P]),
+    "dsx_render_fast_long_fits": (_I, [_I, _I, _I, _I]),
+    "dsx_render_fast_long_workspace_ints": (ctypes.c_longlong, [_I, _I, _I, _I]),
+    "dsx_render_fast_long": (_I, [_P, _P, _I, _I, ctypes.POINTER(RenderParams), _P,
+                                  ctypes.c_longlong, _P, _P, _P]),
     "dsx_euler_to_rt": (_I, [_P, _I, _P, _P]),
     "dsx_euler_to_rt_backward": (_I, [_P, _P, _I, _P, _P]),
     "dsx_render_fast_large": (_I, [_P, _P, _I, _I, ctypes.POINTER(RenderParams), _P,

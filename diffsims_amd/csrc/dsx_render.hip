@@ -785,6 +785,7 @@ struct BandArgs {
   RenderArgs r;     // spot lists, detector mapping, taps, output
   int *rec;         // per pattern: {listed, spots, scale, out_scale}, first spot of rows 0..H
   int2 *ent;        // per pattern: spots sorted by row, {(y << 16) | x, I}
+  int ent_stride;   // entries per pattern (long lists; kPlanMax otherwise)
   int *fallback;    // [0]: patterns listed, [1 + i]: their ids
   int rec_ints;     // stride of rec
   int p0, m;        // first pattern of the round, patterns in it
@@ -1143,14 +1144,286 @@ __global__ __launch_bounds__(kPlanThreads) void render_plan_kernel(BandArgs b) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Plan of long lists (more spots than render_plan_kernel's registers or the
+// splat renderer's tables hold): one block per pattern with the whole list in
+// LDS, 10 B per spot; the band writer follows.  These patterns went through
+// render_fast_large_kernel, one 1,024-thread block per CU that rebuilt and
+// filtered every strip twice with barriers between: 4,000 x 256 x 256, R = 4,
+// with 1,200 / 2,300 / 5,000 / 10,000 spots 6.8 / 6.9 / 7.2 / 7.9 ms there,
+// 0.32 / 0.51 / 1.22 / 4.0 ms here.  The plan waits on LDS and on its barriers
+// (the search for the maximum is a fifth of the stage at 2,300 spots), the
+// writer is bound by the splat's VALU instructions.
+// ---------------------------------------------------------------------------
+
+// waves sharing a list: 2,300 / 10,000 spots take 0.54 / 6.0 ms with 256
+// threads and 0.51 / 4.0 ms with 512, as fewer lists than waves fit a CU
+constexpr int kLongThreads = 512;
+constexpr int kLongWaves = kLongThreads / kWave;
+constexpr int kLongLdsBytes = 144 * 1024;  // dynamic; the static part is 12.4 KB
+// Bound units of the largest spot: 2^14 of them (every spot of the longest
+// list on one tile) stay below 2^31.
+constexpr float kLongUnits = 65536.0f;
+
+// Dynamic LDS: row starts [H + 1] | tile bounds [n_tiles] | keys (x << 16 |
+// list position) and intensities [cap each] | rows [cap shorts].
+__host__ __device__ __forceinline__ long long long_plan_bytes(int cap, int H, int n_tiles) {
+  return 4ll * (H + 1 + n_tiles) + 10ll * cap;
+}
+
+// Fixed-point term of the writer: render_kernel's truncation, or for long
+// lists, where the truncations of many terms would add up, the nearest unit
+// (the terms are non-negative).
+template <bool kLong>
+__device__ __forceinline__ int band_term(float iws, float wy) {
+  return kLong ? static_cast<int>(fmaf(iws, wy, 0.5f)) : fast_fixed(iws, wy);
+}
+
+// Largest pixel of the 16x16 tile t (at least `best`), by one wave: a splat of
+// the spots [e0, e1) of the row-sorted list whose footprint reaches it, item =
+// (spot, column), with the writer's terms, so the
+// result equals the written pixel bit for bit.
+template <int kR>
+__device__ __forceinline__ int tile_max(const RenderArgs &a, int tx, int ty, int e0, int e1,
+                                        const int *s_key, const float *s_I, const short *s_y,
+                                        const float *s_tp, float scale, int *s_tile, int *s_cq,
+                                        int lane, int best) {
+  constexpr int R = kR;
+  const int H = a.H, W = a.W;
+  const int ty0 = ty * kTile, ty1 = min(H, ty0 + kTile) - 1;
+#pragma unroll
+  for (int u = 0; u < kTile * kTile / kWave; ++u) s_tile[lane + u * kWave] = 0;
+  int ncq = 0;
+  for (int eb = e0; eb < e1; eb += kWave) {
+    const int e = eb + lane;
+    bool keep = false;
+    if (e < e1) {
+      const int xi = s_key[e] >> 16;
+      keep = s_I[e] != 0.0f && xi + R >= tx * kTile && xi - R <= tx * kTile + kTile - 1;
+    }
+    const uint64_t mk = __ballot(keep);
+    if (keep) s_cq[ncq + mask_rank(mk)] = e;
+    ncq += __popcll(mk);
+    if (ncq < kWave && eb + kWave < e1) continue;  // splat full batches and the rest
+    wave_lds_sync();
+    for (int it = lane; it < ncq * kTile; it += kWave) {
+      const int q = s_cq[it / kTile], cx = it & (kTile - 1);
+      const int x = tx * kTile + cx;
+      const int qy = s_y[q], qx = s_key[q] >> 16;
+      if (x >= W || x < qx - R || x > qx + R) continue;
+      const float iws = s_I[q] * band_weight(x, qx, W, R, s_tp) * scale;
+      int *col = s_tile + cx - ty0 * kTile;
+      if (qy >= R && qy + R < H) {
+#pragma unroll
+        for (int dd = -R; dd <= R; ++dd) {
+          const int y = qy + dd;
+          if (y >= ty0 && y <= ty1) atomicAdd(col + y * kTile, band_term<true>(iws, a.taps[dd < 0 ? -dd : dd]));
+        }
+      } else {
+        for (int y = max(ty0, qy - R); y <= min(ty1, qy + R); ++y)
+          atomicAdd(col + y * kTile, band_term<true>(iws, reflect_weight3(y, qy, H, R, s_tp)));
+      }
+    }
+    wave_lds_sync();
+    ncq = 0;
+  }
+  int lm = best;
+#pragma unroll
+  for (int u = 0; u < kTile * kTile / kWave; ++u) {
+    const int pix = lane + u * kWave;
+    if (tx * kTile + (pix & (kTile - 1)) < W && ty0 + pix / kTile <= ty1) lm = max(lm, s_tile[pix]);
+  }
+  const int m = wave_max_i(lm);
+  wave_lds_sync();  // the next tile rewrites the pixels
+  return m;
+}
+
+template <int kR>
+__global__ __launch_bounds__(kLongThreads) void render_plan_long_kernel(BandArgs b) {
+  extern __shared__ int s_long[];
+  __shared__ int s_tile[kLongWaves][kTile * kTile];
+  __shared__ int s_cq[kLongWaves][2 * kWave];
+  __shared__ float s_tp[kR + 1];
+  __shared__ float s_pm[kLongWaves];
+  __shared__ int s_n[kLongWaves], s_u[kLongWaves];
+  __shared__ int s_q, s_best;
+  const RenderArgs &a = b.r;
+  constexpr int R = kR;
+  const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
+  // pattern pl is planned on XCD pl mod 8, where its bands are rendered
+  const int pl = blockIdx.x;
+  const int p = b.p0 + pl;
+  const int H = a.H, W = a.W, ntx = b.ntx, n_tiles = b.n_tiles;
+  int *rows = s_long;
+  int *tile_u = rows + (H + 1);
+  int *s_key = tile_u + n_tiles;
+  float *s_I = reinterpret_cast<float *>(s_key + a.cap);
+  short *s_y = reinterpret_cast<short *>(s_I + a.cap);
+  int *rec = b.rec + static_cast<size_t>(pl) * b.rec_ints;
+  const int n = min(a.count[p], a.cap);
+  const float4 *sp = a.spots + static_cast<size_t>(p) * a.cap;
+  for (int t = tid; t <= H; t += kLongThreads) rows[t] = 0;
+  for (int t = tid; t < n_tiles; t += kLongThreads) tile_u[t] = 0;
+  if (tid <= R) s_tp[tid] = a.taps[tid];
+  if (tid == 0) s_q = 0x7fffffff;
+  lds_sync();
+  // ---- spots per row, row starts, the list sorted by row ------------------
+  for (int j = tid; j < n; j += kLongThreads) {
+    float X, Y;
+    if (to_pixel(sp[j], a, X, Y)) atomicAdd(&rows[min(static_cast<int>(Y), H - 1) + 1], 1);
+  }
+  lds_sync();
+  if (wid == 0) {  // rows[1 + y] becomes the start of row y
+    const int per = (H + kWave - 1) / kWave;
+    const int i0 = min(H, lane * per), i1 = min(H, i0 + per);
+    int sum = 0;
+    for (int t = i0; t < i1; ++t) sum += rows[1 + t];
+    int run = wave_inclusive_scan(sum) - sum;
+    for (int t = i0; t < i1; ++t) {
+      const int c = rows[1 + t];
+      rows[1 + t] = run;
+      run += c;
+    }
+  }
+  lds_sync();
+  for (int j = tid; j < n; j += kLongThreads) {  // ... and its end, the start of row y + 1
+    const float4 s = sp[j];
+    float X, Y;
+    if (!to_pixel(s, a, X, Y)) continue;
+    const int yi = min(static_cast<int>(Y), H - 1), xi = min(static_cast<int>(X), W - 1);
+    const int q = atomicAdd(&rows[yi + 1], 1);
+    s_key[q] = (xi << 16) | j;
+    s_I[q] = s.w;
+    s_y[q] = static_cast<short>(yi);
+  }
+  lds_sync();
+  const int total = rows[H];
+  // ---- last write wins: a spot yields to a later one on its pixel ----------
+  float pm = 0.0f;
+  int mine = 0;
+  for (int e = tid; e < total; e += kLongThreads) {
+    const int k = s_key[e], yi = s_y[e];
+    bool lose = false;
+    for (int o = rows[yi]; o < rows[yi + 1]; ++o) {
+      const int ko = s_key[o];
+      lose |= (ko >> 16) == (k >> 16) && ko > k;
+    }
+    if (lose) {
+      s_I[e] = 0.0f;  // contributes nothing
+    } else {
+      pm = fmaxf(pm, fabsf(s_I[e]));
+      ++mine;
+    }
+  }
+  pm = wave_max(pm);
+  mine = wave_sum(mine);
+  if (lane == 0) {
+    s_pm[wid] = pm;
+    s_n[wid] = mine;
+  }
+  lds_sync();
+  float pmax = 0.0f;
+  int ns = 0;
+#pragma unroll
+  for (int w = 0; w < kLongWaves; ++w) {
+    pmax = fmaxf(pmax, s_pm[w]);
+    ns += s_n[w];
+  }
+  // ---- tile bounds and the fixed-point scale (as tile_bounds) --------------
+  const float w0 = s_tp[0];
+  const float inv_p = pmax > 0.0f ? kLongUnits / pmax : 0.0f;
+  for (int e = tid; e < total; e += kLongThreads) {
+    const float I = s_I[e];
+    if (I == 0.0f) continue;
+    if (fabsf(I) == pmax) atomicMin(&s_q, e);
+    const int yi = s_y[e], xi = s_key[e] >> 16;
+    const bool inx = xi >= R && xi + R < W, iny = yi >= R && yi + R < H;
+    const float bx = inx ? w0 : fminf(1.0f, 3.0f * w0);
+    const float by = iny ? w0 : fminf(1.0f, 3.0f * w0);
+    const float aI = fabsf(I);
+    // a footprint of at most 17 pixels reaches at most two tiles per axis
+    const int tx0 = max(0, xi - R) / kTile, tx1 = min(W - 1, xi + R) / kTile;
+    const int ty0 = max(0, yi - R) / kTile, ty1 = min(H - 1, yi + R) / kTile;
+    for (int ty = ty0; ty <= ty1; ++ty)
+      for (int tx = tx0; tx <= tx1; ++tx) {
+        // the taps fall off from the centre: a tile's largest weight is at
+        // its pixel nearest (xi, yi)
+        const bool in = inx && iny;
+        const float wx = in ? s_tp[tile_gap(tx, xi)] : bx, wy = in ? s_tp[tile_gap(ty, yi)] : by;
+        atomicAdd(&tile_u[ty * ntx + tx], bound_units(aI, wx, wy, inv_p));
+      }
+  }
+  lds_sync();
+  int lu = 0;
+  for (int t = tid; t < n_tiles; t += kLongThreads) lu = max(lu, tile_u[t]);
+  lu = wave_max_i(lu);
+  if (lane == 0) s_u[wid] = lu;
+  lds_sync();
+  int Ui = 0;
+#pragma unroll
+  for (int w = 0; w < kLongWaves; ++w) Ui = max(Ui, s_u[w]);
+  const float unit = pmax / kLongUnits;
+  const float U = static_cast<float>(Ui) * unit;
+  const float scale = U > 0.0f ? kScaleRange / (U * 1.00001f) : 1.0f;
+  float out_scale = 1.0f / scale;
+  if (a.normalize && pmax > 0.0f) {
+    // ---- exact maximum: every tile whose bound can reach the value at the
+    // brightest spot's pixel, shared over the waves (the bound keeps every
+    // pixel sum below 2^31)
+    const int qs = s_q;
+    const int ys = s_y[qs], xs = s_key[qs] >> 16;
+    int acc = 0;
+    for (int e = rows[max(0, ys - R)] + lane; e < rows[min(H - 1, ys + R) + 1]; e += kWave) {
+      const int yi = s_y[e], xi = s_key[e] >> 16;
+      if (xs < xi - R || xs > xi + R) continue;
+      const float iws = s_I[e] * band_weight(xs, xi, W, R, s_tp) * scale;
+      if (iws != 0.0f) acc += band_term<true>(iws, band_weight(ys, yi, H, R, s_tp));
+    }
+    const int lfix = wave_sum(acc);
+    // a term rounds up by at most half a unit
+    const float margin = 0.5f * static_cast<float>(ns) + 1.0f;
+    if (tid == 0) s_best = lfix;
+    lds_sync();
+    for (int t = wid; t < n_tiles; t += kLongWaves) {
+      const float bound = static_cast<float>(tile_u[t]) * unit * scale * 1.00001f + margin;
+      const int best = *const_cast<volatile int *>(&s_best);
+      if (static_cast<double>(bound) < static_cast<double>(best)) continue;
+      const int ty = t / ntx;
+      const int m = tile_max<R>(a, t - ty * ntx, ty, rows[max(0, ty * kTile - R)],
+                                rows[min(H - 1, ty * kTile + kTile - 1 + R) + 1], s_key, s_I, s_y,
+                                s_tp, scale, s_tile[wid], s_cq[wid], lane, best);
+      if (lane == 0 && m > best) atomicMax(&s_best, m);
+    }
+    lds_sync();
+    const int best = s_best;
+    // a zero maximum leaves the zeros as they are instead of producing 0/0
+    if (best > 0) out_scale = 1.0f / static_cast<float>(best);
+  }
+  if (tid == 0) {
+    *reinterpret_cast<int4 *>(rec) = make_int4(0, ns, __float_as_int(scale), __float_as_int(out_scale));
+    if (a.status) a.status[p] = 0;
+  }
+  for (int bb = tid; bb < b.nb; bb += kLongThreads) {
+    const int y0 = bb * b.band_rows, y1 = min(H, y0 + b.band_rows) - 1;
+    reinterpret_cast<int2 *>(rec + 4)[bb] = make_int2(rows[max(0, y0 - R)], rows[min(H - 1, y1 + R) + 1]);
+  }
+  int2 *ent = b.ent + static_cast<size_t>(pl) * b.ent_stride;
+  for (int e = tid; e < total; e += kLongThreads)
+    ent[e] = make_int2((static_cast<int>(s_y[e]) << 16) | (s_key[e] >> 16), __float_as_int(s_I[e]));
+}
+
 // Pixels per band: 2,048 (two 16-byte stores per thread) up to R = 5, 4,096
 // for wider taps.  A band of B rows splats the spots of B + 2R rows, so wide
 // taps make the splat's VALU work, not the stores, bound small bands.
 // Render stage of 12,000 x 232 x 200, 235 spots each, with 2,048 / 4,096
 // pixels: R = 4 402 / 461 us, R = 5 458 / 468, R = 6 589 / 472, R = 7
 // 672 / 533, R = 8 782 / 618.
-__host__ __device__ constexpr int band_vec(int R) { return R <= 5 ? 2 : 4; }
-__host__ __device__ constexpr int band_pix(int R) { return 4 * band_vec(R) * kBandThreads; }
+__host__ __device__ constexpr int band_vec(int R, bool long_lists = false) {
+  return R <= 5 && !long_lists ? 2 : 4;
+}
+__host__ __device__ constexpr int band_pix(int R, bool long_lists = false) {
+  return 4 * band_vec(R, long_lists) * kBandThreads;
+}
 
 // kAligned: every row is a whole number of 16-byte vectors.  Otherwise the
 // band's pixels sit in LDS at the offset their first pixel has within its
@@ -1159,9 +1432,16 @@ __host__ __device__ constexpr int band_pix(int R) { return 4 * band_vec(R) * kBa
 // the library's aligned patterns 6 %: 487 -> 519 us per round of 16,384).
 // Odd widths went through render_kernel before (12,000 x 231 x 201, R = 7:
 // 730 us there; 62 us plan and 425 us writer here, 5.3 TB/s).
-template <int kR, bool kAligned>
+// kLong: lists of any length (render_plan_long_kernel), whose window passes
+// through LDS kPlanMax spots at a time.
+template <int kR, bool kAligned, bool kLong = false>
 __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
-  constexpr int kVec = band_vec(kR), kPix = band_pix(kR);
+  constexpr int kVec = band_vec(kR, kLong), kPix = band_pix(kR, kLong);
+  // how the rows outside the band are dropped, as measured (render stage, us,
+  // row tests / flat index): 16,000 x 256 x 256 with R = 2 667 / 666, R = 4
+  // 660 / 646, R = 5 729 / 698, R = 6 701 / 731, R = 7 732 / 710 (231 x 201:
+  // 571 / 599), R = 8 909 / 850; long lists of 2,300 521 / 497
+  constexpr bool kFlat = kLong || kR == 4 || kR == 5 || kR == 8;
   __shared__ __align__(16) racc_t s_acc[kPix + (kAligned ? 0 : 4)];
   __shared__ int2 s_ent[kPlanMax];
   __shared__ float s_tp[kR + 1];
@@ -1182,7 +1462,8 @@ __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
   const int y1 = min(H, y0 + b.band_rows) - 1;  // last row of the band
   float *first = a.out + static_cast<size_t>(p) * H * W + static_cast<size_t>(y0) * W;
   const int shift = kAligned ? 0 : static_cast<int>(reinterpret_cast<uintptr_t>(first) >> 2) & 3;
-  const int last = shift + (y1 - y0 + 1) * W;  // LDS words [shift, last) are the band
+  const unsigned pixels = static_cast<unsigned>((y1 - y0 + 1) * W);
+  const int last = shift + static_cast<int>(pixels);  // LDS words [shift, last) are the band
   const int nvec = kAligned ? last / 4 : (last + 3) / 4;
   // one scalar round: the pattern's header and the band's window of the
   // row-sorted list (rows y0 - R .. y1 + R)
@@ -1195,34 +1476,53 @@ __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
     if (tid == i) s_tp[i] = a.taps[i];
   for (int v = tid; v < nvec; v += kBandThreads) reinterpret_cast<int4 *>(s_acc)[v] = make_int4(0, 0, 0, 0);
   if (h.x != 0) return;  // listed for render_kernel (uniform across the block)
-  const int cnt = e1 - e0;
-  const int2 *ent = b.ent + static_cast<size_t>(pl) * kPlanMax + e0;
-  for (int q = tid; q < cnt; q += kBandThreads) s_ent[q] = ent[q];
-  lds_sync();
+  const int total = e1 - e0;
+  const int2 *ent = b.ent + static_cast<size_t>(pl) * (kLong ? b.ent_stride : kPlanMax) + e0;
   const float scale = __int_as_float(h.z), out_scale = __int_as_float(h.w);
-  for (int it = tid; it < cnt * ncols; it += kBandThreads) {
-    const int q = it / ncols, c = it - q * ncols;
-    const int2 en = s_ent[q];
-    const int yi = en.x >> 16, xi = en.x & 0xffff;
-    const int x = xi - R + c;
-    if (x < 0 || x >= W) continue;
-    // render_kernel's splat terms: ((I wx) scale) wy, truncated
-    const float wx = (xi >= R && xi + R < W) ? s_tp[c > R ? c - R : R - c]
-                                             : reflect_weight3(x, xi, W, R, s_tp);
-    const float iws = __int_as_float(en.y) * wx * scale;
-    const int ya = max(yi - R, y0), yb = min(yi + R, y1);
-    racc_t *col = s_acc + (x - y0 * W + shift);
-    if (yi >= R && yi + R < H) {
+  for (int c0 = 0;; c0 += kPlanMax) {  // one turn unless kLong
+    const int cnt = kLong ? min(kPlanMax, total - c0) : total;
+    for (int q = tid; q < cnt; q += kBandThreads) s_ent[q] = ent[c0 + q];
+    lds_sync();
+    for (int it = tid; it < cnt * ncols; it += kBandThreads) {
+      const int q = it / ncols, c = it - q * ncols;
+      const int2 en = s_ent[q];
+      const int yi = en.x >> 16, xi = en.x & 0xffff;
+      const int x = xi - R + c;
+      if (x < 0 || x >= W) continue;
+      // render_kernel's splat terms: ((I wx) scale) wy, truncated
+      const float wx = (xi >= R && xi + R < W) ? s_tp[c > R ? c - R : R - c]
+                                               : reflect_weight3(x, xi, W, R, s_tp);
+      const float iws = __int_as_float(en.y) * wx * scale;
+      if (yi >= R && yi + R < H) {
+        if (kFlat) {
+          // a column's terms are symmetric, and one unsigned comparison of the
+          // flat index drops the rows outside the band (0 <= x < W)
+          racc_t term[R + 1];
 #pragma unroll
-      for (int dd = -R; dd <= R; ++dd) {
-        const int y = yi + dd;
-        if (y >= ya && y <= yb) atomicAdd(col + y * W, fast_fixed(iws, a.taps[dd < 0 ? -dd : dd]));
+          for (int d = 0; d <= R; ++d) term[d] = band_term<kLong>(iws, a.taps[d]);
+          unsigned at = static_cast<unsigned>((yi - R - y0) * W + x);
+#pragma unroll
+          for (int dd = -R; dd <= R; ++dd, at += W)
+            if (at < pixels) atomicAdd(&s_acc[shift + at], term[dd < 0 ? -dd : dd]);
+        } else {
+          const int ya = max(yi - R, y0), yb = min(yi + R, y1);
+          racc_t *col = s_acc + (x - y0 * W + shift);
+#pragma unroll
+          for (int dd = -R; dd <= R; ++dd) {
+            const int y = yi + dd;
+            if (y >= ya && y <= yb)
+              atomicAdd(col + y * W, band_term<kLong>(iws, a.taps[dd < 0 ? -dd : dd]));
+          }
+        }
+      } else {
+        racc_t *col = s_acc + (x - y0 * W + shift);
+        for (int y = max(yi - R, y0); y <= min(yi + R, y1); ++y)
+          atomicAdd(col + y * W, band_term<kLong>(iws, reflect_weight3(y, yi, H, R, s_tp)));
       }
-    } else {
-      for (int y = ya; y <= yb; ++y) atomicAdd(col + y * W, fast_fixed(iws, reflect_weight3(y, yi, H, R, s_tp)));
     }
+    lds_sync();
+    if (!kLong || c0 + kPlanMax >= total) break;
   }
-  lds_sync();
   float *dst = first - shift;  // words outside [shift, last) are not touched
   auto store = [&](int v) {
     const int4 u = reinterpret_cast<const int4 *>(s_acc)[v];
@@ -2107,8 +2407,8 @@ static int render_common(int mode, const float *spot_d, const int *count_d, int 
 
 // ---- band renderer: host side ----------------------------------------------
 
-static void band_shape(int R, int H, int W, int &band_rows, int &nb) {
-  band_rows = std::max(1, std::min(H, band_pix(R) / std::max(1, W)));
+static void band_shape(int R, int H, int W, int &band_rows, int &nb, bool long_lists = false) {
+  band_rows = std::max(1, std::min(H, band_pix(R, long_lists) / std::max(1, W)));
   nb = (H + band_rows - 1) / band_rows;
 }
 
@@ -2131,6 +2431,51 @@ static long long band_workspace_ints(int n, int H, int W) {
   band_shape(1, H, W, br, nb);  // the narrowest bands
   const long long chunk = std::min(std::max(n, 1), kBandChunk);
   return band_list_ints(std::max(n, 1)) + chunk * band_rec_ints(nb) + chunk * kPlanMax * 2;
+}
+
+// Long lists: patterns per plan/writer round, so that the hand-over (8 B per
+// entry of the list's capacity) stays within kLongHandOver bytes: in the
+// last-level cache from the plan to the writer.
+constexpr long long kLongHandOver = 64ll << 20;
+static int long_chunk(int cap, int n) {
+  const long long m = kLongHandOver / (8ll * cap) / 8 * 8;
+  return static_cast<int>(std::min<long long>(std::max(n, 1), std::max<long long>(256, std::min<long long>(m, kBandChunk))));
+}
+
+static long long long_workspace_ints(int cap, int n, int H, int W) {
+  int br, nb;
+  band_shape(1, H, W, br, nb, true);
+  const long long chunk = long_chunk(cap, n);
+  return chunk * band_rec_ints(nb) + chunk * cap * 2;
+}
+
+// The shapes of band_fits with lists that the plan's LDS holds (about 14,000
+// spots at 256 x 256).
+static bool long_fits(int cap, int R, int H, int W) {
+  const int n_tiles = ((W + kTile - 1) / kTile) * ((H + kTile - 1) / kTile);
+  return cap >= 1 && cap <= 16384 && R >= 1 && R <= 8 && R < std::min(H, W) && W <= kPlanMaxSide &&
+         H <= kPlanMaxSide && n_tiles <= kMaxTiles && long_plan_bytes(cap, H, n_tiles) <= kLongLdsBytes;
+}
+
+template <int kR>
+static int launch_long_r(const BandArgs &b, size_t lds, hipStream_t st) {
+  static int reserved = -1;  // raised once, so graph-recorded launches issue no attribute calls
+  if (reserved < 0) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&render_plan_long_kernel<kR>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kLongLdsBytes) != hipSuccess) {
+      (void)hipGetLastError();
+      set_error("dsx_render_fast_long: cannot reserve %d bytes of LDS", kLongLdsBytes);
+      return DSX_ELAUNCH;
+    }
+    reserved = 1;
+  }
+  hipLaunchKernelGGL(render_plan_long_kernel<kR>, dim3(b.m), dim3(kLongThreads), lds, st, b);
+  const unsigned blocks = static_cast<unsigned>((b.m + 7) / 8) * 8u * static_cast<unsigned>(b.nb);
+  if ((b.r.W & 3) == 0 && (reinterpret_cast<uintptr_t>(b.r.out) & 15) == 0)
+    hipLaunchKernelGGL((render_band_kernel<kR, true, true>), dim3(blocks), dim3(kBandThreads), 0, st, b);
+  else
+    hipLaunchKernelGGL((render_band_kernel<kR, false, true>), dim3(blocks), dim3(kBandThreads), 0, st, b);
+  return DSX_OK;
 }
 
 __global__ void band_list_reset_kernel(int *count) {
@@ -2245,6 +2590,7 @@ extern "C" int dsx_render_fast_bands(const float *spot_d, const int *count_d, in
   b.n_tiles = b.ntx * ((a.H + kTile - 1) / kTile);
   b.wave_ints = plan_wave_ints(a.H, b.n_tiles);
   const int chunk = std::min(n, kBandChunk);
+  b.ent_stride = kPlanMax;
   b.fallback = work_d;
   b.rec_ints = band_rec_ints(b.nb);
   b.rec = work_d + band_list_ints(n);
@@ -2271,6 +2617,82 @@ extern "C" int dsx_render_fast_bands(const float *spot_d, const int *count_d, in
   f.list = b.fallback + 1;
   f.n_dev = b.fallback;
   return launch_splat(kModeFast, f, bpc, s, name);
+}
+
+extern "C" int dsx_render_fast_long_fits(int cap, int radius, int height, int width) {
+  return long_fits(cap, radius, height, width) ? 1 : 0;
+}
+
+extern "C" long long dsx_render_fast_long_workspace_ints(int cap, int n, int height, int width) {
+  if (cap < 1 || n < 0 || height < 1 || width < 1) return -1;
+  return long_workspace_ints(cap, n, height, width);
+}
+
+extern "C" int dsx_render_fast_long(const float *spot_d, const int *count_d, int cap, int n,
+                                    const dsx_render_params *params, int *work_d,
+                                    long long work_ints, float *out_d, int *status_d,
+                                    void *stream) {
+  const char *name = "dsx_render_fast_long";
+  clear_error();
+  if (!params || n < 0 || cap < 1 || work_ints < 0) {
+    set_error("%s: bad arguments (n=%d cap=%d)", name, n, cap);
+    return DSX_EINVAL;
+  }
+  if (n == 0) return DSX_OK;
+  if (!spot_d || !count_d || !out_d || !work_d) {
+    set_error("%s: null device pointer", name);
+    return DSX_EINVAL;
+  }
+  BandArgs b;
+  RenderArgs &a = b.r;
+  const int st = fill_render_args(kModeFast, params, a, name);
+  if (st != DSX_OK) return st;
+  if (!long_fits(cap, a.R, a.H, a.W)) {
+    set_error("%s: lists of %d spots on %dx%d patterns with tap radius %d do not fit "
+              "(dsx_render_fast_long_fits)", name, cap, a.H, a.W, a.R);
+    return DSX_EINVAL;
+  }
+  const long long need = long_workspace_ints(cap, n, a.H, a.W);
+  if (work_ints < need || reinterpret_cast<uintptr_t>(work_d) % 16 != 0) {
+    set_error("%s: workspace of %lld ints is smaller than %lld or not 16-byte aligned", name,
+              work_ints, need);
+    return DSX_EINVAL;
+  }
+  a.spots = reinterpret_cast<const float4 *>(spot_d);
+  a.count = count_d;
+  a.cap = cap;
+  a.n = n;
+  a.out = out_d;
+  a.status = status_d;
+  band_shape(a.R, a.H, a.W, b.band_rows, b.nb, true);
+  b.ntx = (a.W + kTile - 1) / kTile;
+  b.n_tiles = b.ntx * ((a.H + kTile - 1) / kTile);
+  b.wave_ints = 0;
+  b.fallback = nullptr;
+  const int chunk = long_chunk(cap, n);
+  b.rec_ints = band_rec_ints(b.nb);
+  b.rec = work_d;
+  b.ent = reinterpret_cast<int2 *>(work_d + static_cast<long long>(chunk) * b.rec_ints);
+  b.ent_stride = cap;
+  const size_t lds = (static_cast<size_t>(long_plan_bytes(cap, a.H, b.n_tiles)) + 15) & ~static_cast<size_t>(15);
+  hipStream_t s = as_stream(stream);
+  for (int c0 = 0; c0 < n; c0 += chunk) {
+    b.p0 = c0;
+    b.m = std::min(chunk, n - c0);
+    int rc;
+    switch (a.R) {
+      case 1: rc = launch_long_r<1>(b, lds, s); break;
+      case 2: rc = launch_long_r<2>(b, lds, s); break;
+      case 3: rc = launch_long_r<3>(b, lds, s); break;
+      case 4: rc = launch_long_r<4>(b, lds, s); break;
+      case 5: rc = launch_long_r<5>(b, lds, s); break;
+      case 6: rc = launch_long_r<6>(b, lds, s); break;
+      case 7: rc = launch_long_r<7>(b, lds, s); break;
+      default: rc = launch_long_r<8>(b, lds, s);
+    }
+    if (rc != DSX_OK) return rc;
+  }
+  return check_launch(name);
 }
 
 extern "C" int dsx_render_dense_max_pixels(void) { return kDenseMaxPix; }

@@ -67,6 +67,15 @@ def fast_renderer(n: int, height: int, width: int) -> str:
     return "dsx_render_fast_bands"
 
 
+def long_renderer(cap: int, height: int, width: int, radius: int) -> bool:
+    """Whether ``render_spots`` renders fast lists of more than
+    dsx_render_max_spots() spots with dsx_render_fast_long: patterns too large
+    for the dense renderers' LDS, as far as the lists fit its plan."""
+    L = _lib.load()
+    return (height * width > int(L.dsx_render_dense_max_pixels())
+            and bool(L.dsx_render_fast_long_fits(int(cap), int(radius), int(height), int(width))))
+
+
 def _device(device=None) -> torch.device:
     _lib.load(require_gpu=True)
     if device is None:
@@ -529,6 +538,12 @@ def render_spots(spots: torch.Tensor, count: torch.Tensor, cap: int, shape, sigm
             None, _lib.ptr(spots), _lib.ptr(count), cap, n, None, None, 0, None, ctypes.byref(sim),
             ctypes.byref(p), _lib.ADJ_FORWARD, None, 0, _lib.ptr(out), None, None, None, None,
             _lib.ptr(work), work.numel(), _lib.ptr(status), stream), "dsx_render_adjoint")
+    elif fast and cap > int(L.dsx_render_max_spots()) and long_renderer(cap, H, W, p.radius):
+        # the whole list in LDS by a plan kernel, the pixels by the band writer
+        work = _workspace(dev, int(L.dsx_render_fast_long_workspace_ints(int(cap), n, H, W)), stream)
+        _lib.check(L.dsx_render_fast_long(
+            _lib.ptr(spots), _lib.ptr(count), cap, n, ctypes.byref(p), _lib.ptr(work), work.numel(),
+            _lib.ptr(out), _lib.ptr(status), stream), "dsx_render_fast_long")
     elif fast and cap > int(L.dsx_render_max_spots()):
         # more spots than the splat renderer holds: whole pattern in LDS when
         # it fits, otherwise strip windows with spot bins in a workspace

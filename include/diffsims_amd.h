@@ -304,6 +304,28 @@ int dsx_render_fast_bands(const float *spot_d, const int *count_d, int cap, int 
                           float *out_d, int *status_d, void *stream);
 
 /*
+ * fast=True rendering of n patterns with long spot lists (more distinct spots
+ * than dsx_render_fast holds) -- the same reference path (simulation2d.py:405-442,
+ * detector_functions.py:293-300) -- by a plan kernel that holds a pattern's
+ * whole list in LDS and the band writer of dsx_render_fast_bands; no pattern
+ * is left out.  The sums are dsx_render_fast's fixed point with a scale of its
+ * own (a few 1e-9 of the maximum).
+ *   dsx_render_fast_long_fits : 1 when lists of `cap` spots with this tap
+ *            radius (1..8, below both sides) and shape (sides up to 1024) are
+ *            taken, about 14,000 spots at 256 x 256; else use
+ *            dsx_render_fast_large
+ *   work_d : dsx_render_fast_long_workspace_ints(cap, n, height, width) ints,
+ *            16-byte aligned (patterns are taken in rounds that reuse it in
+ *            stream order); overlapping calls must not share it
+ * Other arguments as for dsx_render_fast; status_d is 0 for every pattern.
+ */
+int dsx_render_fast_long_fits(int cap, int radius, int height, int width);
+long long dsx_render_fast_long_workspace_ints(int cap, int n, int height, int width);
+int dsx_render_fast_long(const float *spot_d, const int *count_d, int cap, int n,
+                         const dsx_render_params *params, int *work_d, long long work_ints,
+                         float *out_d, int *status_d, void *stream);
+
+/*
  * fast=True rendering of large patterns with many spots (the same result as
  * dsx_render_fast, no limit on spots per pattern): each output strip rebuilds
  * the spot image of its window in LDS and filters it; in-frame spots are

@@ -261,3 +261,112 @@ def test_render_spots_same_bits_across_the_small_batch_threshold():
                                 1.0, 1.0)
     torch.cuda.synchronize()
     assert torch.equal(big[:700], small)
+
+
+# -- long lists (dsx_render_fast_long) ------------------------------------------
+
+
+def _render_long(spots, cnt, cap, shape, sigma, normalize=True):
+    import torch
+    from diffsims_amd import engine
+    lib, L = _lib()
+    n = int(cnt.shape[0])
+    H, W = shape
+    p = engine.render_params(shape, sigma, 1.0, normalize=normalize)
+    assert L.dsx_render_fast_long_fits(cap, p.radius, H, W) == 1
+    out = torch.full((n, H, W), float("nan"), dtype=torch.float32, device="cuda")
+    st = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+    ws = int(L.dsx_render_fast_long_workspace_ints(cap, n, H, W))
+    work = torch.empty(ws, dtype=torch.int32, device="cuda")
+    lib.check(L.dsx_render_fast_long(lib.ptr(spots), lib.ptr(cnt), cap, n, ctypes.byref(p),
+                                     lib.ptr(work), ws, lib.ptr(out), lib.ptr(st),
+                                     lib.stream_handle(spots.device)), "dsx_render_fast_long")
+    assert not torch.isnan(out).any() and not st.any()
+    return out
+
+
+def _fp64_patterns(spots, cnt, shape, sigma, normalize, which):
+    """scipy's filter of the last-write-wins image, FP64, patterns ``which``."""
+    from scipy.ndimage import gaussian_filter
+    H, W = shape
+    sp, c = spots.cpu().numpy(), np.minimum(cnt.cpu().numpy(), spots.shape[1])
+    out = []
+    for i in which:
+        img = np.zeros(shape)
+        X = sp[i, :c[i], 0] + np.float32(W // 2)
+        Y = sp[i, :c[i], 1] + np.float32(H // 2)
+        for x, y, v in zip(X, Y, sp[i, :c[i], 3]):
+            if 0 <= x < W and 0 <= y < H:
+                img[int(y), int(x)] = v
+        img = gaussian_filter(img, sigma)
+        out.append(img / img.max() if normalize and img.max() > 0 else img)
+    return np.stack(out)
+
+
+# A term has four roundings of 2^-24 (two products, two taps), the output two
+# more, and every term half a unit of U / 2.04e9: with at most ~60 spots in a
+# pixel's reach and U below 60 maxima 60 * 60 / 2 / 2.04e9 = 9e-7.
+LONG_TOL = 6 * 2.0 ** -24 + 9e-7
+
+
+@pytest.mark.parametrize("shape,sigma,cap,mean", [
+    ((129, 128), 1.0, 1100, 1000), ((256, 256), 1.0, 3000, 2300), ((251, 203), 2.0, 2500, 2300),
+    ((512, 512), 0.3, 9000, 8000), ((300, 147), 1.25, 1500, 1400), ((256, 256), 1.0, 14000, 12000)])
+@pytest.mark.parametrize("normalize", [True, False])
+def test_long_lists_against_fp64(shape, sigma, cap, mean, normalize):
+    n, R = 9, int(4 * sigma + 0.5)
+    print(f"long lists: {n} x {shape}, sigma {sigma}, {mean} spots", flush=True)
+    spots, cnt = _spot_lists(n, cap, shape[0], shape[1], mean, seed=mean, edge=0.1, R=R)
+    cnt[3] = cap + 50  # more than the list holds
+    # later spots on the pixels of earlier ones
+    spots[:, cap // 2:cap // 2 + 40, :2] = spots[:, 10:50, :2]
+    out = _render_long(spots, cnt, cap, shape, sigma, normalize).cpu().numpy()
+    which = [0, 3, n - 1]
+    ref = _fp64_patterns(spots, cnt, shape, sigma, normalize, which)
+    for o, r in zip(out[which], ref):
+        assert np.abs(o - r).max() <= LONG_TOL * r.max()
+
+
+def test_long_lists_degenerate_and_several_rounds():
+    import torch
+    print("long lists: 300 x 130x131 in two rounds, empty and zero lists", flush=True)
+    cap, shape = 14000, (130, 131)
+    spots, cnt = _spot_lists(300, cap, *shape, 30, seed=3)
+    cnt[0:4] = 0
+    spots[4:8, :, 0] += 1000.0   # out of frame
+    spots[8:12, :, 3] = 0.0      # maximum 0
+    cnt[12:16] = 1
+    spots[16:20, :, 3] = 2.5     # equal intensities
+    out = _render_long(spots, cnt, cap, shape, 1.0)
+    assert torch.equal(out[:12], torch.zeros_like(out[:12]))
+    which = [12, 16, 255, 256, 299]
+    ref = _fp64_patterns(spots, cnt, shape, 1.0, True, which)
+    assert np.abs(out[which].cpu().numpy() - ref).max() <= LONG_TOL
+
+
+def test_long_lists_dispatch_and_limits():
+    import torch
+    from diffsims_amd import engine
+    lib, L = _lib()
+    fits = L.dsx_render_fast_long_fits
+    assert fits(2000, 4, 256, 256) and not fits(17000, 4, 256, 256)
+    assert not fits(2000, 0, 256, 256) and not fits(2000, 9, 256, 256)
+    assert not fits(2000, 4, 1025, 64) and not fits(2000, 4, 256, 4)
+    assert engine.long_renderer(2000, 256, 256, 4)
+    assert not engine.long_renderer(2000, 128, 128, 4)   # the dense renderers
+    assert not engine.long_renderer(30000, 256, 256, 4)  # dsx_render_fast_large
+    # render_spots on both sides of the lists it takes: the same pixels
+    spots, cnt = _spot_lists(6, 1500, 200, 160, 1400, seed=2)
+    a = engine.render_spots(spots, cnt, 1500, (200, 160), 1.0, 1.0)
+    wide = torch.zeros((6, 16500, 4), dtype=torch.float32, device="cuda")
+    wide[:, :1500] = spots
+    b = engine.render_spots(wide, cnt, 16500, (200, 160), 1.0, 1.0)
+    assert float((a - b).abs().max()) <= 2 * LONG_TOL
+    p = engine.render_params((256, 256), 1.0, 1.0)
+    work = torch.empty(64, dtype=torch.int32, device="cuda")
+    out = torch.empty((6, 256, 256), dtype=torch.float32, device="cuda")
+    for c, ws in ((1500, 64), (16500, 64)):
+        rc = L.dsx_render_fast_long(lib.ptr(wide), lib.ptr(cnt), c, 6, ctypes.byref(p),
+                                    lib.ptr(work), ws, lib.ptr(out), None,
+                                    lib.stream_handle(spots.device))
+        assert rc == lib.DSX_EINVAL
