@@ -33,6 +33,33 @@ inline void fill_physics(Args &a, const dsx_sim_params *p) {
   a.Pt = k * sin(phi);
 }
 
+// sqrt(x), 1/x and a/b for normal, finite x and b of ordinary size (no scaling
+// of denormals and no special values, which the library forms spend half of
+// their instructions on): the hardware estimate (about 2^-26), one coupled
+// Newton step and one residual step, within an ulp or two of the rounded
+// result.  fsqrt_pos(0) is 1e-150 instead of 0.
+__device__ __forceinline__ double fsqrt_pos(double x) {
+  const double v = fmax(x, 1e-300);
+  const double y = __builtin_amdgcn_rsq(v);
+  double g = v * y, h = 0.5 * y;
+  const double e = fma(-h, g, 0.5);
+  g = fma(g, e, g);
+  h = fma(h, e, h);
+  return fma(fma(-g, g, v), h, g);
+}
+
+__device__ __forceinline__ double frcp(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = fma(fma(-x, y, 1.0), y, y);
+  return fma(fma(-x, y, 1.0), y, y);
+}
+
+__device__ __forceinline__ double fdiv(double a, double b) {
+  const double y = frcp(b);
+  const double q = a * y;
+  return fma(fma(-b, q, a), y, q);
+}
+
 // The models of shape_factor_models.py in plain FP64 (the inner function of
 // the full precession average).
 template <class Args>
@@ -177,7 +204,7 @@ __device__ __forceinline__ double shape_factor(double s, double r, const Args &a
       return fmax(1.0 - fabs(s) / a.width, 0.0);
     case DSX_SF_LORENTZIAN: {
       const double t = a.sigma * s;
-      return 1.0 / (1.0 + t * t);
+      return frcp(fma(t, t, 1.0));
     }
     // the transcendental models take their FP64 argument rounded to FP32
     // (relative error ~1e-7 of the factor)
@@ -199,11 +226,11 @@ __device__ __forceinline__ double shape_factor(double s, double r, const Args &a
       // z = sqrt(u^2 + 4 sigma^2 s^2); u + z rewritten for u < 0.
       const double A = r * a.phi;
       const double sg2 = a.sigma * a.sigma;
-      const double u = sg2 * ((A - s) * (A + s)) + 1.0;
+      const double u = fma(sg2, (A - s) * (A + s), 1.0);
       const double ss = 4.0 * sg2 * s * s;
-      const double z = sqrt(u * u + ss);
-      const double upz = u >= 0.0 ? u + z : ss / (z - u);
-      return (a.sigma * 0.31830988618379067) * sqrt(2.0 * upz) / z;
+      const double z = fsqrt_pos(fma(u, u, ss));
+      const double upz = u >= 0.0 ? u + z : fdiv(ss, z - u);
+      return fdiv((a.sigma * 0.31830988618379067) * fsqrt_pos(2.0 * upz), z);
     }
     default:
       if (kAvg && a.model >= DSX_SF_PRECESSION_AVG)
@@ -216,20 +243,25 @@ __device__ __forceinline__ double shape_factor(double s, double r, const Args &a
 // cancellations removed:
 //   k - sqrt(k^2 - r^2)            = r^2 / (k + sqrt(k^2 - r^2))
 //   Pz - sqrt(k^2 - (r +- Pt)^2)   = r (r +- 2 Pt) / (Pz + sqrt(k^2 - (r +- Pt)^2))
+// and the precession bounds compared without their divisions (the
+// denominators are positive).  The FP64 roots and quotients of the candidates
+// are most of the spot kernel's work under precession (six roots and four
+// quotients each; the library forms took about 240 instructions there, these
+// about 130).  r is only formed where a model needs it (precession).
 template <class Args>
 __device__ __forceinline__ bool intersects(double x, double y, double z, const Args &a,
                                            double &s, double &r) {
-  const double r2 = x * x + y * y;
-  r = sqrt(r2);
+  const double r2 = fma(y, y, x * x);
+  r = 0.0;
   if (!(r2 < a.k2)) return false;
-  s = r2 / (a.k + sqrt(a.k2 - r2)) - z;
+  s = fdiv(r2, a.k + fsqrt_pos(a.k2 - r2)) - z;
   if (!a.precession) return fabs(s) < a.me;
+  r = fsqrt_pos(r2);
   const double rp = r + a.Pt, rm = r - a.Pt;
-  const double qp = a.k2 - rp * rp, qm = a.k2 - rm * rm;
+  const double qp = fma(-rp, rp, a.k2), qm = fma(-rm, rm, a.k2);
   if (!(qp >= 0.0) || !(qm >= 0.0)) return false;
-  const double up = r * (r + 2.0 * a.Pt) / (a.Pz + sqrt(qp));
-  const double dn = r * (r - 2.0 * a.Pt) / (a.Pz + sqrt(qm));
-  return (z - a.me <= up) && (z + a.me >= dn);
+  return (z - a.me) * (a.Pz + fsqrt_pos(qp)) <= r * fma(2.0, a.Pt, r) &&
+         (z + a.me) * (a.Pz + fsqrt_pos(qm)) >= r * fma(-2.0, a.Pt, r);
 }
 
 // Shape factor f(s, r) with its partial derivatives df/ds and df/dr (r only

@@ -77,6 +77,28 @@ __host__ __device__ __forceinline__ float pretest_threshold(double me, double k,
                             1e-6 * (2.0 * k * gmax + gmax * gmax));
 }
 
+// One candidate in FP64: lab position of row `row` in the orientation Rd, its
+// membership and its intensity.  Sums are written as fma chains, so every
+// kernel rounds them alike.
+template <bool kAvg>
+__device__ __forceinline__ bool eval_candidate(const SimArgs &a, const int4 *hkl, const float *F2,
+                                               const double *rec, const double *Rd, int row,
+                                               float4 &spot) {
+  const int4 h = hkl[row];
+  const double hx = h.x, hy = h.y, hz = h.z;
+  const double gx = fma(rec[2], hz, fma(rec[1], hy, rec[0] * hx));
+  const double gy = fma(rec[5], hz, fma(rec[4], hy, rec[3] * hx));
+  const double gz = fma(rec[8], hz, fma(rec[7], hy, rec[6] * hx));
+  const double x = fma(Rd[2], gz, fma(Rd[1], gy, Rd[0] * gx));
+  const double y = fma(Rd[5], gz, fma(Rd[4], gy, Rd[3] * gx));
+  const double z = fma(Rd[8], gz, fma(Rd[7], gy, Rd[6] * gx));
+  double s, r;
+  const bool in = intersects(x, y, z, a, s, r);
+  spot = make_float4(static_cast<float>(x), static_cast<float>(y), static_cast<float>(z), 0.0f);
+  if (in) spot.w = static_cast<float>(shape_factor<kAvg>(s, r, a) * static_cast<double>(F2[row]));
+  return in;
+}
+
 // Candidate queue per wave: (reflection row << kSlotBits) | orientation slot, in the
 // order the sweep produced them (row-major, so per orientation ascending rows).
 // Ring of at least one batch plus one worst-case step (64 + kOT * 64
@@ -168,24 +190,12 @@ __global__ __launch_bounds__(kSimThreads, sim_min_waves(kAvg, kLines)) void simu
     auto drain = [&](int nb) {
       bool in = false;
       int row = 0, slot = 0;
-      double x = 0.0, y = 0.0, z = 0.0;
-      float I = 0.0f;
+      float4 spot = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       if (lane < nb) {
         const int e = queue[qpos(head + lane)];
         row = e >> kSlotBits;
         slot = e & (kOT - 1);
-        const int4 h = hkl[row];
-        const double hx = h.x, hy = h.y, hz = h.z;
-        const double gx = rec[0] * hx + rec[1] * hy + rec[2] * hz;
-        const double gy = rec[3] * hx + rec[4] * hy + rec[5] * hz;
-        const double gz = rec[6] * hx + rec[7] * hy + rec[8] * hz;
-        const double *Rd = s_R[wib][slot];
-        x = Rd[0] * gx + Rd[1] * gy + Rd[2] * gz;
-        y = Rd[3] * gx + Rd[4] * gy + Rd[5] * gz;
-        z = Rd[6] * gx + Rd[7] * gy + Rd[8] * gz;
-        double s, r;
-        in = intersects(x, y, z, a, s, r);
-        if (in) I = static_cast<float>(shape_factor<kAvg>(s, r, a) * static_cast<double>(F2[row]));
+        in = eval_candidate<kAvg>(a, hkl, F2, rec, s_R[wib][slot], row, spot);
       }
 #pragma unroll
       for (int o = 0; o < kOT; ++o) {
@@ -194,13 +204,12 @@ __global__ __launch_bounds__(kSimThreads, sim_min_waves(kAvg, kLines)) void simu
         if (m == 0) continue;
         if (mine) {
           const int pos = cnt[o] + mask_rank(m);
-          lmax[o] = fmaxf(lmax[o], I);
-          lmin[o] = fminf(lmin[o], I);
+          lmax[o] = fmaxf(lmax[o], spot.w);
+          lmin[o] = fminf(lmin[o], spot.w);
           if (pos < cap) {
             const size_t off = (size_t)(o0 + o) * cap + pos;
             idx_out[off] = row;
-            spot_out[off] = make_float4(static_cast<float>(x), static_cast<float>(y),
-                                       static_cast<float>(z), I);
+            spot_out[off] = spot;
           }
         }
         cnt[o] += __popcll(m);
@@ -452,6 +461,323 @@ __global__ __launch_bounds__(kSimThreads, sim_min_waves(kAvg, kLines)) void simu
   }
 }
 
+// ---------------------------------------------------------------------------
+// Few orientations: a block of 1, 2, 4 or 8 waves per orientation.
+//
+// With a wave per four orientations, 4,096 orientations are 1,024 waves, one
+// per SIMD with nothing to hide its latencies, and 64 are 16 waves.  Here the
+// waves of a block take consecutive parts of one orientation's rows: a step
+// is 256 candidates per wave in row order, pretested into the wave's queue,
+// evaluated in FP64 up to 64 at a time, the survivors kept in registers until
+// one barrier has published every wave's count, then written at their place.
+// With a line index a chunk is a line per thread (row interval, block prefix
+// sum), and its candidates are taken in steps.
+// The rows tested, their order and every value are those of simulate_kernel.
+// ---------------------------------------------------------------------------
+
+constexpr int kCoopPer = 4;                      // candidates per lane and step
+constexpr int kCoopWaveStep = kCoopPer * kWave;  // candidates per wave and step
+
+template <bool kLines, int kCoopWaves>
+__global__ __launch_bounds__(kCoopWaves *kWave, 4) void simulate_coop_kernel(SimArgs a) {
+  constexpr int kCoopThreads = kCoopWaves * kWave;
+  constexpr int kCoopStep = kCoopWaves * kCoopWaveStep;
+  constexpr int kLW = kLines ? kCoopThreads : 1;
+  __shared__ int s_queue[kCoopWaves][kCoopWaveStep];
+  __shared__ int s_P[kLW], s_rb[kLW];
+  __shared__ float s_eA[kLW], s_eB[kLW], s_wA[kLW], s_wB[kLW];
+  __shared__ int s_sum[kCoopWaves];
+  __shared__ int s_cnt[2][kCoopWaves];
+  __shared__ double s_R[9], s_abc[4];
+  __shared__ float s_mx[kCoopWaves], s_mn[kCoopWaves];
+  const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
+  const dsx_phase_desc &d = a.single;
+  const int4 *hkl = reinterpret_cast<const int4 *>(d.hkl);
+  const float4 *g4 = reinterpret_cast<const float4 *>(d.g4);
+  const float *F2 = d.F2;
+  const double *rec = d.rec;
+  const int n_refl = d.n_refl, cap = d.cap, n_lines = d.n_lines;
+  const int4 *lines = reinterpret_cast<const int4 *>(d.lines);
+  const float two_k = 2.0f * a.k_f;
+  const double two_kd = static_cast<double>(two_k);
+  const float pre_thr = pretest_threshold(a.me, a.k, d.g_max, a.sin_phi);
+  // Under precession the band of a row widens with its own |g| (|e| <= 2 k
+  // (me + r sin(phi)), r <= |g|), not with the table's largest: a row's
+  // threshold is pre0 + pre1 |g|, at most pre_thr.  64,000 -> 48,000 FP64
+  // candidates per orientation of the 500-atom cell at 1 degree.
+  const float pre0 = pretest_threshold(a.me, a.k, d.g_max, 0.0);
+  const float pre1 = static_cast<float>(1.05 * 1.1 * a.sin_phi * (2.0 * a.k + d.g_max));
+  auto passes = [&](float e, float w) {  // w = |g|^2
+    const float t = pre1 > 0.0f ? fmaf(pre1, __builtin_amdgcn_sqrtf(fmaxf(w, 0.0f)), pre0) : pre_thr;
+    return fabsf(e) < t;
+  };
+  const double thr = static_cast<double>(pre_thr) * (1.0 + 1e-6);
+  const double c2 = rec[2] * rec[2] + rec[5] * rec[5] + rec[8] * rec[8];
+  const float c2f = static_cast<float>(c2);
+  int *queue = s_queue[wid];
+
+  for (int o = blockIdx.x; o < d.n_orient; o += gridDim.x) {
+    const double *b = d.Rt + static_cast<size_t>(o) * 9;
+    if (tid < 9) s_R[tid] = b[tid];
+    if (kLines && tid < 4) {
+      const int cc = tid < 3 ? tid : 2;
+      double v = b[6] * rec[cc] + b[7] * rec[3 + cc] + b[8] * rec[6 + cc];
+      if (tid == 3) v = fabs(v) < 1e-200 ? 0.0 : 1.0 / v;
+      s_abc[tid] = v;
+    }
+    lds_sync();
+    const float r0 = static_cast<float>(s_R[6]), r1 = static_cast<float>(s_R[7]),
+                r2 = static_cast<float>(s_R[8]);
+    int *idx_out = d.idx + static_cast<size_t>(o) * cap;
+    float4 *spot_out = reinterpret_cast<float4 *>(d.spots) + static_cast<size_t>(o) * cap;
+    int base = 0, buf = 0;
+    float lmax = 0.0f, lmin = __builtin_huge_valf();
+
+    // Evaluate the wave's queue of q candidates, publish the count, and write
+    // the survivors at their place in the list (one block barrier).
+    auto finish_step = [&](int q) {
+      float4 spot[kCoopPer];
+      int row[kCoopPer], rank[kCoopPer];
+      int cnt = 0;
+#pragma unroll
+      for (int k = 0; k < kCoopPer; ++k) {
+        rank[k] = -1;
+        if (k * kWave >= q) continue;  // uniform
+        bool in = false;
+        if (k * kWave + lane < q) {
+          row[k] = queue[k * kWave + lane];
+          in = eval_candidate<false>(a, hkl, F2, rec, s_R, row[k], spot[k]);
+        }
+        const uint64_t m = __ballot(in);
+        if (in) {
+          rank[k] = cnt + mask_rank(m);
+          lmax = fmaxf(lmax, spot[k].w);
+          lmin = fminf(lmin, spot[k].w);
+        }
+        cnt += __popcll(m);
+      }
+      if (lane == 0) s_cnt[buf][wid] = cnt;
+      lds_sync();
+      int at = base;
+#pragma unroll
+      for (int w = 0; w < kCoopWaves; ++w) {
+        const int c = s_cnt[buf][w];
+        if (w < wid) at += c;
+        base += c;
+      }
+      buf ^= 1;  // rewritten two steps on, after every wave has read it
+#pragma unroll
+      for (int k = 0; k < kCoopPer; ++k) {
+        const int pos = at + rank[k];
+        if (rank[k] >= 0 && pos < cap) {
+          idx_out[pos] = row[k];
+          spot_out[pos] = spot[k];
+        }
+      }
+    };
+    auto wave_sync = [&]() {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    };
+
+    if (kLines) {
+      const double al = s_abc[0], be = s_abc[1], ga = s_abc[2], inv = s_abc[3];
+      for (int l0 = 0; l0 < n_lines; l0 += kCoopThreads) {
+        // the rows of this thread's line that can pass the pretest (as
+        // load_group of simulate_kernel)
+        const int j = l0 + tid;
+        int first = 0, len = 0, t0 = 0;
+        double eA = 0.0, eB = 0.0, wA = 0.0, wB = 0.0;
+        if (j < n_lines) {
+          const int4 e0 = lines[2 * static_cast<size_t>(j)], e1 = lines[2 * static_cast<size_t>(j) + 1];
+          first = e0.x;
+          const int nrow = e0.y;
+          const double hx = e0.z, hy = e0.w, hz = e1.x;
+          const double wmin = __int_as_float(e1.y), wmax = __int_as_float(e1.z);
+          const double zm = 1e-5 * (1.0 + sqrt(wmax));
+          const double zlo = (wmin - thr) / two_kd - zm, zhi = (wmax + thr) / two_kd + zm;
+          const double gx = rec[0] * hx + rec[1] * hy + rec[2] * hz;
+          const double gy = rec[3] * hx + rec[4] * hy + rec[5] * hz;
+          const double gz = rec[6] * hx + rec[7] * hy + rec[8] * hz;
+          const float w0 = static_cast<float>(gx * gx + gy * gy + gz * gz);
+          const float cd = static_cast<float>(gx * rec[2] + gy * rec[5] + gz * rec[8]);
+          const double zt = hx * al + hy * be + hz * ga;
+          if (inv == 0.0) {  // line perpendicular to the beam: all rows or none
+            if (zt >= zlo && zt <= zhi) len = nrow;
+          } else {
+            const double q1 = (zt - zhi) * inv, q2 = (zt - zlo) * inv;
+            const double tlo = fmax(ceil(fmin(q1, q2)), 0.0);
+            const double thi = fmin(floor(fmax(q1, q2)), static_cast<double>(nrow - 1));
+            if (thi >= tlo) {
+              t0 = static_cast<int>(tlo);
+              len = static_cast<int>(thi - tlo) + 1;
+            }
+          }
+          const double tt = static_cast<double>(t0);
+          const double eb = two_kd * ga - 2.0 * static_cast<double>(cd);
+          eA = (static_cast<double>(w0) - two_kd * zt) + tt * (eb + c2 * tt);
+          eB = eb + 2.0 * c2 * tt;
+          wB = -2.0 * static_cast<double>(cd) + 2.0 * c2 * tt;
+          wA = static_cast<double>(w0) + tt * (c2 * tt - 2.0 * static_cast<double>(cd));
+        }
+        const int incl = wave_inclusive_scan(len);
+        if (lane == kWave - 1) s_sum[wid] = incl;
+        lds_sync();
+        int before = 0, total = 0;
+#pragma unroll
+        for (int w = 0; w < kCoopWaves; ++w) {
+          const int c = s_sum[w];
+          if (w < wid) before += c;
+          total += c;
+        }
+        s_P[tid] = before + incl - len;
+        s_rb[tid] = first + t0;
+        s_eA[tid] = static_cast<float>(eA);
+        s_eB[tid] = static_cast<float>(eB);
+        s_wA[tid] = static_cast<float>(wA);
+        s_wB[tid] = static_cast<float>(wB);
+        lds_sync();
+        for (int s0 = 0; s0 < total; s0 += kCoopStep) {
+          int q = 0;
+#pragma unroll
+          for (int k = 0; k < kCoopPer; ++k) {
+            const int w0 = s0 + wid * kCoopWaveStep + k * kWave;
+            if (w0 >= total) break;  // uniform
+            const int c = w0 + lane;
+            int src = 0;  // the last line that starts at or before candidate c holds it
+#pragma unroll
+            for (int step = kCoopThreads / 2; step > 0; step >>= 1)
+              if (s_P[src + step] <= c) src += step;
+            const int u = c - s_P[src];
+            const int row = s_rb[src] + u;
+            const bool v = c < total && static_cast<unsigned>(row) < static_cast<unsigned>(n_refl);
+            const float uf = static_cast<float>(u);
+            const float e = fmaf(fmaf(c2f, uf, s_eB[src]), uf, s_eA[src]);
+            const float w = pre1 > 0.0f ? fmaf(fmaf(c2f, uf, s_wB[src]), uf, s_wA[src]) : 0.0f;
+            const bool pre = v && passes(e, w);
+            const uint64_t m = __ballot(pre);
+            if (pre) queue[q + mask_rank(m)] = row;
+            q += __popcll(m);
+          }
+          wave_sync();
+          finish_step(q);
+        }
+      }
+    } else {
+      for (int s0 = 0; s0 < n_refl; s0 += kCoopStep) {
+        const int w0 = s0 + wid * kCoopWaveStep;
+        float4 g[kCoopPer];
+#pragma unroll
+        for (int k = 0; k < kCoopPer; ++k) {
+          const int i = w0 + k * kWave + lane;
+          g[k] = i < n_refl ? g4[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+        int q = 0;
+#pragma unroll
+        for (int k = 0; k < kCoopPer; ++k) {
+          const int i = w0 + k * kWave + lane;
+          const float zf = fmaf(r0, g[k].x, fmaf(r1, g[k].y, r2 * g[k].z));
+          const bool pre = i < n_refl && passes(fmaf(-two_k, zf, g[k].w), g[k].w);
+          const uint64_t m = __ballot(pre);
+          if (pre) queue[q + mask_rank(m)] = i;
+          q += __popcll(m);
+        }
+        wave_sync();
+        finish_step(q);
+      }
+    }
+
+    // ---- relative cut (as simulate_kernel), the whole block compacting -------
+    lmax = wave_max(lmax);
+    lmin = wave_min(lmin);
+    if (lane == 0) {
+      s_mx[wid] = lmax;
+      s_mn[wid] = lmin;
+    }
+    __syncthreads();  // the list in global memory too
+    float mx = s_mx[0], mn = s_mn[0];
+#pragma unroll
+    for (int w = 1; w < kCoopWaves; ++w) {
+      mx = fmaxf(mx, s_mx[w]);
+      mn = fminf(mn, s_mn[w]);
+    }
+    const int nw = min(base, cap);
+    int final_count = nw;
+    const float cut = mx * a.min_I;
+    if (base > 0 && mx > 0.0f && !(mn > cut)) {
+      int kept = 0;
+      for (int c0 = 0; c0 < nw; c0 += kCoopThreads) {
+        const int j = c0 + tid;
+        float4 sp = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        int id = 0;
+        if (j < nw) {
+          sp = spot_out[j];
+          id = idx_out[j];
+        }
+        const bool keep = j < nw && sp.w > cut;
+        const uint64_t m = __ballot(keep);
+        if (lane == 0) s_cnt[buf][wid] = __popcll(m);
+        __syncthreads();  // every entry of the chunk is read before any is written
+        int at = kept;
+#pragma unroll
+        for (int w = 0; w < kCoopWaves; ++w) {
+          const int c = s_cnt[buf][w];
+          if (w < wid) at += c;
+          kept += c;
+        }
+        buf ^= 1;
+        if (keep) {
+          const int pos = at + mask_rank(m);
+          spot_out[pos] = sp;
+          idx_out[pos] = id;
+        }
+      }
+      final_count = kept;
+    }
+    if (tid == 0) {
+      d.count[o] = final_count;
+      d.ncand[o] = base;
+      d.maxI[o] = mx;
+    }
+    __syncthreads();  // s_R, s_mx and the counts are rewritten for the next orientation
+  }
+}
+
+// Waves per orientation of simulate_coop_kernel, 0: simulate_kernel's wave per
+// four orientations (which shares each row or line among them).  As many
+// waves as fill four per SIMD, in us, by waves (wave per four: last):
+//   500-atom precession (14,306 lines)  16: 451 (8) 776 (4) 2,287 (1) 8,647
+//     1,024: 1,139 (8) 1,164 (4) 1,563 (2) 8,519   2,048: 2,029 (2) 2,640 (1)
+//     4,096: 4,308 (2) 3,669 (1) 9,134   16,384: 13,031 (1) 13,557
+//     (before the per-row threshold: with it 3,334 (1) and 12,015 (1))
+//   40-atom library (1,186 lines)  64: 18 (8) 41 (1) 87   2,000: 68 (8) 38 (2)
+//     51 (1) 93   4,096: 67 (1) 97   8,192: 122 (1) 104
+//   17 A cell (3,482 lines)  8,000: 381 (1) 460   20,000: 877 (1) 866
+//   24-atom cell, full sweep of 4,614 rows  512: 11 (8) 29 (1) 45   2,048: 23
+//     (2) 31 (1) 45   4,096: 40 (1) 48   8,192: 76 (1) 52
+//   256 rows  500: 12 (8) 9 (2) 11   4,000: 10 (1) 11   20,000: 21 (1) 16
+// Under precession with long line lists one wave stays ahead (the per-row
+// threshold saves a quarter of the candidates): 20,000 14,622 (1) 20,271.
+static int coop_waves(int n_orient, int n_refl, int n_lines, bool precession) {
+  const int limit = n_lines >= 2048 ? (precession ? 1 << 30 : 16384) : 6144;
+  if (n_orient > limit) return 0;
+  int w = n_orient <= 512 ? 8 : (n_orient <= 1280 ? 4 : (n_orient <= 2560 ? 2 : 1));
+  while (w > 1 && n_refl < w * 2 * kWave) w /= 2;  // at least two rows per lane
+  return w;
+}
+
+template <bool kLines>
+static void launch_coop(int waves, const SimArgs &a, hipStream_t s) {
+  const dim3 blocks(static_cast<unsigned>(a.single.n_orient)), threads(static_cast<unsigned>(waves * kWave));
+  switch (waves) {
+    case 8: hipLaunchKernelGGL((simulate_coop_kernel<kLines, 8>), blocks, threads, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((simulate_coop_kernel<kLines, 4>), blocks, threads, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((simulate_coop_kernel<kLines, 2>), blocks, threads, 0, s, a); break;
+    default: hipLaunchKernelGGL((simulate_coop_kernel<kLines, 1>), blocks, threads, 0, s, a);
+  }
+}
+
 static int check_physics(const dsx_sim_params *p, const char *name) {
   const bool averaged = p->shape_model >= DSX_SF_PRECESSION_AVG + DSX_SF_LINEAR &&
                         p->shape_model <= DSX_SF_PRECESSION_AVG + DSX_SF_BINARY;
@@ -547,7 +873,14 @@ extern "C" int dsx_simulate(const int *hkl_d, const float *g4_d, const float *F2
   // the averaged-precession model keeps the full sweep: its FP64 evaluation
   // dominates, and the line state would cost it occupancy
   const bool avg = p->shape_model >= DSX_SF_PRECESSION_AVG;
-  if (lines_d && !avg && lines_pay(n_refl, n_lines))
+  const bool use_lines = lines_d && !avg && lines_pay(n_refl, n_lines);
+  const int coop = avg ? 0 : coop_waves(n_orient, n_refl, use_lines ? n_lines : 0, a.precession != 0);
+  if (coop > 0) {
+    if (use_lines)
+      launch_coop<true>(coop, a, s);
+    else
+      launch_coop<false>(coop, a, s);
+  } else if (use_lines)
     hipLaunchKernelGGL((simulate_kernel<false, false, true>), grid, dim3(kSimThreads), 0, s, a);
   else if (avg)
     hipLaunchKernelGGL((simulate_kernel<false, true, false>), grid, dim3(kSimThreads), 0, s, a);

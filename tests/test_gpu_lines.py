@@ -245,3 +245,56 @@ def test_line_sweep_random_cells(seed):
         pytest.skip(f"lines average {tab.n / tab.n_lines:.1f} rows: the kernel keeps the full sweep")
     a, b = sweep_and_lines(tab, rotations(384, 2000 + seed), st, rr)
     assert_same_batches(a, b)
+
+
+@pytest.mark.parametrize("name,spec,rr,wdb,lines,kw", [
+    ("al, extinct rows cut", P.al_c0, 1.5, True, False, {"minimum_intensity": 1e-3}),
+    ("hexagonal", hexagonal, 2.5, False, True, {"shape_model": "linear"}),
+    ("ortho40", P.ortho40, 2.0, True, True, {}),
+    ("ortho40 sweep, precession", P.ortho40, 2.0, False, False, {"precession_angle": 1.0}),
+    ("ortho40 precession", P.ortho40, 2.5, True, True, {"precession_angle": 3.0}),
+    ("ortho40 binary precession", P.ortho40, 2.5, False, True,
+     {"precession_angle": 0.4, "shape_model": "binary"}),
+    ("few rows", P.al_c0, 0.6, False, False, {"max_excitation_error": 0.05}),
+])
+def test_few_orientations_equal_the_large_batch(name, spec, rr, wdb, lines, kw):
+    """The spot kernel gives small batches a block of 8, 4, 2 or 1 waves per
+    orientation and large ones a wave per four: leading parts of one batch of
+    7,000, below and above each width's limit, are its rows bit for bit."""
+    from diffsims_amd import engine
+
+    st = engine.SimSettings(**{"max_excitation_error": 0.02, **kw})
+    tab = engine.build_phase_table(P.to_arrays(spec()), rr, wdb)
+    if not lines:
+        tab = dataclasses.replace(tab, lines=None)
+    else:
+        assert uses_lines(tab)
+    Rt = engine.rotation_matrices_to_device(rotations(6992, 5))
+    big = engine.simulate(tab, Rt, st, rr)
+    assert int(big.count.sum()) > 0
+    for n in (1, 5, 512, 513, 1280, 1281, 2560, 2561, 6144):
+        print(f"{name}: {n} of 7000", flush=True)
+        part = engine.simulate(tab, Rt[:n].contiguous(), st, rr, cap=big.cap)
+        assert_same_batches(part, engine.SpotBatch(tab, big.idx[:n], big.spots[:n], big.count[:n],
+                                                   big.ncand[:n], big.maxI[:n], big.cap))
+
+
+def test_few_orientations_with_a_short_list():
+    """Lists shorter than the candidates: the first `cap` survivors and the
+    full candidate count, as from the large batch."""
+    from diffsims_amd import engine
+
+    tab = engine.build_phase_table(P.to_arrays(P.ortho40()), 2.5, False)
+    st = engine.SimSettings(max_excitation_error=0.02)
+    Rt = engine.rotation_matrices_to_device(rotations(6992, 8))
+    out = []
+    for n in (7000, 40, 1500):
+        b = engine.empty_batch(tab, n, 50, Rt.device)
+        engine.simulate_into(tab, Rt[:n].contiguous(), st, b)
+        out.append(b)
+    big = out[0]
+    assert int(big.ncand.max()) > 50
+    for b in out[1:]:
+        n = b.n
+        assert_same_batches(b, engine.SpotBatch(tab, big.idx[:n], big.spots[:n], big.count[:n],
+                                                big.ncand[:n], big.maxI[:n], 50))
