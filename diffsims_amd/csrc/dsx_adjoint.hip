@@ -22,11 +22,9 @@
 //   orientation and the reciprocal basis): dL/dRt of the pattern, dL/d|F|^2
 //   per reflection (atomics) and dL/drec through g (block partials, summed by
 //   sum_partials_kernel in a fixed order).
-// render_adjoint_large_kernel: the same for spot lists longer than the LDS
-//   spot table: their bins live in a per-block workspace and the spots pass
-//   through LDS in chunks; each spot's gathered sums are added into its
-//   position of the pattern's gsum row (float atomics over the strips it
-//   spans), which spot_chain_kernel then reads like the small kernel's.
+// render_tiles_kernel (dsx_tiles.h): the same for spot lists longer than the
+//   LDS spot table, on the matrix cores; its gsum rows go through the same
+//   spot_chain_kernel.
 // structure_factor_adjoint_kernel (one thread per reflection)
 //   recomputes F(hkl) and reduces dL/d|F|^2 into dL/dxyz and dL/dB per atom
 //   and into dL/d(rec) through |g|.
@@ -36,6 +34,7 @@
 #include "dsx_internal.h"
 #include "dsx_physics.h"
 #include "dsx_splat.h"
+#include "dsx_tiles.h"
 
 namespace dsx {
 
@@ -43,16 +42,7 @@ constexpr int kAdjThreads = 512;
 constexpr int kAdjWaves = kAdjThreads / kWave;
 constexpr int kAdjMaxSpots = 1024;   // longest spot list of the two-blocks-per-CU kernel
 constexpr int kAdjMaxStrips = 256;
-// The large-pattern kernel splits its strip bins by clip-box width (<= 4,
-// <= 8, wider columns), so the (spot, column) items of a class run with that
-// class's column count instead of the pattern's widest box.  (Small patterns
-// hold few spots per strip; one pass per strip fills the waves better.)
-constexpr int kWidthClasses = 3;
 constexpr int kAdjBinCap = 4096;
-// large-pattern kernel: one 64 KB strip buffer (the splat's fixed-point words
-// in pass 1, G in pass 2) and as many LDS spot slots as the rest holds
-constexpr int kAdjStripBytes = 64 * 1024;
-constexpr int kAdjLargeMaxSlots = 4096;
 constexpr int kPixBits = 22;  // argmax key: value << 22 | (2^22 - 1 - pixel)
 constexpr int kNRed = 20;     // block sums: loss, sum G P, dRt[9], dL/drec[9]
 constexpr int kAdjTile = 16;      // tile edge of the fixed-point bound
@@ -60,8 +50,7 @@ constexpr int kAdjMaxTiles = 1024;
 constexpr int kAdjMaxCand = 16;    // candidate tiles of the maximum search
 constexpr int kAdjCandSpots = 64;  // spots touching one candidate tile
 // float4 target values each thread of the two-blocks-per-CU kernel prefetches
-// for one strip of at most kAdjSmallStripBytes / 8 pixels (the large-pattern
-// kernel, whose strips take long to splat, loads them in the read-out)
+// for one strip of at most kAdjSmallStripBytes / 8 pixels
 constexpr int kAdjPre = 4;
 constexpr int kAdjSmallStripBytes = kAdjPre * 4 * kAdjThreads * 8;
 constexpr float kAdjRange = 2040109465.6f;  // 1.9 * 2^30 units per bound
@@ -92,15 +81,18 @@ struct AdjArgs {
   float cal, cx, cy, ca, sa;
   int mirrored, normalize;
   float pref, ep, inv_s2, clip;
+  float log2_clip, two_s2_ln2, tiny_box, box_margin;  // subpixel_box_fast
+  float bound_units;        // long lists: tile-bound units of the largest spot
+  int count_waves;          // long lists: waves that count and scatter the spots
   float e2ep;  // exp(2 ep): ratio of consecutive row ratios of the Gaussian
   int strip_rows, n_strips, acc_words;
   int slots, bin_cap;       // LDS spot slots and strip-bin entries
   int mode;
   int want_grad;
   long long target_stride;  // elements between targets (0: one target for every pattern)
-  int *work;                // large patterns: per-block records, bins and boxes (may be NULL)
+  int *work;                // long lists: per-block entries (may be NULL)
   long long work_per_block; // ints
-  int work_entries;         // bin entries per block
+  int work_entries;         // entries per block
   float4 *gsum;             // per pattern and slot: A, BX, BY, list position (chain kernel input)
   int *gcount;              // per pattern: slots used
   const float *target;
@@ -113,10 +105,9 @@ struct AdjArgs {
   int *status;
 };
 
-template <int kCls>  // width classes per strip
 struct AdjShared {
-  int bin_start[kCls * kAdjMaxStrips + 1];  // bin b = kCls * strip + width class
-  int bin_fill[kCls * kAdjMaxStrips];
+  int bin_start[kAdjMaxStrips + 1];
+  int bin_fill[kAdjMaxStrips];
   int ns, cols_max;
   float wmaxf[kAdjWaves];
   long long wkey[kAdjWaves];
@@ -194,11 +185,6 @@ __device__ __forceinline__ int gauss_term(float amp, float dx, float dy, float e
   return __float2int_rn(amp * fast_exp(ep * fmaf(dy, dy, dx * dx)) * scale);
 }
 
-__device__ __forceinline__ int width_class(int w) { return w <= 4 ? 0 : (w <= 8 ? 1 : 2); }
-__device__ __forceinline__ int class_cols(int c, int cols_max) {
-  return c == 0 ? min(4, cols_max) : (c == 1 ? min(8, cols_max) : cols_max);
-}
-__device__ __forceinline__ int box_width(int xb) { return (xb & 0xffff) - (xb >> 16) + 1; }
 // it / ncols, a shift for powers of two (ncols is uniform)
 __device__ __forceinline__ int item_spot(int it, int ncols) {
   return (ncols & (ncols - 1)) == 0 ? it >> __builtin_ctz(ncols) : it / ncols;
@@ -217,10 +203,8 @@ __device__ __forceinline__ int gather_cols(int w) {
 template <bool kGather>
 __device__ __forceinline__ void strip_pass(const AdjArgs &a, const SpotTab &t, int cols_max,
                                            aacc_t *acc, const float *G, int b0, int nb,
-                                           bool binned, int y0, int y1, float scale, int tid,
-                                           float4 *hand = nullptr) {
-  // unbinned: LDS slots b0 .. b0 + nb - 1; hand: the gather adds each spot's
-  // sums into row jpos of the gradient hand-over instead of its LDS slot
+                                           bool binned, int y0, int y1, float scale, int tid) {
+  // unbinned: LDS slots b0 .. b0 + nb - 1
   const int W = a.W;
   const int ncols = cols_max;
   const int n_items = nb * ncols;
@@ -312,49 +296,15 @@ __device__ __forceinline__ void strip_pass(const AdjArgs &a, const SpotTab &t, i
       if ((ncols & (ncols - 1)) == 0 && ncols <= kWave) {
         // the run lies in this wave and this lane (c == 0) holds its sum;
         // a spot has one run per pass
-        if (hand) {
-          float *h = reinterpret_cast<float *>(hand + t.jpos[q]);
-          unsafeAtomicAdd(h, sa);
-          unsafeAtomicAdd(h + 1, sx);
-          unsafeAtomicAdd(h + 2, sy);
-        } else {
-          t.A[q] += sa;
-          t.BX[q] += sx;
-          t.BY[q] += sy;
-        }
+        t.A[q] += sa;
+        t.BX[q] += sx;
+        t.BY[q] += sy;
       } else {
         atomicAdd(&t.A[q], sa);
         atomicAdd(&t.BX[q], sx);
         atomicAdd(&t.BY[q], sy);
       }
     }
-  }
-}
-
-// Load entries [base, base + m) of a strip's global bin into LDS slots 0..m-1
-// (large patterns: more in-frame spots than the LDS holds).  The clip boxes
-// come from the per-spot cache the first scan wrote (boxes[j] = {(xlo << 16) |
-// xhi, (lo << 16) | hi}); only the pixel position is recomputed.  jpos holds
-// the spot's row of the gradient hand-over (row_of[j]) when there is one.
-__device__ __forceinline__ void load_chunk(const AdjArgs &a, const SpotTab &t, const float4 *spots,
-                                           const int *bins, const int2 *boxes, const int *row_of,
-                                           int base, int m, int tid) {
-  for (int i = tid; i < m; i += kAdjThreads) {
-    const int j = bins[base + i];
-    const float4 sp = spots[j];
-    const int2 bx = boxes[j];
-    float X, Y;
-    to_pixel(sp, a, X, Y);  // in frame: the scan that binned j tested it
-    t.I[i] = sp.w;
-    t.X[i] = X;
-    t.Y[i] = Y;
-    t.A[i] = 0.0f;
-    t.BX[i] = 0.0f;
-    t.BY[i] = 0.0f;
-    t.xb[i] = bx.x;
-    t.jpos[i] = row_of ? row_of[j] : j;
-    t.ylo[i] = static_cast<short>(bx.y >> 16);
-    t.yhi[i] = static_cast<short>(bx.y & 0xffff);
   }
 }
 
@@ -538,41 +488,19 @@ __device__ bool bounded_max_key(const AdjArgs &a, Shared &sh, const SpotTab &t, 
   return true;
 }
 
-// One pattern per block iteration.  kLarge = false: every in-frame spot fits
-// the LDS slots (the host guarantees slots >= cap) and the per-spot sums go to
-// gsum for spot_chain_kernel, which keeps the FP64 chain rule (and its
-// registers) out of this kernel.  kLarge = true: patterns may hold more
-// in-frame spots than the slots (their bins and sums live in the per-block
-// workspace) and the chain rule runs here, per pattern.
-template <bool kLarge>
+// One pattern per block iteration: every in-frame spot fits the LDS slots (the
+// host guarantees slots >= cap) and the per-spot sums go to gsum for
+// spot_chain_kernel, which keeps the FP64 chain rule (and its registers) out
+// of this kernel.
 __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
-                                             AdjShared<kLarge ? kWidthClasses : 1> &sh) {
-  constexpr int kCls = kLarge ? kWidthClasses : 1;
-  // The large-pattern kernel has one strip buffer: pass 1 splats into it, and
-  // pass 2 keeps G there while the fixed-point pixels wait in q.  The small
-  // one splats and reads out into G in the same step, so it has two.
-  float *s_G = kLarge ? reinterpret_cast<float *>(s_acc)
-                      : reinterpret_cast<float *>(s_acc + a.acc_words);
-  const SpotTab t = spot_tab(s_acc, (kLarge ? 1 : 2) * static_cast<size_t>(a.acc_words), a.slots);
+                                             AdjShared &sh) {
+  float *s_G = reinterpret_cast<float *>(s_acc + a.acc_words);
+  const SpotTab t = spot_tab(s_acc, 2 * static_cast<size_t>(a.acc_words), a.slots);
   const int tid = threadIdx.x;
   const int lane = lane_id();
   const int wid = tid / kWave;
   const int H = a.H, W = a.W;
   const size_t HW = static_cast<size_t>(H) * W;
-  // large-pattern workspace of this block: int bins[entries] | int2
-  // boxes[cap] (clip boxes cached by the first scan) | int rows[cap] (each
-  // in-frame spot's row of the gradient hand-over) | int q[H W] (the
-  // fixed-point pattern between the splat and the read-out when there is no
-  // pattern buffer to hold it), each part 16-byte aligned
-  int *wblock = kLarge && a.work ? a.work + (size_t)blockIdx.x * a.work_per_block : nullptr;
-  int *wbins = wblock;
-  int2 *wbox = wblock ? reinterpret_cast<int2 *>(wbins + ((static_cast<size_t>(a.work_entries) + 3) &
-                                                          ~static_cast<size_t>(3)))
-                      : nullptr;
-  int *wrow = wblock ? reinterpret_cast<int *>(wbox) + ((2 * static_cast<size_t>(a.cap) + 3) &
-                                                         ~static_cast<size_t>(3))
-                     : nullptr;
-  int *wq = wblock ? wrow + ((static_cast<size_t>(a.cap) + 3) & ~static_cast<size_t>(3)) : nullptr;
   for (int i = tid; i < a.acc_words; i += kAdjThreads) s_acc[i] = 0;
   lds_sync();
 
@@ -584,38 +512,23 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
       sh.cols_max = 1;
       sh.qstar = 0;
     }
-    for (int b = tid; b <= kCls * kAdjMaxStrips; b += kAdjThreads) sh.bin_start[b] = 0;
+    for (int b = tid; b <= kAdjMaxStrips; b += kAdjThreads) sh.bin_start[b] = 0;
     lds_sync();
 
     // ---- 1. spots in frame with their clip boxes --------------------------
-    // every such spot counts in the strip bins and the maximum; the first
-    // `slots` also go to LDS (all of them unless the pattern is large)
     float tmax = 0.0f;
-    float4 *gsp = kLarge && a.gsum ? a.gsum + (size_t)p * a.cap : nullptr;
     for (int j = tid; j < n; j += kAdjThreads) {
       const float4 sp = spots[j];
       float X = 0.0f, Y = 0.0f;
       int lo = 1, hi = 0, xlo = 0, xhi = 0;
       const bool in = to_pixel(sp, a, X, Y) &&
-                      subpixel_box(sp.w, X, Y, a.pref, a.ep, a.clip, H, W, lo, hi, xlo, xhi);
-      // the large-pattern scans below read the cached box ({0, 1 << 16}: none)
-      if (kLarge && wbox) wbox[j] = in ? make_int2((xlo << 16) | xhi, (lo << 16) | hi) : make_int2(0, 1 << 16);
+                      subpixel_box_fast(sp.w, X, Y, a, lo, hi, xlo, xhi);
       if (!in) continue;
       tmax = fmaxf(tmax, fabsf(sp.w) * a.pref);
       atomicMax(&sh.cols_max, xhi - xlo + 1);
-      const int wc = kCls == 1 ? 0 : width_class(xhi - xlo + 1);
       for (int s = lo / a.strip_rows; s <= hi / a.strip_rows; ++s)
-        atomicAdd(&sh.bin_start[kCls * s + wc + 1], 1);
+        atomicAdd(&sh.bin_start[s + 1], 1);
       const int q = atomicAdd(&sh.ns, 1);
-      if (kLarge) {
-        // gradients: in-frame spot q's gathered sums start at zero in row q
-        // of the hand-over (which names its spot j)
-        if (gsp) {
-          gsp[q] = make_float4(0.0f, 0.0f, 0.0f, __int_as_float(j));
-          wrow[j] = q;
-        }
-        continue;  // its chunks are loaded per strip
-      }
       t.I[q] = sp.w;
       t.X[q] = X;
       t.Y[q] = Y;
@@ -629,17 +542,14 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
     }
     tmax = wave_max(tmax);
     if (lane == 0) sh.wmaxf[wid] = tmax;
-    if (kLarge)
-      __syncthreads();  // the cached boxes in global memory, block-visible
-    else
-      lds_sync();
-    const int ns_all = sh.ns;
+    lds_sync();
+    const int ns = sh.ns;
     float pmax = 0.0f;
     for (int w = 0; w < kAdjWaves; ++w) pmax = fmaxf(pmax, sh.wmaxf[w]);
     float scale = 1.0f;  // set from the tile bounds below
 
     // ---- 2. strip bins ----------------------------------------------------
-    const int n_bins = kCls * a.n_strips;
+    const int n_bins = a.n_strips;
     if (tid == 0) {
       int acc = 0;
       for (int b = 0; b < n_bins; ++b) {
@@ -649,39 +559,14 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
     }
     lds_sync();
     const int entries = sh.bin_start[n_bins];
-    // large-pattern kernel: the bins live in the caller's workspace and the
-    // spots pass through LDS in chunks
-    const bool large = kLarge;
-    const bool fits = !large || (wbins != nullptr && entries <= a.work_entries);
-    if (tid == 0 && a.status) a.status[p] = fits ? 0 : 1;
-    const int ns = large ? 0 : ns_all;  // spots held in LDS for the whole pattern
-    const bool binned = !large && entries <= a.bin_cap;
+    if (tid == 0 && a.status) a.status[p] = 0;
+    const bool binned = entries <= a.bin_cap;
     for (int b = tid; b < n_bins; b += kAdjThreads) sh.bin_fill[b] = sh.bin_start[b];
     lds_sync();
-    if (kLarge && !fits) {
-      // no room: the pattern is reported in status and left as zeros
-      if (a.pattern)
-        for (size_t i = tid; i < HW; i += kAdjThreads) a.pattern[(size_t)p * HW + i] = 0.0f;
-      if (tid < 9 && a.want_grad) a.dRt[(size_t)p * 9 + tid] = 0.0;
-      if (tid == 0 && a.loss) a.loss[p] = 0.0f;
-      lds_sync();
-      continue;
-    }
-    if (large) {
-      for (int j = tid; j < n; j += kAdjThreads) {
-        const int2 bx = wbox[j];
-        const int lo = bx.y >> 16, hi = bx.y & 0xffff;
-        if (lo > hi) continue;  // not in frame
-        const int wc = kCls == 1 ? 0 : width_class(box_width(bx.x));
-        for (int s = lo / a.strip_rows; s <= hi / a.strip_rows; ++s)
-          wbins[atomicAdd(&sh.bin_fill[kCls * s + wc], 1)] = j;
-      }
-      __syncthreads();  // bins in global memory, block-visible
-    } else if (binned) {
+    if (binned) {
       for (int q = tid; q < ns; q += kAdjThreads) {
-        const int wc = kCls == 1 ? 0 : width_class(box_width(t.xb[q]));
         for (int s = t.ylo[q] / a.strip_rows; s <= t.yhi[q] / a.strip_rows; ++s) {
-          const int pos = atomicAdd(&sh.bin_fill[kCls * s + wc], 1);
+          const int pos = atomicAdd(&sh.bin_fill[s], 1);
           t.bin[pos] = static_cast<short>(q);
         }
       }
@@ -706,18 +591,9 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
         for (int ty = lo / kAdjTile; ty <= hi / kAdjTile; ++ty)
           for (int tx = xlo / kAdjTile; tx <= xhi / kAdjTile; ++tx) atomicAdd(&tile_u[ty * ntx + tx], u);
       };
-      if (!large) {
-        for (int q = tid; q < ns; q += kAdjThreads) {
-          if (fabsf(t.I[q]) * a.pref == pmax) sh.qstar = q;  // the brightest spot (any of a tie)
-          add_bound(t.I[q], t.ylo[q], t.yhi[q], t.xb[q] >> 16, t.xb[q] & 0xffff);
-        }
-      } else {
-        for (int j = tid; j < n; j += kAdjThreads) {
-          const int2 bx = wbox[j];
-          const int lo = bx.y >> 16, hi = bx.y & 0xffff;
-          if (lo > hi) continue;  // not in frame
-          add_bound(spots[j].w, lo, hi, bx.x >> 16, bx.x & 0xffff);
-        }
+      for (int q = tid; q < ns; q += kAdjThreads) {
+        if (fabsf(t.I[q]) * a.pref == pmax) sh.qstar = q;  // the brightest spot (any of a tie)
+        add_bound(t.I[q], t.ylo[q], t.yhi[q], t.xb[q] >> 16, t.xb[q] & 0xffff);
       }
       int lu = 0;
       if (tiles) {
@@ -736,75 +612,21 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
       scale = U > 0.0f ? kAdjRange / (U * 1.00001f) : 1.0f;
     }
 
-    // splat (or gather) strip s: every LDS-resident spot of its bin, or, for a
-    // large pattern, its global bin chunk by chunk.  A strip whose bin fits
-    // one chunk is gathered from the slots its splat just loaded.  Large
-    // patterns store each entry's gathered sums in the workspace record of
-    // the entry (no read-modify-write; every entry belongs to one strip).
-    auto pass_range = [&](bool gather, int ncols, int b0, int nb, bool bin, int y0, int y1) {
+    // splat (or gather) strip s: every spot of its bin
+    auto strip_spots = [&](int s, bool gather, int y0, int y1) {
+      const int b0 = binned ? sh.bin_start[s] : 0;
+      const int nb = binned ? sh.bin_start[s + 1] - b0 : ns;
       if (nb <= 0) return;
       if (gather)
-        strip_pass<true>(a, t, gather_cols(ncols), s_acc, s_G, b0, nb, bin, y0, y1, scale, tid,
-                         large ? gsp : nullptr);
+        strip_pass<true>(a, t, gather_cols(cols_max), s_acc, s_G, b0, nb, binned, y0, y1, scale, tid);
       else
-        strip_pass<false>(a, t, ncols, s_acc, nullptr, b0, nb, bin, y0, y1, scale, tid);
-    };
-    auto strip_spots = [&](int s, bool gather, int y0, int y1) {
-      const int bs = kCls * s;
-      if (!large) {
-        // few spots per strip: one pass over the strip's classes together
-        // fills the waves better than a pass per class
-        if (binned)
-          pass_range(gather, cols_max, sh.bin_start[bs],
-                     sh.bin_start[bs + kCls] - sh.bin_start[bs], true, y0, y1);
-        else
-          pass_range(gather, cols_max, 0, ns, false, y0, y1);
-        return;
-      }
-      const int e0 = sh.bin_start[bs], e1 = sh.bin_start[bs + kCls];
-      for (int c0 = e0; c0 < e1; c0 += a.slots) {
-        const int m = min(a.slots, e1 - c0);
-        load_chunk(a, t, spots, wbins, wbox, gsp ? wrow : nullptr, c0, m, tid);
-        lds_sync();
-        // the chunk's entries in slots 0..m-1, ordered by width class
-        auto classes = [&](bool g) {
-          for (int c = 0; c < kCls; ++c) {
-            const int lo = max(c0, sh.bin_start[bs + c]);
-            const int hi = min(c0 + m, sh.bin_start[bs + c + 1]);
-            pass_range(g, kCls == 1 ? cols_max : class_cols(c, cols_max), lo - c0, hi - lo, false,
-                       y0, y1);
-          }
-        };
-        if (gather) {
-          // with boxes up to a wave wide every run lies in one wave and the
-          // gather itself adds the sums into the hand-over rows; wider boxes
-          // collect theirs in the LDS slots, added here (a spot's strips add
-          // in turn; the first scan zeroed its row behind a barrier)
-          classes(true);
-          lds_sync();
-          if (cols_max > kWave) {
-            for (int i = tid; i < m; i += kAdjThreads) {
-              const float A = t.A[i], BX = t.BX[i], BY = t.BY[i];
-              if (A != 0.0f || BX != 0.0f || BY != 0.0f) {
-                float *g = reinterpret_cast<float *>(gsp + t.jpos[i]);
-                unsafeAtomicAdd(g, A);
-                unsafeAtomicAdd(g + 1, BX);
-                unsafeAtomicAdd(g + 2, BY);
-              }
-            }
-            lds_sync();  // the next chunk overwrites the slots
-          }
-        } else {
-          classes(false);
-          lds_sync();  // the next chunk overwrites the slots
-        }
-      }
+        strip_pass<false>(a, t, cols_max, s_acc, nullptr, b0, nb, binned, y0, y1, scale, tid);
     };
 
     // ---- 3. pass A: maximum and its first pixel -----------------------------
     long long key = 0;
     bool have_key = false;
-    if (a.normalize && ns_all > 0 && tiles && !large &&
+    if (a.normalize && ns > 0 && tiles &&
         a.acc_words * sizeof(float) >= sizeof(short) * kAdjMaxCand * kAdjCandSpots) {
       have_key = bounded_max_key(a, sh, t, tile_u, reinterpret_cast<short(*)[kAdjCandSpots]>(s_G),
                                  ntx, n_tiles, ns, scale, unit, tid, lane, wid, key);
@@ -813,64 +635,11 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
       for (int ti = tid; ti < n_tiles; ti += kAdjThreads) tile_u[ti] = 0;
       lds_sync();
     }
-    // A large pattern is splatted once, into the strip buffer (zero again
-    // from here): each strip's fixed-point values go to q (the pattern buffer
-    // when there is one, else the block's workspace) while the maximum key is
-    // formed, and pass B reads them back.  (Small patterns find the maximum
-    // from the tile bounds and splat in pass B.)
-    int *q = large ? (a.pattern ? reinterpret_cast<int *>(a.pattern + (size_t)p * HW) : wq)
-                   : nullptr;
-    if (large) {
+    if (a.normalize && ns > 0 && !have_key) {
       for (int s = 0; s < a.n_strips; ++s) {
         const int y0 = s * a.strip_rows;
         const int y1 = min(H, y0 + a.strip_rows);
-        if (sh.bin_start[kCls * (s + 1)] == sh.bin_start[kCls * s]) continue;
-        strip_spots(s, false, y0, y1);
-        lds_sync();
-        const int cnt = (y1 - y0) * W;
-        const int pix0 = y0 * W;
-        auto take = [&](int v, int pix) {
-          const long long kv = (static_cast<long long>(max(v, 0)) << kPixBits) |
-                               static_cast<long long>((1 << kPixBits) - 1 - pix);
-          key = kv > key ? kv : key;
-        };
-        if ((W & 3) == 0) {
-          for (int i = tid; i < cnt / 4; i += kAdjThreads) {
-            int4 *pv = reinterpret_cast<int4 *>(s_acc) + i;
-            const int4 u = *pv;
-            *pv = make_int4(0, 0, 0, 0);
-            reinterpret_cast<int4 *>(q + pix0)[i] = u;
-            if (a.normalize) {
-              take(u.x, pix0 + 4 * i);
-              take(u.y, pix0 + 4 * i + 1);
-              take(u.z, pix0 + 4 * i + 2);
-              take(u.w, pix0 + 4 * i + 3);
-            }
-          }
-        } else {
-          for (int i = tid; i < cnt; i += kAdjThreads) {
-            const aacc_t v = s_acc[i];
-            s_acc[i] = 0;
-            q[pix0 + i] = v;
-            if (a.normalize) take(v, pix0 + i);
-          }
-        }
-        lds_sync();
-      }
-      if (a.normalize) {
-        key = wave_max_acc(key);
-        if (lane == 0) sh.wkey[wid] = key;
-        lds_sync();
-        key = 0;
-        for (int w = 0; w < kAdjWaves; ++w) key = sh.wkey[w] > key ? sh.wkey[w] : key;
-      }
-      have_key = true;
-    }
-    if (a.normalize && ns_all > 0 && !have_key && !large) {
-      for (int s = 0; s < a.n_strips; ++s) {
-        const int y0 = s * a.strip_rows;
-        const int y1 = min(H, y0 + a.strip_rows);
-        if (sh.bin_start[kCls * (s + 1)] == sh.bin_start[kCls * s]) continue;
+        if (sh.bin_start[s + 1] == sh.bin_start[s]) continue;
         strip_spots(s, false, y0, y1);
         lds_sync();
         const int cnt = (y1 - y0) * W;
@@ -909,7 +678,7 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
     constexpr int kPre = kAdjPre;
     native_float4 tp[kPre];
     auto prefetch = [&](int s) {
-      if (kLarge || fwd_only || (W & 3) != 0 || s >= a.n_strips) return;
+      if (fwd_only || (W & 3) != 0 || s >= a.n_strips) return;
       const int y0 = s * a.strip_rows;
       const int cnt4 = (min(H, y0 + a.strip_rows) - y0) * W / 4;
       const native_float4 *src = reinterpret_cast<const native_float4 *>(tgt + (size_t)y0 * W);
@@ -919,69 +688,12 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
         if (i < cnt4) tp[k] = __builtin_nontemporal_load(src + i);
       }
     };
-    if (large) {
-      __syncthreads();  // q complete (each thread reads back what it wrote)
-      for (int s = 0; s < a.n_strips; ++s) {
-        const int y0 = s * a.strip_rows;
-        const int y1 = min(H, y0 + a.strip_rows);
-        const int cnt = (y1 - y0) * W;
-        const bool any = sh.bin_start[kCls * (s + 1)] > sh.bin_start[kCls * s];
-        const size_t off = (size_t)y0 * W;
-        // one pixel: pattern, loss and G / m (q may be the pattern buffer: it
-        // is read before the same thread overwrites it)
-        auto pixel = [&](float P, float tv, float &g) {
-          if (l2) {
-            const float d = P - tv;
-            lsum += static_cast<double>(d * d);
-            g = 2.0f * d;
-          } else {
-            g = tv;
-          }
-          csum += static_cast<double>(g * P);
-        };
-        if ((W & 3) == 0) {
-          for (int i = tid; i < cnt / 4; i += kAdjThreads) {
-            const int4 u = any ? reinterpret_cast<const int4 *>(q + off)[i] : make_int4(0, 0, 0, 0);
-            const float4 P = make_float4(static_cast<float>(u.x) * out_scale, static_cast<float>(u.y) * out_scale,
-                                         static_cast<float>(u.z) * out_scale, static_cast<float>(u.w) * out_scale);
-            if (pat) store_nt(P, reinterpret_cast<float4 *>(pat + off) + i);
-            if (fwd_only) continue;
-            const native_float4 tv =
-                __builtin_nontemporal_load(reinterpret_cast<const native_float4 *>(tgt + off) + i);
-            float4 g;
-            pixel(P.x, tv.x, g.x);
-            pixel(P.y, tv.y, g.y);
-            pixel(P.z, tv.z, g.z);
-            pixel(P.w, tv.w, g.w);
-            reinterpret_cast<float4 *>(s_G)[i] =
-                make_float4(g.x * gscale, g.y * gscale, g.z * gscale, g.w * gscale);
-          }
-        } else {
-          for (int i = tid; i < cnt; i += kAdjThreads) {
-            const float P = static_cast<float>(any ? q[off + i] : 0) * out_scale;
-            if (pat) __builtin_nontemporal_store(P, pat + off + i);
-            if (fwd_only) continue;
-            float g;
-            pixel(P, tgt[off + i], g);
-            s_G[i] = g * gscale;
-          }
-        }
-        if (fwd_only) continue;
-        lds_sync();
-        if (a.want_grad && any) strip_spots(s, true, y0, y1);
-        lds_sync();
-      }
-      // G leaves the shared strip buffer; the next pattern's tile bounds and
-      // splat start from zero (ordered by the barrier that ends the pattern)
-      if (!fwd_only)
-        for (int i = tid; i < a.acc_words; i += kAdjThreads) s_acc[i] = 0;
-    }
     prefetch(0);
-    for (int s = 0; s < a.n_strips && !large; ++s) {
+    for (int s = 0; s < a.n_strips; ++s) {
       const int y0 = s * a.strip_rows;
       const int y1 = min(H, y0 + a.strip_rows);
       const int cnt = (y1 - y0) * W;
-      const bool any = sh.bin_start[kCls * (s + 1)] > sh.bin_start[kCls * s];
+      const bool any = sh.bin_start[s + 1] > sh.bin_start[s];
       if (any) {
         strip_spots(s, false, y0, y1);
         lds_sync();
@@ -1010,12 +722,9 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
               make_float4(g.x * gscale, g.y * gscale, g.z * gscale, g.w * gscale);
         };
         const int n4 = cnt / 4;
-        if (kLarge || fwd_only) {
+        if (fwd_only) {
           const native_float4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-          for (int i = tid; i < n4; i += kAdjThreads)
-            readout4(i, fwd_only ? zero
-                                 : __builtin_nontemporal_load(
-                                       reinterpret_cast<const native_float4 *>(tgt + off) + i));
+          for (int i = tid; i < n4; i += kAdjThreads) readout4(i, zero);
         } else {
 #pragma unroll
           for (int k = 0; k < kPre; ++k) {
@@ -1065,77 +774,39 @@ __device__ __forceinline__ void adjoint_body(const AdjArgs &a, aacc_t *s_acc,
       // ---- 5. per spot: the normalisation's max term, then the chain rule ----
       const float corr = norm ? static_cast<float>(ctot) * gscale : 0.0f;
       const int px = pstar % W, py = pstar / W;
-      if (!kLarge) {
-        // sums with the max term to gsum; spot_chain_kernel does the rest
-        float4 *gs = a.gsum + (size_t)p * a.slots;
-        for (int q = tid; q < ns; q += kAdjThreads) {
-          float A = t.A[q], BX = t.BX[q], BY = t.BY[q];
-          if (norm)
-            max_term(a, corr, px, py, t.X[q], t.Y[q], t.xb[q] >> 16, t.xb[q] & 0xffff, t.ylo[q],
-                     t.yhi[q], A, BX, BY);
-          gs[q] = make_float4(A, BX, BY, __int_as_float(t.jpos[q]));
-        }
-        if (tid == 0) a.gcount[p] = ns;
-      } else {
-        // the max term of each spot whose box holds p*, into its gsum entry;
-        // spot_chain_kernel applies the chain rule to the whole row
-        if (norm) {
-          for (int j = tid; j < n; j += kAdjThreads) {
-            const int2 bx = wbox[j];
-            const int lo = bx.y >> 16, hi = bx.y & 0xffff, xlo = bx.x >> 16, xhi = bx.x & 0xffff;
-            if (py < lo || py > hi || px < xlo || px > xhi) continue;
-            const float4 sp = spots[j];
-            float X, Y;
-            to_pixel(sp, a, X, Y);
-            float A = 0.0f, BX = 0.0f, BY = 0.0f;
-            max_term(a, corr, px, py, X, Y, xlo, xhi, lo, hi, A, BX, BY);
-            float *g = reinterpret_cast<float *>(gsp + wrow[j]);
-            unsafeAtomicAdd(g, A);
-            unsafeAtomicAdd(g + 1, BX);
-            unsafeAtomicAdd(g + 2, BY);
-          }
-        }
-        if (tid == 0) a.gcount[p] = ns_all;
+      // sums with the max term to gsum; spot_chain_kernel does the rest
+      float4 *gs = a.gsum + (size_t)p * a.slots;
+      for (int q = tid; q < ns; q += kAdjThreads) {
+        float A = t.A[q], BX = t.BX[q], BY = t.BY[q];
+        if (norm)
+          max_term(a, corr, px, py, t.X[q], t.Y[q], t.xb[q] >> 16, t.xb[q] & 0xffff, t.ylo[q],
+                   t.yhi[q], A, BX, BY);
+        gs[q] = make_float4(A, BX, BY, __int_as_float(t.jpos[q]));
       }
+      if (tid == 0) a.gcount[p] = ns;
     }
     if (tid == 0 && a.loss) a.loss[p] = static_cast<float>(ltot);
-    if (kLarge)
-      __syncthreads();  // LDS and workspace state of this pattern is dead before the next one
-    else
-      lds_sync();  // LDS state of this pattern is dead before the next one
+    lds_sync();  // LDS state of this pattern is dead before the next one
   }
 }
 
 // Two blocks per CU: at most 128 VGPRs (four waves per SIMD).
 __global__ __launch_bounds__(kAdjThreads, 4) void render_adjoint_kernel(AdjArgs a) {
   extern __shared__ __align__(16) aacc_t s_acc[];  // 16-byte aligned for the 16-byte read-out
-  __shared__ AdjShared<1> sh;
-  adjoint_body<false>(a, s_acc, sh);
+  __shared__ AdjShared sh;
+  adjoint_body(a, s_acc, sh);
 }
 
-// Two blocks per CU, each with half the LDS (at most 128 VGPRs).
-__global__ __launch_bounds__(kAdjThreads, 4) void render_adjoint_large_kernel(AdjArgs a) {
-  extern __shared__ __align__(16) aacc_t s_acc[];
-  __shared__ AdjShared<kWidthClasses> sh;
-  adjoint_body<true>(a, s_acc, sh);
+__global__ __launch_bounds__(kTileThreads, 4) void render_tiles_kernel(AdjArgs a) {
+  extern __shared__ int s_tiles[];
+  __shared__ TileShared sh;
+  tiles_body<false>(a, s_tiles, sh);
 }
 
-// Forward mode of the large-pattern kernel (the sub-pixel renderer of long
-// spot lists): with the mode and the missing gradient outputs known at
-// compile time the gather and the FP64 chain rule drop out, and the kernel
-// needs about 100 VGPRs.
-__global__ __launch_bounds__(kAdjThreads, 4) void render_adjoint_large_fwd_kernel(AdjArgs a) {
-  extern __shared__ __align__(16) aacc_t s_acc[];
-  __shared__ AdjShared<kWidthClasses> sh;
-  a.mode = DSX_ADJ_FORWARD;
-  a.want_grad = 0;
-  a.target = nullptr;
-  a.dRt = nullptr;
-  a.dF2 = nullptr;
-  a.drec = nullptr;
-  a.loss = nullptr;
-  a.gsum = nullptr;
-  adjoint_body<true>(a, s_acc, sh);
+__global__ __launch_bounds__(kTileThreads, 4) void render_tiles_fwd_kernel(AdjArgs a) {
+  extern __shared__ int s_tiles[];
+  __shared__ TileShared sh;
+  tiles_body<true>(a, s_tiles, sh);
 }
 
 // Chain rule of every spot gathered by the render adjoint: one block per
@@ -1381,9 +1052,9 @@ __global__ __launch_bounds__(kSfaThreads) void structure_factor_adjoint_kernel(S
 
 using namespace dsx;
 
-// Workspace of the large-pattern kernel, per block (E = kWorkEntriesPerSpot *
-// cap bin entries): int bins[E] | int2 boxes[cap] | int rows[cap] | int
-// q[H W], each part padded to 16 bytes; with gradients the chain-rule hand-over follows the
+// Workspace of the long lists' kernel, per block: large_block_ints(cap, H W)
+// ints, filled with the entries' records and rows and the first row of every
+// 64 listed spots (dsx_tiles.h); with gradients the chain-rule hand-over follows the
 // blocks.  Chain-rule hand-over (the small-pattern kernel's whole workspace):
 // float4 gsum[n * cap] | int gcount[n] | (8-byte aligned) double
 // dpart[chain blocks][9].
@@ -1399,8 +1070,8 @@ static long long large_block_ints(int cap, long long hw) {
   const long long e = kWorkEntriesPerSpot * static_cast<long long>(cap);
   return ((e + 3) & ~3ll) + ((2ll * cap + 3) & ~3ll) + ((cap + 3ll) & ~3ll) + ((hw + 3) & ~3ll);
 }
-// blocks of the large-pattern kernels: two per CU
-static int large_blocks(int n, int per_cu = 2) { return std::min(n, per_cu * cu_count()); }
+// blocks of the long lists' kernel: two per CU
+static int large_blocks(int n) { return std::min(n, 2 * cu_count()); }
 
 extern "C" long long dsx_render_adjoint_workspace_ints(int cap, int n, int height, int width,
                                                        int gradients) {
@@ -1432,6 +1103,74 @@ static int adjoint_static_lds(const void *kernel, int *cache, int *raised) {
     *raised = 1;
   }
   return *cache;
+}
+
+// Chain rule of the gathered sums (rows of `slots` entries).
+static int launch_chain(const AdjArgs &a, hipStream_t s) {
+  const int cblocks = std::min(a.n, chain_blocks_max());
+  hipLaunchKernelGGL(spot_chain_kernel, dim3(cblocks), dim3(kChainThreads), 0, s, a);
+  if (a.drec)
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(9 * kWave), 0, s, a.dpart, cblocks, a.drec);
+  return check_launch("dsx_render_adjoint (chain)");
+}
+
+// Long lists: two blocks per CU (one when the tiles' LDS needs it), each with
+// its part of the workspace.
+static int launch_tiles(AdjArgs &a, int *work_d, long long work_ints, hipStream_t s) {
+  const bool fwd = a.mode == DSX_ADJ_FORWARD;
+  const long long n_tiles = static_cast<long long>((a.W + kTileEdge - 1) / kTileEdge) *
+                            ((a.H + kTileEdge - 1) / kTileEdge);
+  // counters of as many waves as leave room for two blocks per CU
+  a.count_waves = 8;
+  while (a.count_waves > 1 && 4 * (a.count_waves + 1) * n_tiles > 64 * 1024) a.count_waves /= 2;
+  const long long lds = (4 * (a.count_waves + 1) * n_tiles + 15) & ~15ll;
+  static int static_grad = -1, static_fwd = -1, raised_grad = 0, raised_fwd = 0;
+  const int st = fwd ? adjoint_static_lds(reinterpret_cast<const void *>(&render_tiles_fwd_kernel),
+                                          &static_fwd, &raised_fwd)
+                     : adjoint_static_lds(reinterpret_cast<const void *>(&render_tiles_kernel),
+                                          &static_grad, &raised_grad);
+  if (st < 0) {
+    set_error("dsx_render_adjoint: cannot query or reserve the kernel's LDS");
+    return DSX_ELAUNCH;
+  }
+  if (st + lds > kAdjLdsBytes) {
+    set_error("dsx_render_adjoint: %lld tiles of a %dx%d pattern exceed the LDS", n_tiles, a.H, a.W);
+    return DSX_EINVAL;
+  }
+  // the widths and heights of the strip kernel that these patterns had before
+  const int strip_rows = std::min(a.H, (a.W <= 8192 ? 8192 : 16384) / a.W);
+  if (strip_rows < 1 || (a.H + strip_rows - 1) / strip_rows > kAdjMaxStrips) {
+    set_error("dsx_render_adjoint: a %dx%d pattern exceeds the sides taken", a.H, a.W);
+    return DSX_EINVAL;
+  }
+  const int blocks = large_blocks(a.n);
+  const long long per_block = large_block_ints(a.cap, static_cast<long long>(a.H) * a.W);
+  const long long need = per_block * blocks + (a.want_grad ? small_work_ints(a.cap, a.n) : 0);
+  if (work_d ? work_ints < need || reinterpret_cast<uintptr_t>(work_d) % 16 != 0 : a.want_grad != 0) {
+    set_error("dsx_render_adjoint: workspace of %lld ints is smaller than %lld or not 16-byte "
+              "aligned (dsx_render_adjoint_workspace_ints)", work_d ? work_ints : 0ll, need);
+    return DSX_EINVAL;
+  }
+  a.work = work_d;
+  a.work_per_block = per_block;
+  // records and rows fill a block's part after the first rows per 64 listed spots
+  const long long entries = (per_block - (a.cap + kWave - 1) / kWave) / kRecInts;
+  a.work_entries = static_cast<int>(std::min<long long>(entries, 1ll << 28));
+  if (a.want_grad) {
+    int *hand = work_d + per_block * blocks;  // a multiple of 4 ints: 16-byte aligned
+    a.gsum = reinterpret_cast<float4 *>(hand);
+    a.gcount = hand + static_cast<size_t>(a.n) * 4 * a.cap;
+    const size_t off = (static_cast<size_t>(a.n) * (4ull * a.cap + 1) + 1) & ~static_cast<size_t>(1);
+    a.dpart = reinterpret_cast<double *>(hand + off);
+  }
+  if (fwd)
+    hipLaunchKernelGGL(render_tiles_fwd_kernel, dim3(blocks), dim3(kTileThreads), static_cast<size_t>(lds), s, a);
+  else
+    hipLaunchKernelGGL(render_tiles_kernel, dim3(blocks), dim3(kTileThreads), static_cast<size_t>(lds), s, a);
+  const int rc = check_launch("dsx_render_adjoint");
+  if (rc != DSX_OK || !a.want_grad) return rc;
+  a.slots = a.cap;
+  return launch_chain(a, s);
 }
 
 extern "C" int dsx_render_adjoint(const int *idx_d, const float *spot_d, const int *count_d, int cap,
@@ -1505,6 +1244,12 @@ extern "C" int dsx_render_adjoint(const int *idx_d, const float *spot_d, const i
   a.inv_s2 = static_cast<float>(1.0 / (sg * sg));
   a.e2ep = static_cast<float>(exp(-1.0 / (sg * sg)));
   a.clip = rp->clip_threshold;
+  a.log2_clip = static_cast<float>(log2(static_cast<double>(rp->clip_threshold)));
+  a.two_s2_ln2 = static_cast<float>(2.0 * sg * sg * M_LN2);
+  a.tiny_box = static_cast<float>(0.04 * sg * sg);
+  a.box_margin = static_cast<float>(2e-4 * std::max(1.0, sg) + 1e-6 * std::max(rp->height, rp->width));
+  // every spot of the list on one tile stays below 2^31 units
+  a.bound_units = static_cast<float>((1 << 30) / std::max(cap, 1024));
   a.mode = mode;
   a.want_grad = want_grad ? 1 : 0;
   a.target = target_d;
@@ -1522,59 +1267,30 @@ extern "C" int dsx_render_adjoint(const int *idx_d, const float *spot_d, const i
   a.gsum = nullptr;
   a.gcount = nullptr;
 
+  if (adjoint_large(cap)) return launch_tiles(a, work_d, work_ints, as_stream(stream));
+
   // LDS per block: the static part, the spot table (slots entries; bins) and
-  // two strip buffers of rows x W words.  Patterns up to kAdjMaxSpots spots
-  // use two blocks per CU when their strips hold at least 8 rows (or the whole
-  // pattern); larger lists use the large-pattern kernel, one block per CU.
-  const bool large = adjoint_large(cap);
-  static int static_small = -1, static_large = -1, static_fwd = -1;
-  static int raised_small = 0, raised_large = 0, raised_fwd = 0;
-  const bool fwd_large = large && mode == DSX_ADJ_FORWARD;
-  const void *kern = fwd_large ? reinterpret_cast<const void *>(&render_adjoint_large_fwd_kernel)
-                     : large   ? reinterpret_cast<const void *>(&render_adjoint_large_kernel)
-                               : reinterpret_cast<const void *>(&render_adjoint_kernel);
-  const int st = fwd_large ? adjoint_static_lds(kern, &static_fwd, &raised_fwd)
-                 : large   ? adjoint_static_lds(kern, &static_large, &raised_large)
-                           : adjoint_static_lds(kern, &static_small, &raised_small);
+  // two strip buffers of rows x W words; two blocks per CU when their strips
+  // hold at least 8 rows (or the whole pattern).
+  static int static_small = -1, raised_small = 0;
+  const int st = adjoint_static_lds(reinterpret_cast<const void *>(&render_adjoint_kernel), &static_small,
+                                    &raised_small);
   if (st < 0) {
     set_error("dsx_render_adjoint: cannot query or reserve the kernel's LDS");
     return DSX_ELAUNCH;
   }
-  int bpc = 2;  // large kernels: two blocks per CU, one block's barrier waits overlap the other's work
-  int rows = 0;
-  long long table = 0;
-  if (large) {
-    // one strip buffer of up to 64 KB (32 KB with two blocks per CU), at least
-    // 512 spot slots, the rest slots; one block per CU when a row of the
-    // pattern does not fit half the budget
-    a.bin_cap = 0;
-    auto size_large = [&](int b) {
-      const long long per_block = kAdjLdsBytes / b;
-      const long long strip = std::min<long long>(kAdjStripBytes / b,
-                                                  per_block - st - 16 - 512ll * kSpotTabBytes);
-      rows = strip < 4ll * a.W ? 0 : static_cast<int>(std::min<long long>(a.H, strip / (4ll * a.W)));
-      a.slots = static_cast<int>(std::min<long long>(
-          kAdjLargeMaxSlots, (per_block - st - 16 - 4ll * rows * a.W) / kSpotTabBytes));
-      table = static_cast<long long>(kSpotTabBytes) * a.slots + 16;
-    };
-    size_large(bpc);
-    if (rows < 1) {
-      bpc = 1;
-      size_large(bpc);
-    }
-  } else {
-    a.slots = cap;
-    a.bin_cap = std::min(kAdjBinCap, 4 * cap + 256);
-    table = static_cast<long long>(kSpotTabBytes) * a.slots + 2ll * a.bin_cap + 16;
-    auto rows_for = [&](int per_block) {
-      const long long strip = std::min<long long>(kAdjSmallStripBytes, per_block - st - table);
-      return strip < 8ll * a.W ? 0 : static_cast<int>(std::min<long long>(a.H, strip / (8ll * a.W)));
-    };
-    rows = rows_for(kAdjLdsBytes / bpc);
-    if (rows < std::min(a.H, 8)) {
-      bpc = 1;
-      rows = rows_for(kAdjLdsBytes);
-    }
+  int bpc = 2;
+  a.slots = cap;
+  a.bin_cap = std::min(kAdjBinCap, 4 * cap + 256);
+  const long long table = static_cast<long long>(kSpotTabBytes) * a.slots + 2ll * a.bin_cap + 16;
+  auto rows_for = [&](int per_block) {
+    const long long strip = std::min<long long>(kAdjSmallStripBytes, per_block - st - table);
+    return strip < 8ll * a.W ? 0 : static_cast<int>(std::min<long long>(a.H, strip / (8ll * a.W)));
+  };
+  int rows = rows_for(kAdjLdsBytes / bpc);
+  if (rows < std::min(a.H, 8)) {
+    bpc = 1;
+    rows = rows_for(kAdjLdsBytes);
   }
   if (rows < 1) {
     set_error("dsx_render_adjoint: pattern width %d exceeds the LDS strip budget", a.W);
@@ -1589,37 +1305,8 @@ extern "C" int dsx_render_adjoint(const int *idx_d, const float *spot_d, const i
   a.strip_rows = rows;
   a.n_strips = n_strips;
   a.acc_words = rows * a.W;
-  const int blocks = large ? large_blocks(n, bpc) : std::min(n, cu_count() * bpc);
-  if (large) {
-    const long long per_block = large_block_ints(cap, static_cast<long long>(a.H) * a.W);
-    const long long need = per_block * blocks + (want_grad ? small_work_ints(cap, n) : 0);
-    if (work_d && reinterpret_cast<uintptr_t>(work_d) % 16 != 0) {
-      set_error("dsx_render_adjoint: workspace must be 16-byte aligned");
-      return DSX_EINVAL;
-    }
-    if (want_grad && !work_d) {
-      set_error("dsx_render_adjoint: gradients need a workspace of %lld ints "
-                "(dsx_render_adjoint_workspace_ints)", need);
-      return DSX_EINVAL;
-    }
-    if (work_d && work_ints >= need &&
-        kWorkEntriesPerSpot * static_cast<long long>(cap) < (1ll << 31)) {
-      a.work = work_d;
-      a.work_per_block = per_block;
-      a.work_entries = kWorkEntriesPerSpot * cap;
-      if (want_grad) {
-        int *hand = work_d + per_block * blocks;  // a multiple of 4 ints: 16-byte aligned
-        a.gsum = reinterpret_cast<float4 *>(hand);
-        a.gcount = hand + static_cast<size_t>(n) * 4 * cap;
-        const size_t off = (static_cast<size_t>(n) * (4ull * cap + 1) + 1) & ~static_cast<size_t>(1);
-        a.dpart = reinterpret_cast<double *>(hand + off);
-      }
-    } else if (work_d) {
-      set_error("dsx_render_adjoint: workspace of %lld ints is smaller than %lld "
-                "(dsx_render_adjoint_workspace_ints)", work_ints, need);
-      return DSX_EINVAL;
-    }
-  } else if (want_grad) {
+  const int blocks = std::min(n, cu_count() * bpc);
+  if (want_grad) {
     const long long need = small_work_ints(cap, n);
     if (!work_d || work_ints < need) {
       set_error("dsx_render_adjoint: gradients need a workspace of %lld ints, got %lld "
@@ -1635,27 +1322,12 @@ extern "C" int dsx_render_adjoint(const int *idx_d, const float *spot_d, const i
     const size_t off = (static_cast<size_t>(n) * (4ull * cap + 1) + 1) & ~static_cast<size_t>(1);
     a.dpart = reinterpret_cast<double *>(work_d + off);
   }
-  const size_t lds = (((large ? 1ull : 2ull) * a.acc_words * 4 + static_cast<size_t>(table)) + 15) &
-                     ~static_cast<size_t>(15);
+  const size_t lds = (2ull * a.acc_words * 4 + static_cast<size_t>(table) + 15) & ~static_cast<size_t>(15);
   hipStream_t s = as_stream(stream);
-  if (large) {
-    if (fwd_large)
-      hipLaunchKernelGGL(render_adjoint_large_fwd_kernel, dim3(blocks), dim3(kAdjThreads), lds, s, a);
-    else
-      hipLaunchKernelGGL(render_adjoint_large_kernel, dim3(blocks), dim3(kAdjThreads), lds, s, a);
-  } else {
-    hipLaunchKernelGGL(render_adjoint_kernel, dim3(blocks), dim3(kAdjThreads), lds, s, a);
-  }
-  int rc = check_launch("dsx_render_adjoint");
+  hipLaunchKernelGGL(render_adjoint_kernel, dim3(blocks), dim3(kAdjThreads), lds, s, a);
+  const int rc = check_launch("dsx_render_adjoint");
   if (rc != DSX_OK || !want_grad) return rc;
-  // the chain kernel reads gsum rows of `slots` entries: the large kernel's
-  // rows are indexed by spot position (cap entries)
-  if (large) a.slots = cap;
-  const int cblocks = std::min(n, chain_blocks_max());
-  hipLaunchKernelGGL(spot_chain_kernel, dim3(cblocks), dim3(kChainThreads), 0, s, a);
-  if (drec_d)
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(9 * kWave), 0, s, a.dpart, cblocks, drec_d);
-  return check_launch("dsx_render_adjoint (chain)");
+  return launch_chain(a, s);
 }
 
 // ---------------------------------------------------------------------------

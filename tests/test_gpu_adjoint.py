@@ -468,3 +468,91 @@ def test_stage_atoms_matches_host_fixed_point():
     assert np.array_equal(got[:, :3], want)
     assert np.all(got[:, 3] == 0)
     assert np.array_equal(Bs.cpu().numpy(), B[order].astype(np.float32))
+
+
+# -- long lists (matrix-core tiles) against the small-list kernels -----------------
+
+
+def _copy_lists(b, cap):
+    """The same spot lists with another capacity."""
+    import torch
+    from diffsims_amd import engine
+    assert int(b.ncand.max()) <= b.cap
+    out = engine.empty_batch(b.table, b.n, cap, b.idx.device)
+    m = min(cap, b.cap)
+    out.idx[:, :m], out.spots[:, :m] = b.idx[:, :m], b.spots[:, :m]
+    for k in ("count", "ncand", "maxI"):
+        setattr(out, k, getattr(b, k).clone())
+    return out
+
+
+@pytest.mark.parametrize("shape,sigma,clip,kw", [
+    ((256, 256), 1.0, 1.0, {}),
+    ((97, 131), 1.6, 1.0, {}),                    # partial tiles, odd rows
+    ((64, 80), 6.0, 1e-3, {}),                    # boxes over many tiles: several ranges
+    ((33, 400), 1.0, 1.0, {"in_plane_angle": 20.0, "mirrored": True}),
+    ((128, 128), 0.6, 1.0, {"normalize": False}),
+    ((16, 16), 1.0, 1.0, {}),                     # one tile
+    ((1200, 1100), 1.0, 1.0, {}),                 # more tiles than eight waves' counters hold
+])
+def test_long_list_kernel_equals_small_list_kernel(shape, sigma, clip, kw):
+    """One set of spot lists through both kernels (a capacity above 1,024
+    selects the tiles): patterns, loss and every gradient.  Each side rounds a
+    pixel's terms within ~1e-6 of the maximum; a gathered sum runs over at most
+    some 2,000 pixels with both signs, so the gradients agree to 1e-4 of the
+    largest component."""
+    import torch
+    from diffsims_amd import _lib, engine
+    from diffsims_amd import differentiable as D
+    from tests import parity as P
+
+    print(f"tiles: {shape}, sigma {sigma}, clip {clip}, {kw}", flush=True)
+    spec = P.triclinic(20, 9, edges=(7, 12))
+    st = engine.SimSettings(max_excitation_error=0.02)
+    cal = 3.2 / min(shape)
+    m = D.RefinementModel(P.to_arrays(spec), 1.6, st, shape, sigma, cal, clip_threshold=clip, **kw)
+    rng = np.random.default_rng(5)
+    leaves = D.leaf_parameters(P.to_arrays(spec), rng.uniform(0, 2 * np.pi, (7, 3)), requires_grad=False)
+    with torch.no_grad():
+        Rt, rec, xyz, B = D.forward_args(leaves)
+        t = m.tables(rec, xyz, B)
+        b = m.spots(t, Rt)
+    small, long_ = _copy_lists(b, 1000), _copy_lists(b, 1100)
+    small.count[5], long_.count[5] = 0, 0          # an empty list
+    H, W = shape
+    gen = torch.Generator("cuda").manual_seed(2)
+    for mode, target in ((_lib.ADJ_L2, torch.rand((7, H, W), generator=gen, device="cuda") * 0.2),
+                         (_lib.ADJ_L2, torch.rand((H, W), generator=gen, device="cuda") * 0.2),
+                         (_lib.ADJ_PATTERN_GRAD, torch.randn((7, H, W), generator=gen, device="cuda"))):
+        got = []
+        for batch in (small, long_):
+            pat = torch.full((7, H, W), float("nan"), device="cuda")
+            got.append((m.adjoint(t, Rt, batch, mode, target, True, pattern=pat), pat))
+        (a, pa), (c, pc) = got
+        top = float(pa.abs().max())
+        assert not torch.isnan(pc).any() and float((pa - pc).abs().max()) <= 2e-6 * top
+        if mode == _lib.ADJ_L2:
+            assert torch.allclose(a[0], c[0], rtol=1e-5)
+        for x, y in zip(a[1:], c[1:]):
+            assert float((x - y).abs().max()) <= 1e-4 * float(x.abs().max()) + 1e-12
+    fwd = engine.render_spots(long_.spots, long_.count, long_.cap, shape, sigma, cal, **m.render_kw)
+    assert torch.equal(fwd, pc)
+
+
+def test_long_lists_without_workspace_report_their_patterns():
+    import ctypes
+    import torch
+    from diffsims_amd import _lib, engine
+    L = _lib.load(require_gpu=True)
+    p = engine.render_params((40, 40), 1.0, 1.0, fast=False)
+    sim = _lib.SimParams()
+    sim.k, sim.shape_width, sim.shape_model = 1.0, 1.0, _lib.SF_LINEAR
+    spots = torch.full((3, 2000, 4), 5.0, device="cuda")
+    cnt = torch.full((3,), 1500, dtype=torch.int32, device="cuda")
+    out = torch.full((3, 40, 40), float("nan"), device="cuda")
+    st = torch.zeros(3, dtype=torch.int32, device="cuda")
+    _lib.check(L.dsx_render_adjoint(None, _lib.ptr(spots), _lib.ptr(cnt), 2000, 3, None, None, 0, None,
+                                    ctypes.byref(sim), ctypes.byref(p), _lib.ADJ_FORWARD, None, 0,
+                                    _lib.ptr(out), None, None, None, None, None, 0, _lib.ptr(st),
+                                    _lib.stream_handle()), "dsx_render_adjoint")
+    assert bool((st == 1).all()) and bool((out == 0).all())
