@@ -341,7 +341,7 @@ __device__ __forceinline__ double atomic_f(const double *c, double g2, int scatt
     for (int t = 0; t < 5; ++t) {
       const double bg = c[2 * t + 1] * g2;
       const double d = 1.0 + bg;
-      f += c[2 * t] * (2.0 + bg) / (d * d);
+      f += c[2 * t] * (2.0 + bg) * frcp(d * d);
     }
   } else {
 #pragma unroll
@@ -363,9 +363,10 @@ __device__ __forceinline__ double atomic_f_grad(const double *c, double g2, int 
       const double b = c[2 * t + 1];
       const double bg = b * g2;
       const double d = 1.0 + bg;
-      const double id2 = 1.0 / (d * d);
+      const double id = frcp(d);
+      const double id2 = id * id;
       f += c[2 * t] * (2.0 + bg) * id2;
-      df -= c[2 * t] * b * (3.0 + bg) * id2 / d;
+      df -= c[2 * t] * b * (3.0 + bg) * (id2 * id);
     }
   } else {
 #pragma unroll

@@ -1,0 +1,199 @@
+// Structure factors of many atoms and their adjoint with one atom per lane.
+//
+// F(h) = sum_a f_a(|g|) occ_a exp(-B_a |g|^2 / 4) e^(2 pi i h.x_a).  The kernels
+// of dsx_tables.hip / dsx_adjoint.hip give every reflection a thread and form
+// each atom's phase anew: an integer phase, a sine and cosine, an exponential
+// (about 85 instructions per reflection and atom, and another 48 cross-lane
+// steps in the adjoint).  Here a lane keeps an atom and a wave walks down
+// consecutive rows of the table: along a line (equal h and k, l falling by
+// one) the phase turns by -2 pi z_a, two FP64 products and two fmas, and only
+// a row that starts a line (the same for all lanes) forms it anew.  The sums
+// over atoms collect in registers, one set per row of a short run of rows, and
+// are folded over the lanes once per run; the adjoint's sums over reflections
+// stay with the atom's lane.
+#pragma once
+
+#include "dsx_internal.h"
+#include "dsx_physics.h"
+
+namespace dsx {
+
+constexpr int kAtomThreads = 256;
+constexpr int kAtomWaves = kAtomThreads / kWave;
+constexpr int kAtomRows = 16;     // rows a wave stages at a time
+constexpr int kAtomMax = 512;     // atoms that fit the block's LDS
+constexpr int kAtomElems = 20;    // elements whose factors of the staged rows fit it
+
+// Sum over the lanes of each of n values, v[i] -> lanes i mod n.  Every step
+// halves the values: a lane keeps those with its bit of the index and hands
+// the others to its partner.
+template <int w>
+__device__ __forceinline__ void fold_step(double *v, int lane) {
+  const bool high = (lane & w) != 0;
+#pragma unroll
+  for (int i = 0; i < w; ++i) {
+    const double keep = high ? v[i + w] : v[i];
+    const double give = high ? v[i] : v[i + w];
+    v[i] = keep + __shfl_xor(give, w, kWave);
+  }
+}
+
+// (a loop over the widths is not unrolled and would index v at run time)
+template <int n>
+__device__ __forceinline__ double fold(double (&v)[n], int lane) {
+  static_assert(n == 16 || n == 32, "values");
+  if (n == 32) fold_step<(n == 32 ? 16 : 8)>(v, lane);
+  fold_step<8>(v, lane);
+  fold_step<4>(v, lane);
+  fold_step<2>(v, lane);
+  fold_step<1>(v, lane);
+  double s = v[0];
+  if (n == 16) s += __shfl_xor(s, 16, kWave);
+  return s + __shfl_xor(s, 32, kWave);
+}
+
+struct AtomLane {
+  uint4 x;        // fixed-point fractional position
+  float B, occ;   // occ = 0 past the last atom
+  int el;
+  double ct, st;  // one row down a line: cos(2 pi z), -sin(2 pi z)
+  double c, s;    // the current row's phase
+};
+
+// The block's atoms in LDS, 44 B each, with e^(-2 pi i z).
+struct AtomTable {
+  double2 *turn;
+  uint4 *x;
+  float2 *Bo;  // B, occ
+  int *el;
+};
+
+__host__ __device__ __forceinline__ int atom_table_doubles(int n) { return (44 * n + 15) / 16 * 2; }
+
+__device__ __forceinline__ AtomTable atom_table(double *s, int n) {
+  AtomTable t;
+  t.turn = reinterpret_cast<double2 *>(s);
+  t.x = reinterpret_cast<uint4 *>(t.turn + n);
+  t.Bo = reinterpret_cast<float2 *>(t.x + n);
+  t.el = reinterpret_cast<int *>(t.Bo + n);
+  return t;
+}
+
+template <class Args>
+__device__ __forceinline__ void stage_atoms(const Args &a, const AtomTable &t) {
+  for (int i = threadIdx.x; i < a.n_atoms; i += kAtomThreads) {
+    const uint4 x = a.xyz_fx[i];
+    double sn, cs;
+    sincospi(static_cast<double>(static_cast<int32_t>(x.z)) * (2.0 / 4294967296.0), &sn, &cs);
+    t.turn[i] = make_double2(cs, -sn);
+    t.x[i] = x;
+    t.Bo[i] = make_float2(a.B[i], a.occ[i]);
+    t.el[i] = min(max(a.elem[i], 0), a.n_elem - 1);
+  }
+}
+
+__device__ __forceinline__ AtomLane load_atom(const AtomTable &tab, int atom, int n) {
+  AtomLane t;
+  const int i = atom < n ? atom : 0;
+  t.x = tab.x[i];
+  const float2 bo = tab.Bo[i];
+  t.B = bo.x;
+  t.occ = atom < n ? bo.y : 0.0f;
+  t.el = tab.el[i];
+  const double2 turn = tab.turn[i];
+  t.ct = turn.x;
+  t.st = turn.y;
+  t.c = t.s = 0.0;
+  return t;
+}
+
+// cos and sin of u / 2^32 turns in FP64: the nearest quarter turn is taken off
+// in integers, the rest (at most an eighth) goes through the Taylor series to
+// 2e-18 (cos) and 5e-17 (sin); multiples of a quarter are exact.
+__device__ __forceinline__ void turn_sincos(uint32_t u, double &c, double &s) {
+  const uint32_t q = (u + (1u << 29)) >> 30;
+  const double x = static_cast<double>(static_cast<int32_t>(u - (q << 30))) * (2.0 * M_PI / 4294967296.0);
+  const double y = x * x;
+  constexpr double f2 = 2, f4 = 24, f6 = 720, f8 = 40320, f10 = 3628800, f12 = 479001600,
+                   f14 = 87178291200.0, f16 = 20922789888000.0;
+  const double cs = fma(y, fma(y, fma(y, fma(y, fma(y, fma(y, fma(y, fma(y, 1 / f16, -1 / f14), 1 / f12),
+                    -1 / f10), 1 / f8), -1 / f6), 1 / f4), -1 / f2), 1.0);
+  const double sn = x * fma(y, fma(y, fma(y, fma(y, fma(y, fma(y, fma(y, -1 / (f14 * 15), 1 / (f12 * 13)),
+                    -1 / (f10 * 11)), 1 / (f8 * 9)), -1 / (f6 * 7)), 1 / (f4 * 5)), -1 / (f2 * 3)), 1.0);
+  const double p = (q & 1) ? sn : cs, r = (q & 1) ? cs : sn;
+  c = ((q + 1) & 2) ? -p : p;
+  s = (q & 2) ? -r : r;
+}
+
+// Phase of the row h: turned on from the row before it in its line, or anew.
+// The tables form it in FP64 (kExact): where atoms cancel, the turned phases and
+// the newly formed ones have to agree to rounding, or extinct reflections come
+// out at 1e-16 of the strongest |F|^2 (FP32 phases, atoms at eighths of the
+// cell) instead of 1e-32 and pass the relative cut.  The adjoint sees only
+// reflections that passed and takes sincospif.
+template <bool kExact>
+__device__ __forceinline__ void row_phase(AtomLane &t, bool anew, const int4 &h) {
+  if (anew) {  // uniform
+    const uint32_t u = static_cast<uint32_t>(h.x) * t.x.x + static_cast<uint32_t>(h.y) * t.x.y +
+                       static_cast<uint32_t>(h.z) * t.x.z;
+    if (kExact) {
+      turn_sincos(u, t.c, t.s);
+    } else {
+      float sn, cs;
+      sincospif(2.0f * (static_cast<float>(static_cast<int32_t>(u)) * 2.3283064365386963e-10f), &sn, &cs);
+      t.c = cs;
+      t.s = sn;
+    }
+  } else {
+    const double c = fma(t.c, t.ct, -(t.s * t.st));
+    t.s = fma(t.s, t.ct, t.c * t.st);
+    t.c = c;
+  }
+}
+
+__device__ __forceinline__ bool line_goes_on(const int4 &before, const int4 &h) {
+  return before.x == h.x && before.y == h.y && before.z == h.z + 1;
+}
+
+__device__ __forceinline__ void atom_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// Rows per block: enough to pay for the staged turns, few enough to fill the chip.
+static inline int atom_rows_per_block(int n, int most) {
+  const int unit = kAtomRows * kAtomWaves;
+  int rows = (n / 1024 + unit - 1) / unit * unit;
+  return rows < unit ? unit : (rows > most ? most : rows);
+}
+
+// Which tables take these kernels.  They cost the same from 1 to 64 atoms, a
+// thread per reflection costs in proportion to the atoms but needs many rows to
+// fill the chip.  Measured in us, thread per reflection | atom per lane:
+//   rows        24 atoms    32         48         64         100          500
+//   1,563,972   115 | 230   145 | 230  182 | 230  229 | 228  -            1225 | 930   forward
+//               568 | 549   568 | 538  592 | 557  727 | 560  -            4393 | 2560  adjoint
+//   195,590     21 | 38     26 | 39    32 | 39    39 | 39                              forward
+//               104 | 126   120 | 129  139 | 131  160 | 129                            adjoint
+//   58,076      15 | 17     18 | 17    23 | 17    28 | 18    40 | 23                   forward
+//               58 | 83     67 | 83    85 | 83    104 | 84   151 | 88                  adjoint
+//   17,332      14 | 11     18 | 11    22 | 11    28 | 11                              forward
+//               44 | 36     55 | 37    72 | 37    91 | 37                              adjoint
+//   4,614       14 | 10     17 | 9     21 | 9     27 | 9     38 | 12                   forward
+//               42 | 20     53 | 20    70 | 20    89 | 20    136 | 25                  adjoint
+// (at 17,332 rows of 16 atoms both take 10 forward and 31 adjoint).
+static inline bool atoms_fit(int n_atoms, int n_elem) {
+  return n_atoms <= kAtomMax && n_elem >= 1 && n_elem <= kAtomElems;
+}
+
+static inline bool atoms_per_lane(int n, int n_atoms, int n_elem) {
+  const bool few_rows = n <= 24 * 1024 ? n_atoms >= 24 : (n <= 64 * 1024 && n_atoms >= 32);
+  return atoms_fit(n_atoms, n_elem) && (n_atoms > kWave || few_rows);
+}
+
+static inline bool atoms_per_lane_adjoint(int n, int n_atoms, int n_elem) {
+  return atoms_fit(n_atoms, n_elem) && (n_atoms >= 48 || (n_atoms >= 24 && n <= 24 * 1024));
+}
+
+}  // namespace dsx

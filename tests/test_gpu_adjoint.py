@@ -556,3 +556,138 @@ def test_long_lists_without_workspace_report_their_patterns():
                                     _lib.ptr(out), None, None, None, None, None, 0, _lib.ptr(st),
                                     _lib.stream_handle()), "dsx_render_adjoint")
     assert bool((st == 1).all()) and bool((out == 0).all())
+
+
+# rows, atoms, elements, table: either side of the lines between the kernels with
+# a thread per reflection and a lane per atom (23/24, 47/48, 64/65 and 512/513
+# atoms, 20/21 elements, 24,576 and 65,536 rows), and row counts around a wave's 16
+SF_SIZES = [(1, 24, 3, "lobato"), (15, 23, 3, "lobato"), (17, 48, 20, "xtables"), (64, 64, 1, None),
+            (65, 65, 2, "lobato"), (999, 47, 20, "lobato"), (1000, 100, 21, "xtables"),
+            (1003, 512, 20, "lobato"), (700, 513, 5, "lobato"), (24577, 24, 2, "lobato"),
+            (24576, 30, 2, None), (65537, 33, 1, "lobato"), (65536, 32, 1, "lobato"), (33000, 130, 4, "xtables")]
+
+
+@pytest.mark.parametrize("n,n_atoms,n_elem,table", SF_SIZES)
+def test_structure_factor_and_adjoint_of_any_table(n, n_atoms, n_elem, table):
+    """F, |F|^2 and the gradients of sum w |F|^2 against FP64 on the same
+    fixed-point positions, for tables of whole lines, broken lines and rows in
+    any order.  Per atom the phase and the Debye-Waller factor are FP32: an
+    angle off by 2^-26 turns (9.4e-8) and the errors of sincospif, expf and two
+    products, together below 5e-7 of |t_a|, t_a the atom's term.  With S = sum
+    |t_a|: |dF| <= 5e-7 S, |d|F|^2| <= 1e-6 S |F| + (5e-7 S)^2 + rounding, and each
+    gradient within 2e-6 of its sum of magnitudes (conj(F) t_a is off by 1e-6
+    S |t_a|, and the FP32 sums over the blocks as much again)."""
+    import ctypes
+
+    from diffsims_amd import _lib
+
+    print(f"structure factors {n} rows {n_atoms} atoms {n_elem} elements {table}", flush=True)
+    rng = np.random.default_rng(n + n_atoms)
+    # lines of 1 to 40 rows, then some rows moved
+    hkl, left = [], n
+    while left:
+        m = min(left, int(rng.integers(1, 41)))
+        h, k, l0 = (int(v) for v in rng.integers(-12, 13, 3))
+        hkl += [(h, k, l0 - i, 0) for i in range(m)]
+        left -= m
+    hkl = np.array(hkl, dtype=np.int32)
+    moved = rng.choice(n, n // 8, replace=False)
+    hkl[np.sort(moved)] = hkl[moved]
+    rec = np.array([[0.05, 0.003, 0.001], [0.0, 0.04, -0.002], [0.0, 0.0, 0.03]])
+    fx = rng.integers(0, 2 ** 32, (n_atoms, 4), dtype=np.uint64).astype(np.uint32)
+    fx[:2, :3] = [[0, 0, 0], [2 ** 31, 2 ** 30, 3 * 2 ** 30]][:min(2, n_atoms)]
+    elem = rng.integers(0, n_elem, n_atoms).astype(np.int32)
+    occ = rng.uniform(0.2, 1.0, n_atoms).astype(np.float32)
+    B = rng.uniform(0.0, 2.0, n_atoms).astype(np.float32)
+    co = np.stack([rng.uniform(0.2, 2.0, (n_elem, 5)), rng.uniform(0.5, 8.0, (n_elem, 5))], -1)
+    w = rng.uniform(-1.0, 1.0, n).astype(np.float32)
+    w[rng.random(n) < 0.3] = 0.0
+
+    L = _lib.load()
+    dev = lambda v: torch.from_numpy(np.ascontiguousarray(v)).cuda()
+    d_hkl, d_fx, d_el, d_occ, d_B, d_co, d_w = (dev(v) for v in (
+        hkl, fx.view(np.int32), elem, occ, B, co.reshape(n_elem, 10), w))
+    F, F2 = torch.empty((n, 2), device="cuda"), torch.empty(n, device="cuda")
+    g4 = torch.empty((n, 4), device="cuda")
+    dx, dB = torch.zeros((n_atoms, 3), device="cuda"), torch.zeros(n_atoms, device="cuda")
+    dr = torch.zeros(9, dtype=torch.float64, device="cuda")
+    rec9 = (ctypes.c_double * 9)(*rec.reshape(-1).tolist())
+    sc = {None: _lib.SCATTER_NONE, "lobato": _lib.SCATTER_LOBATO, "xtables": _lib.SCATTER_XTABLES}[table]
+    _lib.check(L.dsx_structure_factor(
+        _lib.ptr(d_hkl), n, rec9, _lib.ptr(d_fx), _lib.ptr(d_el), _lib.ptr(d_occ), _lib.ptr(d_B),
+        n_atoms, _lib.ptr(d_co), n_elem, sc, _lib.ptr(g4), _lib.ptr(F2), _lib.ptr(F),
+        _lib.stream_handle()), "structure factors")
+    _lib.check(L.dsx_structure_factor_adjoint(
+        _lib.ptr(d_hkl), n, rec9, _lib.ptr(d_fx), _lib.ptr(d_el), _lib.ptr(d_occ), _lib.ptr(d_B),
+        n_atoms, _lib.ptr(d_co), n_elem, sc, _lib.ptr(d_w), _lib.ptr(dx), _lib.ptr(dB),
+        _lib.ptr(dr), _lib.stream_handle()), "adjoint")
+    torch.cuda.synchronize()
+
+    H = hkl[:, :3].astype(np.int64)
+    g = H @ rec.T
+    g2 = (g * g).sum(1)
+    grad, mag = np.zeros((n_atoms, 4)), np.zeros((n_atoms, 4))
+    gr, gm = np.zeros((3, 3)), np.zeros((3, 3))
+    got, got2 = F.cpu().numpy().astype(np.float64), F2.cpu().numpy().astype(np.float64)
+    assert np.abs(g4.cpu().numpy() - np.c_[g, g2]).max() <= 1e-7 * max(np.abs(g).max(), g2.max())
+    for r0 in range(0, n, 4096):
+        s = slice(r0, r0 + 4096)
+        q = g2[s, None]
+        f = O.atomic_f(g2[s], co, table)
+        e = 1e-6 * np.maximum(g2[s], 1e-3)[:, None]  # central difference of f in g^2
+        df = (O.atomic_f(g2[s] + e[:, 0], co, table) - O.atomic_f(g2[s] - e[:, 0], co, table)) / (2 * e)
+        turn = (H[s] @ fx[:, :3].astype(np.int64).T) % 2 ** 32
+        od = occ.astype(np.float64) * np.exp(-0.25 * q * B.astype(np.float64))
+        ph = np.exp(2j * np.pi * (turn / 2.0 ** 32))
+        t = f[:, elem] * od * ph
+        tq = (df[:, elem] - 0.25 * B * f[:, elem]) * od * ph
+        F64, S, SQ = t.sum(1), np.abs(t).sum(1), np.abs(tq).sum(1)
+        err = np.abs(got[s, 0] + 1j * got[s, 1] - F64)
+        assert (err <= 5e-7 * S).all(), (err / S).max()
+        err2 = np.abs(got2[s] - np.abs(F64) ** 2)
+        assert (err2 <= 1e-6 * S * np.abs(F64) + (5e-7 * S) ** 2 + 1e-7 * np.abs(F64) ** 2).all()
+        ww = w[s, None].astype(np.float64)
+        c = F64.conj()[:, None] * t
+        m = np.abs(ww) * S[:, None] * np.abs(t)
+        for j in range(3):
+            grad[:, j] += (-4 * np.pi * ww * H[s, j, None] * c.imag).sum(0)
+            mag[:, j] += (4 * np.pi * m * np.abs(H[s, j, None])).sum(0)
+        grad[:, 3] += (-0.5 * ww * q * c.real).sum(0)
+        mag[:, 3] += (0.5 * m * q).sum(0)
+        dq = w[s] * 2.0 * (F64.conj() * tq.sum(1)).real
+        dm = np.abs(w[s]) * 2.0 * S * SQ
+        gr += np.einsum("n,ni,nj->ij", dq, 2 * g[s], H[s])
+        gm += np.einsum("n,ni,nj->ij", dm, np.abs(2 * g[s]), np.abs(H[s]))
+    out = np.c_[dx.cpu().numpy(), dB.cpu().numpy()]
+    assert (np.abs(out - grad) <= 2e-6 * mag + 1e-30).all(), (np.abs(out - grad) / (mag + 1e-30)).max()
+    out = dr.cpu().numpy().reshape(3, 3)
+    assert (np.abs(out - gr) <= 2e-6 * gm + 1e-30).all(), (np.abs(out - gr) / (gm + 1e-30)).max()
+
+
+@pytest.mark.parametrize("atoms_of_cell,reps,radius", [(8, 2, 1.5), (4, 2, 1.5), (8, 2, 2.5), (8, 3, 0.7)])
+def test_extinct_reflections_of_large_cells_stay_extinct(atoms_of_cell, reps, radius):
+    """Supercells of the diamond and face-centred cell: every reflection that is
+    not one of the small cell's, or is extinct in it, has |F|^2 below 1e-20 of the
+    largest, the relative cut's default, where the positions (eighths) are exact
+    in 32-bit fixed point; for the 3 x 3 x 3 cell, whose thirds are off by up to
+    2^-33 turns per index (|h| + |k| + |l| <= 3 x 12), within (2 pi 36 / 2^33)^2 =
+    7e-16 x 64 of it (all the error in one direction, FP32 phases 1.3e-7)."""
+    from diffsims_amd import engine
+    from diffsims_amd.crystallography import PhaseArrays
+
+    si = np.array([(0, 0, 0), (0, 2, 2), (2, 0, 2), (2, 2, 0), (1, 1, 1), (1, 3, 3), (3, 1, 3),
+                   (3, 3, 1)])[:atoms_of_cell] / 4.0
+    xyz = np.concatenate([(si + np.array(t)) / reps for t in np.ndindex(reps, reps, reps)])
+    pa = PhaseArrays((5.43 * reps,) * 3, (90.0,) * 3, ["Si"] * len(xyz), xyz, np.ones(len(xyz)),
+                     np.full(len(xyz), 0.3), "t")
+    tab = engine.build_phase_table(pa, radius, False, "lobato")
+    hkl = tab.hkl_host()[:, :3].astype(np.int64)
+    F2 = tab.F2.cpu().numpy().astype(np.float64)[:len(hkl)]
+    sub = (hkl % reps == 0).all(1)
+    m = hkl // reps
+    allowed = sub & ((m % 2 == m[:, :1] % 2).all(1))
+    if atoms_of_cell == 8:
+        allowed &= (m % 2 == 1).all(1) | (m.sum(1) % 4 == 0)
+    print(f"{len(hkl)} reflections, {allowed.sum()} allowed", flush=True)
+    assert allowed.any() and (F2[allowed] > 0).all()
+    assert F2[~allowed].max() <= (1e-20 if reps == 2 else 7e-14) * F2.max()
