@@ -280,7 +280,7 @@ __device__ __forceinline__ double shape_factor_grad(double s, double r, const Ar
     }
     case DSX_SF_LORENTZIAN: {
       const double t = a.sigma * s;
-      const double f = 1.0 / (1.0 + t * t);
+      const double f = frcp(fma(t, t, 1.0));
       fs = -2.0 * a.sigma * t * f * f;
       return f;
     }
@@ -312,14 +312,16 @@ __device__ __forceinline__ double shape_factor_grad(double s, double r, const Ar
       const double sg2 = a.sigma * a.sigma;
       const double u = sg2 * ((A - s) * (A + s)) + 1.0;
       const double ss = 4.0 * sg2 * s * s;
-      const double z = sqrt(u * u + ss);
-      const double upz = u >= 0.0 ? u + z : ss / (z - u);
-      const double f = (a.sigma * 0.31830988618379067) * sqrt(2.0 * upz) / z;
+      const double z = fsqrt_pos(fma(u, u, ss));
+      const double iz = frcp(z);
+      const double upz = u >= 0.0 ? u + z : fdiv(ss, z - u);
+      const double f = (a.sigma * 0.31830988618379067) * fsqrt_pos(2.0 * upz) * iz;
       if (upz > 0.0) {
         const double du_s = -2.0 * sg2 * s, du_r = 2.0 * sg2 * A * a.phi;
-        const double dz_s = (u * du_s + 4.0 * sg2 * s) / z, dz_r = u * du_r / z;
-        const double dl_s = 0.5 * (du_s / z + 4.0 * sg2 * s / (z * upz)) - dz_s / z;
-        const double dl_r = 0.5 * du_r / z - dz_r / z;
+        const double dss = 4.0 * sg2 * s;  // half of d(4 sg2 s^2)/ds
+        const double dz_s = fma(u, du_s, dss) * iz, dz_r = u * du_r * iz;
+        const double dl_s = (0.5 * fma(dss, frcp(upz), du_s) - dz_s) * iz;
+        const double dl_r = (0.5 * du_r - dz_r) * iz;
         fs = f * dl_s;
         fr = f * dl_r;
       }
