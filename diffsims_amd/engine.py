@@ -529,7 +529,7 @@ def render_spots(spots: torch.Tensor, count: torch.Tensor, cap: int, shape, sigm
     stream = _lib.stream_handle(dev) if stream is None else stream
     if not fast and cap > int(L.dsx_render_max_spots()):
         # more spots than the render LDS holds: the adjoint kernel's forward
-        # mode renders them chunk by chunk (same pixels as dsx_render_subpixel)
+        # mode renders them tile by tile (same pixels as dsx_render_subpixel)
         work = _workspace(dev, int(L.dsx_render_adjoint_workspace_ints(int(cap), int(n), H, W, 0)),
                           stream)
         sim = _lib.SimParams()
@@ -637,21 +637,22 @@ def polar_templates(spots: torch.Tensor, count: torch.Tensor, cap: int, radial_a
     if width is None:
         width = int(count.max().item()) if n else 0
     axes = radial_axes is not None and azimuthal_axes is not None
-    I = torch.zeros((n, width), dtype=torch.float32, device=dev)
-    n_out = torch.zeros(n, dtype=torch.int32, device=dev)
+    # the kernel writes every entry: its row's spots, then zeros to the width
+    I = torch.empty((n, width), dtype=torch.float32, device=dev)
+    n_out = torch.empty(n, dtype=torch.int32, device=dev)
     stream = _lib.stream_handle(dev) if stream is None else stream
     if axes:
         ra = torch.as_tensor(np.asarray(radial_axes, dtype=np.float64)).to(dev)
         az = torch.as_tensor(np.asarray(azimuthal_axes, dtype=np.float64)).to(dev)
-        r = torch.zeros((n, width), dtype=torch.int32, device=dev)
-        t = torch.zeros((n, width), dtype=torch.int32, device=dev)
+        r = torch.empty((n, width), dtype=torch.int32, device=dev)
+        t = torch.empty((n, width), dtype=torch.int32, device=dev)
         _lib.check(L.dsx_polar_templates(_lib.ptr(spots), _lib.ptr(count), cap, n, width,
                                          _lib.ptr(ra), int(ra.numel()), _lib.ptr(az),
                                          int(az.numel()), None, None, _lib.ptr(r), _lib.ptr(t),
                                          _lib.ptr(I), _lib.ptr(n_out), stream), "dsx_polar_templates")
     else:
-        r = torch.zeros((n, width), dtype=torch.float32, device=dev)
-        t = torch.zeros((n, width), dtype=torch.float32, device=dev)
+        r = torch.empty((n, width), dtype=torch.float32, device=dev)
+        t = torch.empty((n, width), dtype=torch.float32, device=dev)
         _lib.check(L.dsx_polar_templates(_lib.ptr(spots), _lib.ptr(count), cap, n, width, None, 0,
                                          None, 0, _lib.ptr(r), _lib.ptr(t), None, None, _lib.ptr(I),
                                          _lib.ptr(n_out), stream), "dsx_polar_templates")

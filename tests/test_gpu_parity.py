@@ -408,3 +408,47 @@ def test_stream_handle_is_the_current_stream():
             for d in names:
                 assert _lib.stream_handle(d) == want, d
     assert side.cuda_stream != 0
+
+
+@pytest.mark.parametrize("width", [1, 64, 130, 200])
+@pytest.mark.parametrize("axes", [False, True])
+def test_polar_rows_around_a_wave_are_written_to_their_width(width, axes):
+    """Lists of 0 to 130 spots (a wave takes 64 at a time) into buffers that held
+    other values: every entry of a row is its spot's or zero.  r and theta are the
+    FP64 values rounded to FP32, so within one unit of the last place."""
+    import torch
+
+    from diffsims_amd import engine
+
+    counts = [0, 1, 63, 64, 65, 127, 128, 129, 130]
+    print("polar rows", width, axes, flush=True)
+    rng = np.random.default_rng(width)
+    sp = rng.normal(size=(len(counts), 130, 4)).astype(np.float32)
+    dirty = [torch.full((len(counts), width), float("nan"), device="cuda") for _ in range(4)]
+    del dirty
+    kw = {}
+    if axes:
+        ra, az = np.linspace(0, 3, 40), np.linspace(-np.pi, np.pi, 90)
+        kw = dict(radial_axes=ra, azimuthal_axes=az)
+    r, t, I = engine.polar_templates(torch.from_numpy(sp).cuda(),
+                                     torch.tensor(counts, dtype=torch.int32, device="cuda"), 130,
+                                     width=width, **kw)
+    r, t, I = r.cpu().numpy(), t.cpu().numpy(), I.cpu().numpy()
+
+    def nearest(axis, v):
+        i = np.searchsorted(axis, v, side="left")
+        lo, hi = np.clip(i - 1, 0, None), np.clip(i, None, len(axis) - 1)
+        left = (i == len(axis)) | (np.abs(v - axis[lo]) < np.abs(v - axis[hi]))
+        return np.where(left, i - 1, i)
+
+    for o, c in enumerate(counts):
+        x, y = sp[o, :c, 0].astype(np.float64), sp[o, :c, 1].astype(np.float64)
+        er, et, eI = np.hypot(x, y), np.arctan2(y, x), sp[o, :c, 3]
+        if axes:
+            er, et = nearest(ra, er), nearest(az, et)
+            keep = (er < len(ra) - 1) & (et < len(az) - 1)
+            er, et, eI = er[keep], et[keep], eI[keep]
+        m = min(len(er), width)
+        for got, want in ((r, er), (t, et), (I, eI)):
+            assert np.allclose(got[o, :m], want[:m], rtol=1.2e-7, atol=0)
+            assert (got[o, m:] == 0).all()
