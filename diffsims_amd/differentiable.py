@@ -388,7 +388,7 @@ class RefinementModel:
     def workspace(self, cap: int, n: int, gradients: bool = True) -> torch.Tensor:
         """Scratch of dsx_render_adjoint: per-spot sums between its render and
         chain-rule passes and, for spot lists longer than the render LDS
-        holds, per-block strip bins and fixed-point pixels."""
+        holds, per-block tile lists and spots."""
         H, W = self.shape
         need = max(1, int(self.L.dsx_render_adjoint_workspace_ints(int(cap), int(n), H, W,
                                                                    int(gradients))))

@@ -102,7 +102,8 @@ int dsx_hkl_points_in_sphere(const int highest[3], const double metric[6], doubl
  *       value = round(frac * 2^32) mod 2^32),
  *   F2_d[i] = |F|^2,  F_d[i] = {Re F, Im F} (F_d may be NULL).
  * f_e is evaluated and F accumulated in FP64 (the Lobato sums cancel by up to
- * two digits); the per-atom sincos and Debye-Waller exp are FP32.
+ * two digits); the Debye-Waller exp is FP32, and so is the per-atom sincos
+ * except for larger cells (more than 64 atoms, 24 in short tables: FP64).
  * Atoms: elem_d int32 [n_atoms] (row into coeff_d), occ_d, B_d float
  * [n_atoms]; coeff_d double [n_elem][10] = {a1,b1,...,a5,b5};
  * scatter = DSX_SCATTER_*.
@@ -409,11 +410,11 @@ int dsx_render_fast_ragged(const float *spot_d, const long long *spot_off_d, con
  * With cap <= dsx_render_max_spots() it is needed only for gradients
  * (per-spot sums handed from the render pass to the chain-rule pass; EINVAL
  * without it) and every status_d entry is 0.  With a larger cap it holds
- * the strip bins and clip boxes of the patterns, their fixed-point pixels
- * between the splat and the read-out when pattern_d is NULL, and with
- * gradients n * cap per-spot sums (EINVAL without it); when it is missing
- * without gradients, or too small for a pattern's bins, that pattern's
- * status_d entry is 1.  At most 2^22 pixels per pattern.
+ * the spots and tile lists of the patterns and their unscaled pixels until the
+ * maximum is known when pattern_d is NULL, and with gradients n * cap per-spot
+ * sums (EINVAL without it); when it is missing without gradients, or too small
+ * for a pattern's lists, that pattern's status_d entry is 1.  At most 2^22
+ * pixels per pattern.
  * This entry point also serves as the sub-pixel renderer for such large
  * patterns (mode DSX_ADJ_FORWARD).
  */
