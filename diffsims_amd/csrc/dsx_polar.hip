@@ -52,59 +52,64 @@ constexpr int kPolarThreads = 256;
 // arctangent of these are formed.  50,000 orientations of the 40-atom cell: 169 us
 // with 8 blocks per CU looping over the orientations and no loads ahead, 131 with
 // the loads, 120 with a block for every four orientations (floor 58: 272 MB).
-// The rows are written to their full width, so the caller clears nothing.
+// The loop only turns beyond kPolarBlocks blocks (a launch holds less than 2^32
+// threads).  The rows are written to their full width, so the caller clears nothing.
+constexpr int kPolarBlocks = 1 << 23;
+
 __global__ __launch_bounds__(kPolarThreads) void polar_kernel(PolarArgs a) {
   const int lane = lane_id();
   const bool axes = a.radial != nullptr && a.azimuthal != nullptr;
-  const int o = blockIdx.x * (kPolarThreads / kWave) + threadIdx.x / kWave;
-  if (o >= a.n) return;
-  const int n = min(a.count[o], a.cap);
-  const float4 *sp = a.spots + (size_t)o * a.cap;
-  const size_t row = (size_t)o * a.width;
-  int base = 0;
-  const float4 none = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  float4 next = lane < n ? sp[lane] : none;
-  for (int j0 = 0; j0 < n; j0 += kWave) {
-    const int j = j0 + lane;
-    const bool valid = j < n;
-    const float4 s = next;  // the following spots are on their way meanwhile
-    next = j + kWave < n ? sp[j + kWave] : none;
-    const double x = s.x, y = s.y;
-    const double r = sqrt(x * x + y * y);
-    const double t = atan2(y, x);
-    int ri = 0, ti = 0;
-    bool keep = valid;
-    if (axes && valid) {
-      ri = nearest_index(a.radial, a.n_radial, r);
-      ti = nearest_index(a.azimuthal, a.n_azimuthal, t);
-      keep = ri < a.n_radial - 1 && ti < a.n_azimuthal - 1;
-    }
-    const uint64_t m = __ballot(keep);
-    const int pos = base + mask_rank(m);
-    if (keep && pos < a.width) {  // a row narrower than the list keeps its head
-      const size_t q = row + pos;
-      if (axes) {
-        a.r_idx[q] = ri;
-        a.theta_idx[q] = ti;
-      } else {
-        a.r[q] = static_cast<float>(r);
-        a.theta[q] = static_cast<float>(t);
+  const long long waves = static_cast<long long>(gridDim.x) * (kPolarThreads / kWave);
+  for (long long o = static_cast<long long>(blockIdx.x) * (kPolarThreads / kWave) + threadIdx.x / kWave;
+       o < a.n; o += waves) {
+    const int n = min(a.count[o], a.cap);
+    const float4 *sp = a.spots + o * a.cap;
+    const size_t row = (size_t)o * a.width;
+    int base = 0;
+    const float4 none = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 next = lane < n ? sp[lane] : none;
+    for (int j0 = 0; j0 < n; j0 += kWave) {
+      const int j = j0 + lane;
+      const bool valid = j < n;
+      const float4 s = next;  // the following spots are on their way meanwhile
+      next = j + kWave < n ? sp[j + kWave] : none;
+      const double x = s.x, y = s.y;
+      const double r = sqrt(x * x + y * y);
+      const double t = atan2(y, x);
+      int ri = 0, ti = 0;
+      bool keep = valid;
+      if (axes && valid) {
+        ri = nearest_index(a.radial, a.n_radial, r);
+        ti = nearest_index(a.azimuthal, a.n_azimuthal, t);
+        keep = ri < a.n_radial - 1 && ti < a.n_azimuthal - 1;
       }
-      a.I[q] = s.w;
+      const uint64_t m = __ballot(keep);
+      const int pos = base + mask_rank(m);
+      if (keep && pos < a.width) {  // a row narrower than the list keeps its head
+        const size_t q = row + pos;
+        if (axes) {
+          a.r_idx[q] = ri;
+          a.theta_idx[q] = ti;
+        } else {
+          a.r[q] = static_cast<float>(r);
+          a.theta[q] = static_cast<float>(t);
+        }
+        a.I[q] = s.w;
+      }
+      base += __popcll(m);
     }
-    base += __popcll(m);
-  }
-  for (int q = base + lane; q < a.width; q += kWave) {
-    if (axes) {
-      a.r_idx[row + q] = 0;
-      a.theta_idx[row + q] = 0;
-    } else {
-      a.r[row + q] = 0.0f;
-      a.theta[row + q] = 0.0f;
+    for (int q = base + lane; q < a.width; q += kWave) {
+      if (axes) {
+        a.r_idx[row + q] = 0;
+        a.theta_idx[row + q] = 0;
+      } else {
+        a.r[row + q] = 0.0f;
+        a.theta[row + q] = 0.0f;
+      }
+      a.I[row + q] = 0.0f;
     }
-    a.I[row + q] = 0.0f;
+    if (lane == 0 && a.n_out) a.n_out[o] = base;
   }
-  if (lane == 0 && a.n_out) a.n_out[o] = base;
 }
 
 }  // namespace dsx
@@ -149,7 +154,7 @@ extern "C" int dsx_polar_templates(const float *spot_d, const int *count_d, int 
   a.I = I_d;
   a.n_out = n_out_d;
   const int waves_per_block = kPolarThreads / kWave;
-  const int blocks = (n + waves_per_block - 1) / waves_per_block;
+  const int blocks = std::min(n / waves_per_block + (n % waves_per_block != 0), kPolarBlocks);
   hipLaunchKernelGGL(polar_kernel, dim3(blocks), dim3(kPolarThreads), 0, as_stream(stream), a);
   return check_launch("dsx_polar_templates");
 }

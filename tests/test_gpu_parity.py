@@ -452,3 +452,22 @@ def test_polar_rows_around_a_wave_are_written_to_their_width(width, axes):
         for got, want in ((r, er), (t, et), (I, eI)):
             assert np.allclose(got[o, :m], want[:m], rtol=1.2e-7, atol=0)
             assert (got[o, m:] == 0).all()
+
+
+def test_polar_templates_of_more_orientations_than_one_launch_holds():
+    """2^26 + 3 lists of one spot: four orientations per block of 256 threads
+    would be more than the 2^32 threads of a launch."""
+    import torch
+
+    from diffsims_amd import engine
+
+    n = 2 ** 26 + 3
+    print(f"polar: {n} orientations", flush=True)
+    spots = torch.zeros((n, 1, 4), device="cuda")
+    spots[:, 0, 0] = 2.0
+    spots[:, 0, 3] = 5.0
+    spots[-1, 0, :2] = torch.tensor([3.0, 4.0])
+    count = torch.ones(n, dtype=torch.int32, device="cuda")
+    r, t, I = engine.polar_templates(spots, count, 1, width=1)
+    assert bool((r[:-1] == 2).all()) and bool((t[:-1] == 0).all()) and bool((I == 5).all())
+    assert float(r[-1]) == 5.0 and abs(float(t[-1]) - np.arctan2(4.0, 3.0)) < 1e-7
