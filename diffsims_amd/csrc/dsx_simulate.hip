@@ -516,7 +516,7 @@ __global__ __launch_bounds__(kCoopWaves *kWave, 4) void simulate_coop_kernel(Sim
   const float c2f = static_cast<float>(c2);
   int *queue = s_queue[wid];
 
-  for (int o = blockIdx.x; o < d.n_orient; o += gridDim.x) {
+  for (long long o = blockIdx.x; o < d.n_orient; o += gridDim.x) {
     const double *b = d.Rt + static_cast<size_t>(o) * 9;
     if (tid < 9) s_R[tid] = b[tid];
     if (kLines && tid < 4) {
@@ -767,9 +767,14 @@ static int coop_waves(int n_orient, int n_refl, int n_lines, bool precession) {
   return w;
 }
 
+// Blocks of a launch; beyond them the kernel's loop takes the remaining
+// orientations (a launch holds less than 2^32 threads).
+constexpr int kCoopBlocks = 1 << 23;
+
 template <bool kLines>
 static void launch_coop(int waves, const SimArgs &a, hipStream_t s) {
-  const dim3 blocks(static_cast<unsigned>(a.single.n_orient)), threads(static_cast<unsigned>(waves * kWave));
+  const dim3 blocks(static_cast<unsigned>(std::min(a.single.n_orient, kCoopBlocks))),
+      threads(static_cast<unsigned>(waves * kWave));
   switch (waves) {
     case 8: hipLaunchKernelGGL((simulate_coop_kernel<kLines, 8>), blocks, threads, 0, s, a); break;
     case 4: hipLaunchKernelGGL((simulate_coop_kernel<kLines, 4>), blocks, threads, 0, s, a); break;

@@ -318,3 +318,35 @@ def test_few_orientations_with_a_short_list():
         n = b.n
         assert_same_batches(b, engine.SpotBatch(tab, big.idx[:n], big.spots[:n], big.count[:n],
                                                 big.ncand[:n], big.maxI[:n], 50))
+
+
+def test_precession_batch_of_more_orientations_than_one_launch_holds():
+    """Under precession a table of long line lists takes a wave per orientation at
+    any batch size: 2^26 + 3 of them would be more than the 2^32 threads of a
+    launch.  Rows far above the Ewald sphere of every orientation but the last."""
+    from diffsims_amd import engine
+
+    n = 2 ** 26 + 3
+    print(f"precession: {n} orientations", flush=True)
+    h, k, l = np.meshgrid(np.arange(-16, 16), np.arange(-32, 32), np.arange(100, 90, -1), indexing="ij")
+    hkl = np.stack([h, k, l, 0 * h], -1).reshape(-1, 4).astype(np.int32)
+    rec = 0.05 * np.eye(3)
+    g = hkl[:, :3] @ rec.T
+    g4 = np.c_[g, (g * g).sum(1)].astype(np.float32)
+    d_hkl, d_g4 = torch.from_numpy(hkl).cuda(), torch.from_numpy(g4).cuda()
+    tab = engine.PhaseTable(d_hkl, d_g4, torch.ones(len(hkl), device="cuda"), None, len(hkl), False,
+                            float(np.sqrt(g4[:, 3].max())), rec, np.eye(3), "",
+                            engine.build_lines(d_hkl, d_g4))
+    assert uses_lines(tab) and tab.n_lines == 2048
+    st = engine.SimSettings(max_excitation_error=0.02, precession_angle=0.2)
+    Rt = torch.eye(3, dtype=torch.float64, device="cuda").reshape(1, 9).expand(n, 9).contiguous()
+    Rt[-1] = torch.tensor([0, 0, 1, 0, 1, 0, -1, 0, 0], dtype=torch.float64)
+    out = engine.empty_batch(tab, n, 1, Rt.device)
+    out.ncand.fill_(-1)
+    out.count.fill_(-1)
+    engine.simulate_into(tab, Rt, st, out)
+    one = engine.empty_batch(tab, 1, 1, Rt.device)
+    engine.simulate_into(tab, Rt[-1:].contiguous(), st, one)
+    assert not out.ncand[:-1].any() and not out.count[:-1].any()
+    assert int(one.ncand) > 0 and int(out.ncand[-1]) == int(one.ncand)
+    assert torch.equal(out.spots[-1], one.spots[0])
