@@ -1172,11 +1172,32 @@ __host__ __device__ __forceinline__ long long long_plan_bytes(int cap, int H, in
 }
 
 // Fixed-point term of the writer: render_kernel's truncation, or for long
-// lists, where the truncations of many terms would add up, the nearest unit
-// (the terms are non-negative).
+// lists, where the truncations of many terms would add up, the nearest unit.
 template <bool kLong>
 __device__ __forceinline__ int band_term(float iws, float wy) {
-  return kLong ? static_cast<int>(fmaf(iws, wy, 0.5f)) : fast_fixed(iws, wy);
+  return kLong ? static_cast<int>(fmaf(iws, wy, copysignf(0.5f, iws))) : fast_fixed(iws, wy);
+}
+
+// A pattern of a long list that fixed point cannot hold: a NaN or an infinity
+// among the spots that are seen, or a largest intensity so small or large that
+// the scale or the bounds leave FP32's range.  Its pixels are formed in FP32,
+// so that NaN and infinities reach the pixels of their taps.
+constexpr float kLongLeast = 1e-24f, kLongMost = 1e33f;
+constexpr int kFloatPattern = 2;  // rec[0]: the writer takes band_pixel_sum
+
+// FP32 value of pixel (x, y) from the entries [e0, e1); at(e, xi, yi, I).
+template <int kR, class At>
+__device__ __forceinline__ float band_pixel_sum(int x, int y, int e0, int e1, int H, int W,
+                                                const float *taps, const At &at) {
+  float v = 0.0f;
+  for (int e = e0; e < e1; ++e) {
+    int xi, yi;
+    float I;
+    at(e, xi, yi, I);
+    if (I == 0.0f || x < xi - kR || x > xi + kR || y < yi - kR || y > yi + kR) continue;
+    v = fmaf(I * band_weight(x, xi, W, kR, taps), band_weight(y, yi, H, kR, taps), v);
+  }
+  return v;
 }
 
 // Largest pixel of the 16x16 tile t (at least `best`), by one wave: a splat of
@@ -1246,7 +1267,7 @@ __global__ __launch_bounds__(kLongThreads) void render_plan_long_kernel(BandArgs
   __shared__ float s_tp[kR + 1];
   __shared__ float s_pm[kLongWaves];
   __shared__ int s_n[kLongWaves], s_u[kLongWaves];
-  __shared__ int s_q, s_best;
+  __shared__ int s_q, s_best, s_odd;
   const RenderArgs &a = b.r;
   constexpr int R = kR;
   const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
@@ -1265,7 +1286,10 @@ __global__ __launch_bounds__(kLongThreads) void render_plan_long_kernel(BandArgs
   for (int t = tid; t <= H; t += kLongThreads) rows[t] = 0;
   for (int t = tid; t < n_tiles; t += kLongThreads) tile_u[t] = 0;
   if (tid <= R) s_tp[tid] = a.taps[tid];
-  if (tid == 0) s_q = 0x7fffffff;
+  if (tid == 0) {
+    s_q = 0x7fffffff;
+    s_odd = 0;
+  }
   lds_sync();
   // ---- spots per row, row starts, the list sorted by row ------------------
   for (int j = tid; j < n; j += kLongThreads) {
@@ -1311,7 +1335,9 @@ __global__ __launch_bounds__(kLongThreads) void render_plan_long_kernel(BandArgs
     if (lose) {
       s_I[e] = 0.0f;  // contributes nothing
     } else {
-      pm = fmaxf(pm, fabsf(s_I[e]));
+      const float aI = fabsf(s_I[e]);
+      if (!(aI < INFINITY)) s_odd = 1;
+      pm = fmaxf(pm, aI);
       ++mine;
     }
   }
@@ -1329,78 +1355,105 @@ __global__ __launch_bounds__(kLongThreads) void render_plan_long_kernel(BandArgs
     pmax = fmaxf(pmax, s_pm[w]);
     ns += s_n[w];
   }
-  // ---- tile bounds and the fixed-point scale (as tile_bounds) --------------
-  const float w0 = s_tp[0];
-  const float inv_p = pmax > 0.0f ? kLongUnits / pmax : 0.0f;
-  for (int e = tid; e < total; e += kLongThreads) {
-    const float I = s_I[e];
-    if (I == 0.0f) continue;
-    if (fabsf(I) == pmax) atomicMin(&s_q, e);
-    const int yi = s_y[e], xi = s_key[e] >> 16;
-    const bool inx = xi >= R && xi + R < W, iny = yi >= R && yi + R < H;
-    const float bx = inx ? w0 : fminf(1.0f, 3.0f * w0);
-    const float by = iny ? w0 : fminf(1.0f, 3.0f * w0);
-    const float aI = fabsf(I);
-    // a footprint of at most 17 pixels reaches at most two tiles per axis
-    const int tx0 = max(0, xi - R) / kTile, tx1 = min(W - 1, xi + R) / kTile;
-    const int ty0 = max(0, yi - R) / kTile, ty1 = min(H - 1, yi + R) / kTile;
-    for (int ty = ty0; ty <= ty1; ++ty)
-      for (int tx = tx0; tx <= tx1; ++tx) {
-        // the taps fall off from the centre: a tile's largest weight is at
-        // its pixel nearest (xi, yi)
-        const bool in = inx && iny;
-        const float wx = in ? s_tp[tile_gap(tx, xi)] : bx, wy = in ? s_tp[tile_gap(ty, yi)] : by;
-        atomicAdd(&tile_u[ty * ntx + tx], bound_units(aI, wx, wy, inv_p));
+  float scale = 0.0f, out_scale = 1.0f;
+  // uniform: s_odd was written before the barrier
+  const bool in_float = s_odd != 0 || (pmax > 0.0f && !(pmax >= kLongLeast && pmax <= kLongMost));
+  if (in_float) {
+    if (a.normalize) {  // the maximum passes over NaN (an infinite one leaves NaN and zeros)
+      float m = 0.0f;
+      for (int i = tid; i < H * W; i += kLongThreads) {
+        const int y = i / W;
+        m = fmaxf(m, band_pixel_sum<R>(i - y * W, y, rows[max(0, y - R)], rows[min(H - 1, y + R) + 1], H, W,
+                                       s_tp, [&](int e, int &xi, int &yi, float &I) {
+                                         xi = s_key[e] >> 16;
+                                         yi = s_y[e];
+                                         I = s_I[e];
+                                       }));
       }
-  }
-  lds_sync();
-  int lu = 0;
-  for (int t = tid; t < n_tiles; t += kLongThreads) lu = max(lu, tile_u[t]);
-  lu = wave_max_i(lu);
-  if (lane == 0) s_u[wid] = lu;
-  lds_sync();
-  int Ui = 0;
+      m = wave_max(m);
+      lds_sync();  // every wave has read s_pm
+      if (lane == 0) s_pm[wid] = m;
+      lds_sync();
+      m = 0.0f;
 #pragma unroll
-  for (int w = 0; w < kLongWaves; ++w) Ui = max(Ui, s_u[w]);
-  const float unit = pmax / kLongUnits;
-  const float U = static_cast<float>(Ui) * unit;
-  const float scale = U > 0.0f ? kScaleRange / (U * 1.00001f) : 1.0f;
-  float out_scale = 1.0f / scale;
-  if (a.normalize && pmax > 0.0f) {
-    // ---- exact maximum: every tile whose bound can reach the value at the
-    // brightest spot's pixel, shared over the waves (the bound keeps every
-    // pixel sum below 2^31)
-    const int qs = s_q;
-    const int ys = s_y[qs], xs = s_key[qs] >> 16;
-    int acc = 0;
-    for (int e = rows[max(0, ys - R)] + lane; e < rows[min(H - 1, ys + R) + 1]; e += kWave) {
+      for (int w = 0; w < kLongWaves; ++w) m = fmaxf(m, s_pm[w]);
+      if (m > 0.0f) out_scale = 1.0f / m;
+    }
+  } else {
+    // ---- tile bounds and the fixed-point scale (as tile_bounds) --------------
+    const float w0 = s_tp[0];
+    const float inv_p = pmax > 0.0f ? kLongUnits / pmax : 0.0f;
+    for (int e = tid; e < total; e += kLongThreads) {
+      const float I = s_I[e];
+      if (I == 0.0f) continue;
+      if (fabsf(I) == pmax) atomicMin(&s_q, e);
       const int yi = s_y[e], xi = s_key[e] >> 16;
-      if (xs < xi - R || xs > xi + R) continue;
-      const float iws = s_I[e] * band_weight(xs, xi, W, R, s_tp) * scale;
-      if (iws != 0.0f) acc += band_term<true>(iws, band_weight(ys, yi, H, R, s_tp));
-    }
-    const int lfix = wave_sum(acc);
-    // a term rounds up by at most half a unit
-    const float margin = 0.5f * static_cast<float>(ns) + 1.0f;
-    if (tid == 0) s_best = lfix;
-    lds_sync();
-    for (int t = wid; t < n_tiles; t += kLongWaves) {
-      const float bound = static_cast<float>(tile_u[t]) * unit * scale * 1.00001f + margin;
-      const int best = *const_cast<volatile int *>(&s_best);
-      if (static_cast<double>(bound) < static_cast<double>(best)) continue;
-      const int ty = t / ntx;
-      const int m = tile_max<R>(a, t - ty * ntx, ty, rows[max(0, ty * kTile - R)],
-                                rows[min(H - 1, ty * kTile + kTile - 1 + R) + 1], s_key, s_I, s_y,
-                                s_tp, scale, s_tile[wid], s_cq[wid], lane, best);
-      if (lane == 0 && m > best) atomicMax(&s_best, m);
+      const bool inx = xi >= R && xi + R < W, iny = yi >= R && yi + R < H;
+      const float bx = inx ? w0 : fminf(1.0f, 3.0f * w0);
+      const float by = iny ? w0 : fminf(1.0f, 3.0f * w0);
+      const float aI = fabsf(I);
+      // a footprint of at most 17 pixels reaches at most two tiles per axis
+      const int tx0 = max(0, xi - R) / kTile, tx1 = min(W - 1, xi + R) / kTile;
+      const int ty0 = max(0, yi - R) / kTile, ty1 = min(H - 1, yi + R) / kTile;
+      for (int ty = ty0; ty <= ty1; ++ty)
+        for (int tx = tx0; tx <= tx1; ++tx) {
+          // the taps fall off from the centre: a tile's largest weight is at
+          // its pixel nearest (xi, yi)
+          const bool in = inx && iny;
+          const float wx = in ? s_tp[tile_gap(tx, xi)] : bx, wy = in ? s_tp[tile_gap(ty, yi)] : by;
+          atomicAdd(&tile_u[ty * ntx + tx], bound_units(aI, wx, wy, inv_p));
+        }
     }
     lds_sync();
-    const int best = s_best;
-    // a zero maximum leaves the zeros as they are instead of producing 0/0
-    if (best > 0) out_scale = 1.0f / static_cast<float>(best);
+    int lu = 0;
+    for (int t = tid; t < n_tiles; t += kLongThreads) lu = max(lu, tile_u[t]);
+    lu = wave_max_i(lu);
+    if (lane == 0) s_u[wid] = lu;
+    lds_sync();
+    int Ui = 0;
+#pragma unroll
+    for (int w = 0; w < kLongWaves; ++w) Ui = max(Ui, s_u[w]);
+    const float unit = pmax / kLongUnits;
+    const float U = static_cast<float>(Ui) * unit;
+    scale = U > 0.0f ? kScaleRange / (U * 1.00001f) : 1.0f;
+    out_scale = 1.0f / scale;
+    if (a.normalize && pmax > 0.0f) {
+      // ---- exact maximum: every tile whose bound can reach the value at the
+      // brightest spot's pixel, shared over the waves (the bound keeps every
+      // pixel sum below 2^31)
+      const int qs = s_q;
+      const int ys = s_y[qs], xs = s_key[qs] >> 16;
+      int acc = 0;
+      for (int e = rows[max(0, ys - R)] + lane; e < rows[min(H - 1, ys + R) + 1]; e += kWave) {
+        const int yi = s_y[e], xi = s_key[e] >> 16;
+        if (xs < xi - R || xs > xi + R) continue;
+        const float iws = s_I[e] * band_weight(xs, xi, W, R, s_tp) * scale;
+        if (iws != 0.0f) acc += band_term<true>(iws, band_weight(ys, yi, H, R, s_tp));
+      }
+      const int lfix = wave_sum(acc);
+      // a term rounds up by at most half a unit
+      const float margin = 0.5f * static_cast<float>(ns) + 1.0f;
+      if (tid == 0) s_best = lfix;
+      lds_sync();
+      for (int t = wid; t < n_tiles; t += kLongWaves) {
+        const float bound = static_cast<float>(tile_u[t]) * unit * scale * 1.00001f + margin;
+        const int best = *const_cast<volatile int *>(&s_best);
+        if (static_cast<double>(bound) < static_cast<double>(best)) continue;
+        const int ty = t / ntx;
+        const int m = tile_max<R>(a, t - ty * ntx, ty, rows[max(0, ty * kTile - R)],
+                                  rows[min(H - 1, ty * kTile + kTile - 1 + R) + 1], s_key, s_I, s_y,
+                                  s_tp, scale, s_tile[wid], s_cq[wid], lane, best);
+        if (lane == 0 && m > best) atomicMax(&s_best, m);
+      }
+      lds_sync();
+      const int best = s_best;
+      // a zero maximum leaves the zeros as they are instead of producing 0/0
+      if (best > 0) out_scale = 1.0f / static_cast<float>(best);
+    }
   }
   if (tid == 0) {
-    *reinterpret_cast<int4 *>(rec) = make_int4(0, ns, __float_as_int(scale), __float_as_int(out_scale));
+    *reinterpret_cast<int4 *>(rec) =
+        make_int4(in_float ? kFloatPattern : 0, ns, __float_as_int(scale), __float_as_int(out_scale));
     if (a.status) a.status[p] = 0;
   }
   for (int bb = tid; bb < b.nb; bb += kLongThreads) {
@@ -1475,10 +1528,24 @@ __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
   for (int i = 0; i <= R; ++i)
     if (tid == i) s_tp[i] = a.taps[i];
   for (int v = tid; v < nvec; v += kBandThreads) reinterpret_cast<int4 *>(s_acc)[v] = make_int4(0, 0, 0, 0);
-  if (h.x != 0) return;  // listed for render_kernel (uniform across the block)
+  if (!kLong && h.x != 0) return;  // listed for render_kernel (uniform across the block)
   const int total = e1 - e0;
   const int2 *ent = b.ent + static_cast<size_t>(pl) * (kLong ? b.ent_stride : kPlanMax) + e0;
   const float scale = __int_as_float(h.z), out_scale = __int_as_float(h.w);
+  if (kLong && h.x == kFloatPattern) {  // uniform
+    lds_sync();                         // the taps
+    for (int i = tid; i < static_cast<int>(pixels); i += kBandThreads) {
+      const int r = i / W;
+      first[i] = out_scale * band_pixel_sum<R>(i - r * W, y0 + r, 0, total, H, W, s_tp,
+                                               [&](int e, int &xi, int &yi, float &I) {
+                                                 const int2 en = ent[e];
+                                                 xi = en.x & 0xffff;
+                                                 yi = en.x >> 16;
+                                                 I = __int_as_float(en.y);
+                                               });
+    }
+    return;
+  }
   for (int c0 = 0;; c0 += kPlanMax) {  // one turn unless kLong
     const int cnt = kLong ? min(kPlanMax, total - c0) : total;
     for (int q = tid; q < cnt; q += kBandThreads) s_ent[q] = ent[c0 + q];

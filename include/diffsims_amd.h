@@ -318,6 +318,9 @@ int dsx_render_fast_bands(const float *spot_d, const int *count_d, int cap, int 
  *   work_d : dsx_render_fast_long_workspace_ints(cap, n, height, width) ints,
  *            16-byte aligned (patterns are taken in rounds that reuse it in
  *            stream order); overlapping calls must not share it
+ * NaN and infinite intensities reach the pixels of their taps, as in the
+ * reference's filter; such a pattern, and one whose largest intensity is below
+ * 1e-24 or above 1e33, is formed in FP32.  Negative intensities are taken.
  * Other arguments as for dsx_render_fast; status_d is 0 for every pattern.
  */
 int dsx_render_fast_long_fits(int cap, int radius, int height, int width);

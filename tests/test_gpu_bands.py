@@ -268,6 +268,13 @@ def test_render_spots_same_bits_across_the_small_batch_threshold():
 
 def _render_long(spots, cnt, cap, shape, sigma, normalize=True):
     import torch
+    out = _render_long_any(spots, cnt, cap, shape, sigma, normalize)
+    assert not torch.isnan(out).any()
+    return out
+
+
+def _render_long_any(spots, cnt, cap, shape, sigma, normalize=True):
+    import torch
     from diffsims_amd import engine
     lib, L = _lib()
     n = int(cnt.shape[0])
@@ -281,7 +288,7 @@ def _render_long(spots, cnt, cap, shape, sigma, normalize=True):
     lib.check(L.dsx_render_fast_long(lib.ptr(spots), lib.ptr(cnt), cap, n, ctypes.byref(p),
                                      lib.ptr(work), ws, lib.ptr(out), lib.ptr(st),
                                      lib.stream_handle(spots.device)), "dsx_render_fast_long")
-    assert not torch.isnan(out).any() and not st.any()
+    assert not st.any()
     return out
 
 
@@ -370,3 +377,67 @@ def test_long_lists_dispatch_and_limits():
                                     lib.ptr(work), ws, lib.ptr(out), None,
                                     lib.stream_handle(spots.device))
         assert rc == lib.DSX_EINVAL
+
+
+def _render_windowed(spots, cnt, cap, shape, sigma, normalize):
+    """dsx_render_fast_large: the spot image filtered in FP32."""
+    import torch
+    from diffsims_amd import engine
+    lib, L = _lib()
+    n = int(cnt.shape[0])
+    p = engine.render_params(shape, sigma, 1.0, normalize=normalize)
+    out = torch.full((n, *shape), float("inf"), dtype=torch.float32, device="cuda")
+    ws = int(L.dsx_render_fast_large_workspace_ints(cap))
+    work = torch.empty(ws, dtype=torch.int32, device="cuda")
+    lib.check(L.dsx_render_fast_large(lib.ptr(spots), lib.ptr(cnt), cap, n, ctypes.byref(p),
+                                      lib.ptr(work), ws, lib.ptr(out), None,
+                                      lib.stream_handle(spots.device)), "dsx_render_fast_large")
+    return out
+
+
+@pytest.mark.parametrize("shape,sigma", [((256, 256), 1.0), ((231, 201), 1.75)])
+@pytest.mark.parametrize("normalize", [True, False])
+def test_long_lists_of_intensities_beyond_fixed_point(shape, sigma, normalize):
+    """NaN, infinities, negative and very small or large intensities: NaN and
+    infinities where the FP32 filter has them, every other pixel within its
+    tolerance of the largest (LONG_TOL, and the filter's own 2 R + 1 roundings
+    along both axes)."""
+    import torch
+    print(f"long lists beyond fixed point: {shape}, sigma {sigma}, normalize {normalize}", flush=True)
+    n, cap = 12, 1400
+    spots, cnt = _spot_lists(n, cap, *shape, 1300, seed=21, edge=0.1, R=7)
+    inf, nan = float("inf"), float("nan")
+    spots[0, 5, 3] = nan
+    spots[1, 7, 3] = inf
+    spots[2, 9, 3] = -inf
+    spots[3, 11, 3], spots[3, 12, 3] = nan, inf
+    spots[4, 3, 3] = nan                      # under a later spot: not seen
+    spots[4, 900, :2] = spots[4, 3, :2]
+    spots[5, :, 3] = nan
+    spots[6, ::3, 3] *= -1.0
+    spots[7, :, 3] *= -1.0                    # no positive pixel: not normalised
+    spots[8, :, 3] *= 1e-31
+    spots[9, :, 3] *= 1e34
+    spots[10, 0:2, :2] = torch.tensor([[-shape[1] // 2 + 1.5, 0.0], [0.0, -shape[0] // 2 + 0.5]])
+    spots[10, 0:2, 3] = torch.tensor([nan, inf])   # reflected at the edges
+    cnt[11] = 2
+    spots[11, 0:2, 3] = torch.tensor([nan, 1.0])
+    got = _render_long_any(spots, cnt, cap, shape, sigma, normalize)
+    ref = _render_windowed(spots, cnt, cap, shape, sigma, normalize)
+    for i in range(n):
+        a, r = got[i], ref[i]
+        assert torch.equal(torch.isnan(a), torch.isnan(r)), i
+        assert torch.equal(torch.isinf(a), torch.isinf(r)), i
+        ok = torch.isfinite(r)
+        assert torch.equal(a[~ok].sign().nan_to_num(2.0), r[~ok].sign().nan_to_num(2.0)), i
+        top = float(r[ok].double().abs().max()) if ok.any() else 0.0
+        tol = LONG_TOL + 2 * 15 * 2.0 ** -24
+        assert float((a[ok].double() - r[ok].double()).abs().max() if ok.any() else 0.0) <= tol * top, i
+    # patterns of ordinary lists do not notice their neighbours
+    plain = _render_long(spots[6:8].contiguous(), cnt[6:8].contiguous(), cap, shape, sigma, normalize)
+    assert torch.equal(plain, got[6:8])
+    which = [4, 6]
+    clean = spots.clone()
+    clean[4, 3, 3] = 1.0
+    for i, r in zip(which, _fp64_patterns(clean, cnt, shape, sigma, normalize, which)):
+        assert np.abs(got[i].cpu().numpy() - r).max() <= LONG_TOL * np.abs(r).max()
