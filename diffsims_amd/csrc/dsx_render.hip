@@ -1005,7 +1005,8 @@ __global__ __launch_bounds__(kPlanThreads) void render_plan_kernel(BandArgs b) {
 #pragma unroll
         for (int k = 0; k < kPlanPerLane; ++k)
           if (key[k] >= 0 && fabsf(Iv[k]) == pmax) qc = min(qc, pos[k]);
-        const int qs = wave_min_i(qc);
+        // (no spot matches when every intensity is NaN: any entry then)
+        const int qs = min(wave_min_i(qc), rows[H] - 1);
         const int ys = key_y(s_key[qs]), xs = key_x(s_key[qs]);
         long long acc = 0;
 #pragma unroll

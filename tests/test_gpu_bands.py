@@ -441,3 +441,22 @@ def test_long_lists_of_intensities_beyond_fixed_point(shape, sigma, normalize):
     clean[4, 3, 3] = 1.0
     for i, r in zip(which, _fp64_patterns(clean, cnt, shape, sigma, normalize, which)):
         assert np.abs(got[i].cpu().numpy() - r).max() <= LONG_TOL * np.abs(r).max()
+
+
+@pytest.mark.parametrize("shape", [(96, 101), (96, 100)])
+def test_short_lists_of_any_intensity_equal_the_splat_renderer(shape):
+    # the same bits, NaN included, as the renderer whose calls they take over
+    import torch
+    print(f"bands: intensities of any kind, {shape}", flush=True)
+    spots, cnt = _spot_lists(8, 96, *shape, 60, seed=4)
+    inf, nan = float("inf"), float("nan")
+    spots[0, 5, 3] = nan
+    spots[1, 7, 3] = inf
+    spots[2, :, 3] = nan
+    spots[3, ::3, 3] *= -1.0
+    spots[4, :, 3] *= -1.0
+    spots[5, :, 3] = 0.0
+    spots[6, 9, 3] = -inf
+    ref, out, st_ref, st, _ = _render_both(spots, cnt, 96, shape, 1.0)
+    assert torch.equal(st_ref, st)
+    assert torch.equal(out.view(torch.int32), ref.view(torch.int32))
