@@ -184,12 +184,20 @@ __device__ __forceinline__ void tiles_body(const Args &a, int *s_tiles, TileShar
   const int pos = lane & 15, sub = lane >> 4;
   const bool grad = !kFwd && a.want_grad;
 
+  // no room: the pattern is reported in status and left as zeros
+  auto refuse = [&](int p) {
+    if (a.pattern)
+      for (size_t i = tid; i < HW; i += kTileThreads) a.pattern[static_cast<size_t>(p) * HW + i] = 0.0f;
+    if (tid == 0) {
+      if (a.loss) a.loss[p] = 0.0f;
+      if (a.status) a.status[p] = 1;
+      if (grad) a.gcount[p] = 0;
+    }
+  };
+
   for (int p = blockIdx.x; p < a.n; p += gridDim.x) {
-    if (!a.work) {  // no room: the pattern is reported in status and left as zeros
-      if (a.pattern)
-        for (size_t i = tid; i < HW; i += kTileThreads) a.pattern[static_cast<size_t>(p) * HW + i] = 0.0f;
-      if (tid == 0 && a.loss) a.loss[p] = 0.0f;
-      if (tid == 0 && a.status) a.status[p] = 1;
+    if (!a.work) {
+      refuse(p);
       continue;
     }
     const int n = min(a.count[p], a.cap);
@@ -272,6 +280,24 @@ __device__ __forceinline__ void tiles_body(const Args &a, int *s_tiles, TileShar
     // ---- starts: exclusive scan over the tiles -----------------------------
     const int per = (n_tiles + kTileThreads - 1) / kTileThreads;
     const int i0 = min(n_tiles, tid * per), i1 = min(n_tiles, i0 + per);
+    // entries are numbered in 32 bits: lists with more of them (131,100 boxes
+    // over all of a 256 x 16,384 pattern's tiles) are not taken
+    if (static_cast<long long>(n) * n_tiles > 0x7fffffffll) {
+      double all = 0.0;
+      for (int t = i0; t < i1; ++t)
+        for (int w = 0; w < cw; ++w) all += s_start[w * n_tiles + t];
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) all += __shfl_xor(all, off, kWave);
+      if (lane == 0) sh.red[wid][0] = all;
+      lds_sync();
+      all = 0.0;
+      for (int w = 0; w < kTileWaves; ++w) all += sh.red[w][0];
+      if (all > 2147483647.0) {
+        refuse(p);
+        __syncthreads();
+        continue;
+      }
+    }
     {
       int sum = 0;
       for (int t = i0; t < i1; ++t)
@@ -299,6 +325,8 @@ __device__ __forceinline__ void tiles_body(const Args &a, int *s_tiles, TileShar
     bool bounded = false;
     auto scatter = [&](int t0, int t1) {
       const int first = s_start[t0];
+      // later ranges only visit the tile rows they hold
+      const int row0 = bounded ? t0 / ntx : 0, row1 = bounded ? (t1 - 1) / ntx : n_tiles;
       const float inv_p = pmax > 0.0f ? a.bound_units / pmax : 0.0f;
       lds_sync();
       each_spot([&](int j0, int j, bool in, float amp, float X, float Y, int lo, int hi, int xlo, int xhi) {
@@ -335,7 +363,7 @@ __device__ __forceinline__ void tiles_body(const Args &a, int *s_tiles, TileShar
             if (tx1 > tx0) entry(t + ntx + 1, x - 16.0f, y - 16.0f, yhigh | xhigh, gx1, gy1);
           }
         } else {
-          for (int ty = ty0; ty <= ty1; ++ty)
+          for (int ty = max(ty0, row0); ty <= min(ty1, row1); ++ty)
             for (int tx = tx0; tx <= tx1; ++tx) {
               const float x = X - static_cast<float>(tx * kTileEdge), y = Y - static_cast<float>(ty * kTileEdge);
               const int bits = tile_bits(lo - ty * kTileEdge, hi - ty * kTileEdge) |

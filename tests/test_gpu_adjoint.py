@@ -558,6 +558,30 @@ def test_long_lists_without_workspace_report_their_patterns():
     assert bool((st == 1).all()) and bool((out == 0).all())
 
 
+def test_more_tile_entries_than_are_numbered_are_refused():
+    """131,100 boxes over all 16,384 tiles of a 256 x 16,384 pattern are more than
+    2^31 - 1 entries: the pattern is reported and left as zeros, its neighbour in
+    the batch is not touched by it."""
+    import torch
+    from diffsims_amd import engine
+
+    cap, sigma, shape = 131100, 1800.0, (256, 16384)
+    print("tiles: 2^31 entries", flush=True)
+    spots = torch.zeros((2, cap, 4), device="cuda")
+    spots[0, :, 3] = 1e13          # radius 9,200 pixels from the centre
+    spots[1, :100, 3] = 1e9        # radius 5,000
+    spots[1, :100, 0] = torch.arange(100.0, device="cuda") * 8 - 400
+    count = torch.tensor([cap, 100], dtype=torch.int32, device="cuda")
+    status = torch.full((2,), -1, dtype=torch.int32, device="cuda")
+    out = torch.full((2, *shape), float("nan"), device="cuda")
+    engine.render_spots(spots, count, cap, shape, sigma, 1.0, fast=False, out=out, status=status)
+    assert status.tolist() == [1, 0]
+    assert not out[0].any() and float(out[1].max()) == 1.0
+    alone = engine.render_spots(spots[1:, :2000].contiguous(), count[1:], 2000, shape, sigma, 1.0,
+                                fast=False)
+    assert torch.equal(alone[0], out[1])
+
+
 # rows, atoms, elements, table: either side of the lines between the kernels with
 # a thread per reflection and a lane per atom (23/24, 47/48, 64/65 and 512/513
 # atoms, 20/21 elements, 24,576 and 65,536 rows), and row counts around a wave's 16
