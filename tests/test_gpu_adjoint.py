@@ -558,6 +558,35 @@ def test_long_lists_without_workspace_report_their_patterns():
     assert bool((st == 1).all()) and bool((out == 0).all())
 
 
+@pytest.mark.parametrize("n", [60, 64, 65, 130, 20000])
+def test_pixels_of_many_boxes_in_one_place_keep_fp32_precision(n):
+    """n equal boxes: every pixel within the error of its terms and of the sum of
+    64 of them.  A term has two exponentials (2^-23 each), five roundings of
+    2^-24 and arguments of at most log2(7) that are off by three; 64 terms are 33
+    additions; the sum over the sixty-fours is FP64."""
+    import torch
+    from diffsims_amd import engine
+
+    print(f"tiles: {n} boxes in one place", flush=True)
+    cap, H, W, sigma, X, Y = 20480, 64, 72, 6.0, 32.3, 31.7   # box edges are 0.1 and more off a pixel
+    pref = 1.0 / (2.0 * np.pi * sigma ** 2)
+    spots = torch.zeros((1, cap, 4), device="cuda")
+    spots[0, :n] = torch.tensor([X - (W - 1) / 2, Y - (H - 1) / 2, 0.0, 7.0 / pref], device="cuda")
+    count = torch.tensor([n], dtype=torch.int32, device="cuda")
+    got = engine.render_spots(spots, count, cap, (H, W), sigma, 1.0, fast=False, normalize=False)[0]
+    s = spots[0, 0].double().cpu().numpy()
+    x, y = s[0] + (W - 1) / 2, s[1] + (H - 1) / 2
+    d2 = (np.arange(W) - x) ** 2, (np.arange(H) - y) ** 2
+    rad2 = 2 * sigma ** 2 * np.log(s[3] * pref)
+    k = [np.where(d <= rad2, np.exp(-d / (2 * sigma ** 2)), 0.0) for d in d2]
+    ref = n * s[3] * pref * np.outer(k[1], k[0])
+    assert (ref > 0).sum() == 24 * 24
+    # and the pixel position itself is one FP32 addition: 2^-19 at 32
+    tol = 2 * 2.0 ** -23 + (5 + 33) * 2.0 ** -24 + 3 * 2.0 ** -24 * np.log(7.0)
+    shift = 2.0 ** -19 / sigma ** 2 * 12 * 2
+    assert (np.abs(got.cpu().numpy() - ref) <= (tol + shift) * ref).all()
+
+
 def test_more_tile_entries_than_are_numbered_are_refused():
     """131,100 boxes over all 16,384 tiles of a 256 x 16,384 pattern are more than
     2^31 - 1 entries: the pattern is reported and left as zeros, its neighbour in
