@@ -1056,27 +1056,37 @@ __global__ __launch_bounds__(kSfaThreads) void structure_factor_adjoint_kernel(S
 // reflection (whose per-atom sums cross the wave 24 times), 2.56 here.
 constexpr int kSfaRun = 4;
 
-__global__ __launch_bounds__(kAtomThreads, 4) void structure_factor_adjoint_atoms_kernel(SfAdjArgs a,
-                                                                                        int rows) {
+// FP32 sums of the blocks meet in float atomics, whose rounding grows with the
+// number of blocks: with 64 rows a block the gradients' error was 1.3 to 2 times
+// that of the thread-per-reflection kernel (256 rows a block) up to 64 k rows
+// (60,000 rows x 48 atoms 2.9e-7 -> 5.1e-7 of the norm).  A block takes at least
+// 256 rows, with as many waves as its LDS holds: 2.9e-7, and 84 -> 44 us there,
+// 17,332 rows x 48 atoms 35 -> 29; 4,614 rows x 24 atoms 1.4e-7 -> 1.9e-7 -> 1.2e-7,
+// where 18.5 us (64 rows) become 25.5 (a thread per reflection: 48).
+constexpr int kSfaAtomRows = 256;
+
+template <int kWaves>
+__global__ __launch_bounds__(kWaves *kWave, 4) void structure_factor_adjoint_atoms_kernel(SfAdjArgs a,
+                                                                                          int rows) {
   // the atoms | their sums [4][n_atoms] | per wave: f and df/dq [n_elem][kAtomRows + 1]
   extern __shared__ double s_dyn[];
-  __shared__ int4 s_hkl[kAtomWaves][kAtomRows];
-  __shared__ double s_g2[kAtomWaves][kAtomRows], s_w[kAtomWaves][kAtomRows];
-  __shared__ double s_F[kAtomWaves][kSfaRun][4];  // of the run: Fr, Fi, then w Fr, w Fi
-  __shared__ double s_rec[kAtomWaves][9];
+  __shared__ int4 s_hkl[kWaves][kAtomRows];
+  __shared__ double s_g2[kWaves][kAtomRows], s_w[kWaves][kAtomRows];
+  __shared__ double s_F[kWaves][kSfaRun][4];  // of the run: Fr, Fi, then w Fr, w Fi
+  __shared__ double s_rec[kWaves][9];
   const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
   const AtomTable tab = atom_table(s_dyn, a.n_atoms);
   double *s_g = s_dyn + atom_table_doubles(a.n_atoms);
   double *s_f = s_g + 4 * a.n_atoms + wid * 2 * a.n_elem * (kAtomRows + 1);
   double *s_df = s_f + a.n_elem * (kAtomRows + 1);
   stage_atoms(a, tab);
-  for (int i = tid; i < 4 * a.n_atoms; i += kAtomThreads) s_g[i] = 0.0;
+  for (int i = tid; i < 4 * a.n_atoms; i += kWaves * kWave) s_g[i] = 0.0;
   __syncthreads();
   double dr[9];  // lanes below kSfaRun: dL/drec over their rows
 #pragma unroll
   for (int i = 0; i < 9; ++i) dr[i] = 0.0;
   const int end = min(a.n, (static_cast<int>(blockIdx.x) + 1) * rows);
-  for (int r0 = blockIdx.x * rows + wid * kAtomRows; r0 < end; r0 += kAtomWaves * kAtomRows) {
+  for (int r0 = blockIdx.x * rows + wid * kAtomRows; r0 < end; r0 += kWaves * kAtomRows) {
     int4 h = make_int4(0, 0, 0, 0);
     bool anew = true;
     double w = 0.0;
@@ -1187,7 +1197,7 @@ __global__ __launch_bounds__(kAtomThreads, 4) void structure_factor_adjoint_atom
     for (int i = 0; i < 9; ++i) s_rec[wid][i] = dr[i];
   }
   __syncthreads();
-  for (int i = tid; i < a.n_atoms; i += kAtomThreads) {
+  for (int i = tid; i < a.n_atoms; i += kWaves * kWave) {
     const float v[3] = {static_cast<float>(-4.0 * M_PI * s_g[i]),
                         static_cast<float>(-4.0 * M_PI * s_g[a.n_atoms + i]),
                         static_cast<float>(-4.0 * M_PI * s_g[2 * a.n_atoms + i])};
@@ -1199,9 +1209,26 @@ __global__ __launch_bounds__(kAtomThreads, 4) void structure_factor_adjoint_atom
   }
   if (tid < 9) {
     double v = 0.0;
-    for (int ww = 0; ww < kAtomWaves; ++ww) v += s_rec[ww][tid];
+    for (int ww = 0; ww < kWaves; ++ww) v += s_rec[ww][tid];
     if (v != 0.0) unsafeAtomicAdd(&a.drec[tid], v);
   }
+}
+
+// Dynamic LDS of the kernel with this many waves, and whether it fits beside the static part.
+static size_t sfa_atoms_lds(int n_atoms, int n_elem, int waves) {
+  return 8 * (static_cast<size_t>(atom_table_doubles(n_atoms)) + 4 * n_atoms +
+              2 * static_cast<size_t>(waves) * n_elem * (kAtomRows + 1));
+}
+
+static bool sfa_atoms_fit(int n_atoms, int n_elem, int waves) {
+  return sfa_atoms_lds(n_atoms, n_elem, waves) + 712 * static_cast<size_t>(waves) <= 64 * 1024;
+}
+
+template <int kWaves>
+static void launch_sfa_atoms(const SfAdjArgs &a, hipStream_t s) {
+  const int rows = atom_rows_per_block(a.n, kWaves, kSfaAtomRows);
+  hipLaunchKernelGGL(structure_factor_adjoint_atoms_kernel<kWaves>, dim3((a.n + rows - 1) / rows),
+                     dim3(kWaves * kWave), sfa_atoms_lds(a.n_atoms, a.n_elem, kWaves), s, a, rows);
 }
 
 }  // namespace dsx
@@ -1598,11 +1625,12 @@ extern "C" int dsx_structure_factor_adjoint(const int *hkl_d, int n, const doubl
   a.dB = dB_d;
   a.drec = drec_d;
   if (atoms_per_lane_adjoint(n, n_atoms, n_elem)) {
-    const int rows = atom_rows_per_block(n, 512);
-    const size_t lds = 8 * (static_cast<size_t>(atom_table_doubles(n_atoms)) + 4 * n_atoms +
-                            2 * static_cast<size_t>(kAtomWaves) * n_elem * (kAtomRows + 1));
-    hipLaunchKernelGGL(structure_factor_adjoint_atoms_kernel, dim3((n + rows - 1) / rows),
-                       dim3(kAtomThreads), lds, as_stream(stream), a, rows);
+    if (sfa_atoms_fit(n_atoms, n_elem, 16))
+      launch_sfa_atoms<16>(a, as_stream(stream));
+    else if (sfa_atoms_fit(n_atoms, n_elem, 8))
+      launch_sfa_atoms<8>(a, as_stream(stream));
+    else
+      launch_sfa_atoms<4>(a, as_stream(stream));
   } else {
     hipLaunchKernelGGL(structure_factor_adjoint_kernel, dim3((n + kSfaThreads - 1) / kSfaThreads),
                        dim3(kSfaThreads), 0, as_stream(stream), a);

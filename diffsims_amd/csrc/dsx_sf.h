@@ -81,7 +81,7 @@ __device__ __forceinline__ AtomTable atom_table(double *s, int n) {
 
 template <class Args>
 __device__ __forceinline__ void stage_atoms(const Args &a, const AtomTable &t) {
-  for (int i = threadIdx.x; i < a.n_atoms; i += kAtomThreads) {
+  for (int i = threadIdx.x; i < a.n_atoms; i += blockDim.x) {
     const uint4 x = a.xyz_fx[i];
     double sn, cs;
     sincospi(static_cast<double>(static_cast<int32_t>(x.z)) * (2.0 / 4294967296.0), &sn, &cs);
@@ -161,11 +161,12 @@ __device__ __forceinline__ void atom_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
-// Rows per block: enough to pay for the staged turns, few enough to fill the chip.
-static inline int atom_rows_per_block(int n, int most) {
-  const int unit = kAtomRows * kAtomWaves;
-  int rows = (n / 1024 + unit - 1) / unit * unit;
-  return rows < unit ? unit : (rows > most ? most : rows);
+// Rows per block, a whole number of its waves' rows: enough to pay for the staged
+// turns, few enough to fill the chip.
+static inline int atom_rows_per_block(int n, int waves, int least) {
+  const int unit = kAtomRows * waves, most = 512;
+  const int rows = (n / 1024 + unit - 1) / unit * unit;
+  return rows < least ? least : (rows > most ? most : rows);
 }
 
 // Which tables take these kernels.  They cost the same from 1 to 64 atoms, a

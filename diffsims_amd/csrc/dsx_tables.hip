@@ -569,7 +569,7 @@ extern "C" int dsx_structure_factor(const int *hkl_d, int n, const double rec[9]
   a.F2 = F2_d;
   a.F = reinterpret_cast<float2 *>(F_d);
   if (atoms_per_lane(n, n_atoms, n_elem)) {
-    const int rows = atom_rows_per_block(n, 512);
+    const int rows = atom_rows_per_block(n, kAtomWaves, kAtomRows * kAtomWaves);
     const size_t lds = 8 * (static_cast<size_t>(atom_table_doubles(n_atoms)) +
                             static_cast<size_t>(kAtomWaves) * n_elem * (kAtomRows + 1));
     hipLaunchKernelGGL(structure_factor_atoms_kernel, dim3((n + rows - 1) / rows), dim3(kAtomThreads),

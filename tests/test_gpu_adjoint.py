@@ -717,6 +717,61 @@ def test_structure_factor_and_adjoint_of_any_table(n, n_atoms, n_elem, table):
     assert (np.abs(out - gr) <= 2e-6 * gm + 1e-30).all(), (np.abs(out - gr) / (gm + 1e-30)).max()
 
 
+@pytest.mark.parametrize("n_atoms", [48, 200])
+def test_structure_factor_adjoint_sums_few_block_partials(n_atoms):
+    """dL/dxyz and dL/dB of 60,000 rows: blocks of at least 256 rows add their FP32
+    sums to the output.  b partial sums of random sign reach the total M as
+    sqrt(i / b) M, each addition rounds with 2^-24 / sqrt(6) of that, so the error is
+    2^-24 sqrt(b / 12) M; the rows' FP32 phases and factors add some 1.2e-7 M.  A
+    third more is granted, over the mean of four runs (the additions' order
+    varies); blocks of 64 rows come out at twice the first part."""
+    import ctypes
+
+    from diffsims_amd import _lib
+
+    n, n_elem = 60000, 4
+    print(f"structure-factor adjoint: {n} rows {n_atoms} atoms", flush=True)
+    rng = np.random.default_rng(n_atoms)
+    h, l = np.divmod(np.arange(n), 40)
+    hkl = np.stack([h % 41 - 20, h // 41 - 18, 19 - l, 0 * l], 1).astype(np.int32)
+    rec = np.array([[0.05, 0.003, 0.001], [0.0, 0.04, -0.002], [0.0, 0.0, 0.03]])
+    fx = rng.integers(0, 2 ** 32, (n_atoms, 4), dtype=np.uint64).astype(np.uint32)
+    elem = rng.integers(0, n_elem, n_atoms).astype(np.int32)
+    occ = rng.uniform(0.5, 1.0, n_atoms).astype(np.float32)
+    B = rng.uniform(0.2, 2.0, n_atoms).astype(np.float32)
+    co = np.stack([rng.uniform(0.2, 2.0, (n_elem, 5)), rng.uniform(0.5, 8.0, (n_elem, 5))], -1)
+    w = rng.normal(size=n).astype(np.float32)
+    L = _lib.load()
+    dev = lambda v: torch.from_numpy(np.ascontiguousarray(v)).cuda()
+    d_hkl, d_fx, d_el, d_occ, d_B, d_co, d_w = (dev(v) for v in (
+        hkl, fx.view(np.int32), elem, occ, B, co.reshape(n_elem, 10), w))
+    rec9 = (ctypes.c_double * 9)(*rec.reshape(-1).tolist())
+    got = []
+    for _ in range(4):
+        dx, dB = torch.zeros((n_atoms, 3), device="cuda"), torch.zeros(n_atoms, device="cuda")
+        dr = torch.zeros(9, dtype=torch.float64, device="cuda")
+        _lib.check(L.dsx_structure_factor_adjoint(
+            _lib.ptr(d_hkl), n, rec9, _lib.ptr(d_fx), _lib.ptr(d_el), _lib.ptr(d_occ), _lib.ptr(d_B),
+            n_atoms, _lib.ptr(d_co), n_elem, _lib.SCATTER_LOBATO, _lib.ptr(d_w), _lib.ptr(dx),
+            _lib.ptr(dB), _lib.ptr(dr), _lib.stream_handle()), "adjoint")
+        got.append(torch.cat([dx, dB[:, None]], 1).double())
+    H = d_hkl[:, :3].long()
+    g2 = ((H.double() @ dev(rec).T) ** 2).sum(1)
+    f = dev(np.stack([O.atomic_f(g2.cpu().numpy(), c[None], "lobato")[:, 0] for c in co], 1))
+    ref = torch.zeros_like(got[0])
+    for s in (slice(r, r + 10000) for r in range(0, n, 10000)):
+        turn = (H[s, None, :] * dev(fx[:, :3].astype(np.int64))[None]).sum(-1) & 0xffffffff
+        t = f[s][:, d_el.long()] * d_occ.double() * torch.exp(-0.25 * g2[s, None] * d_B.double())
+        t = t * torch.exp(2j * np.pi * (turn.double() / 2.0 ** 32))
+        c = d_w[s, None].double() * t.sum(1).conj()[:, None] * t
+        ref[:, :3] += torch.stack([(-4 * np.pi * H[s, j, None] * c.imag).sum(0) for j in range(3)], 1)
+        ref[:, 3] += (-0.5 * g2[s, None] * c.real).sum(0)
+    tol = 1.33 * np.hypot(2.0 ** -24 * np.sqrt(n / 256 / 12), 1.2e-7)
+    for part in (slice(0, 3), slice(3, 4)):
+        err = [float((v[:, part] - ref[:, part]).norm() / ref[:, part].norm()) for v in got]
+        assert np.mean(err) <= tol, (err, tol)
+
+
 @pytest.mark.parametrize("atoms_of_cell,reps,radius", [(8, 2, 1.5), (4, 2, 1.5), (8, 2, 2.5), (8, 3, 0.7)])
 def test_extinct_reflections_of_large_cells_stay_extinct(atoms_of_cell, reps, radius):
     """Supercells of the diamond and face-centred cell: every reflection that is
