@@ -54,6 +54,9 @@ __device__ __forceinline__ double frcp(double x) {
   return fma(fma(-x, y, 1.0), y, y);
 }
 
+// 1/x where x may have overflowed to infinity.
+__device__ __forceinline__ double frcp_large(double x) { return frcp(fmin(x, 1e300)); }
+
 __device__ __forceinline__ double fdiv(double a, double b) {
   const double y = frcp(b);
   const double q = a * y;
@@ -204,7 +207,7 @@ __device__ __forceinline__ double shape_factor(double s, double r, const Args &a
       return fmax(1.0 - fabs(s) / a.width, 0.0);
     case DSX_SF_LORENTZIAN: {
       const double t = a.sigma * s;
-      return frcp(fma(t, t, 1.0));
+      return frcp_large(fma(t, t, 1.0));
     }
     // the transcendental models take their FP64 argument rounded to FP32
     // (relative error ~1e-7 of the factor)
@@ -280,7 +283,7 @@ __device__ __forceinline__ double shape_factor_grad(double s, double r, const Ar
     }
     case DSX_SF_LORENTZIAN: {
       const double t = a.sigma * s;
-      const double f = frcp(fma(t, t, 1.0));
+      const double f = frcp_large(fma(t, t, 1.0));
       fs = -2.0 * a.sigma * t * f * f;
       return f;
     }

@@ -350,3 +350,21 @@ def test_precession_batch_of_more_orientations_than_one_launch_holds():
     assert not out.ncand[:-1].any() and not out.count[:-1].any()
     assert int(one.ncand) > 0 and int(out.ncand[-1]) == int(one.ncand)
     assert torch.equal(out.spots[-1], one.spots[0])
+
+
+@pytest.mark.parametrize("n", [3, 7000])
+def test_lorentzian_of_a_vanishing_width_is_zero(n):
+    """1 / (1 + (pi s / w)^2) is 0 where the square overflows, for the kernel of few
+    orientations and of many."""
+    from diffsims_amd import engine
+
+    print(f"vanishing width: {n} orientations", flush=True)
+    tab = engine.build_phase_table(P.to_arrays(P.ortho40()), 1.0, False)
+    Rt = engine.rotation_matrices_to_device(rotations(7000, 5)[:n])
+    wide = engine.simulate(tab, Rt, engine.SimSettings(max_excitation_error=0.02), 1.0)
+    b = engine.simulate(tab, Rt, engine.SimSettings(max_excitation_error=0.02, shape_factor_width=1e-160),
+                        1.0, cap=wide.cap)
+    assert torch.equal(b.ncand, wide.ncand) and int(b.count.sum()) > 0
+    assert bool((b.maxI == 0).all())
+    listed = torch.arange(b.cap, device="cuda")[None] < b.count[:, None]
+    assert bool((b.spots[..., 3][listed] == 0).all())
