@@ -1162,6 +1162,12 @@ __global__ __launch_bounds__(kPlanThreads) void render_plan_kernel(BandArgs b) {
 constexpr int kLongThreads = 512;
 constexpr int kLongWaves = kLongThreads / kWave;
 constexpr int kLongLdsBytes = 144 * 1024;  // dynamic; the static part is 12.4 KB
+// Spots of a row that are compared with each other; more of them (zone axes, coarse
+// calibrations) go through the map of the row's pixels.  256 patterns with 10,000
+// spots in all rows / 8 rows / 13 x 13 pixels / one row: 490 / 295 / 217 / 280 us, with
+// comparisons throughout 510 / 1,960 / 1,463 / 13,510 (the windowed renderer: 534 /
+// 495 / 485 / 488).  Limits of 32 and 128 spots measure the same.
+constexpr int kLongRow = 64;
 // Bound units of the largest spot: 2^14 of them (every spot of the longest
 // list on one tile) stay below 2^31.
 constexpr float kLongUnits = 65536.0f;
@@ -1268,7 +1274,7 @@ __global__ __launch_bounds__(kLongThreads) void render_plan_long_kernel(BandArgs
   __shared__ float s_tp[kR + 1];
   __shared__ float s_pm[kLongWaves];
   __shared__ int s_n[kLongWaves], s_u[kLongWaves];
-  __shared__ int s_q, s_best, s_odd;
+  __shared__ int s_q, s_best, s_odd, s_most;
   const RenderArgs &a = b.r;
   constexpr int R = kR;
   const int tid = threadIdx.x, lane = lane_id(), wid = tid / kWave;
@@ -1304,11 +1310,15 @@ __global__ __launch_bounds__(kLongThreads) void render_plan_long_kernel(BandArgs
     int sum = 0;
     for (int t = i0; t < i1; ++t) sum += rows[1 + t];
     int run = wave_inclusive_scan(sum) - sum;
+    int most = 0;
     for (int t = i0; t < i1; ++t) {
       const int c = rows[1 + t];
       rows[1 + t] = run;
       run += c;
+      most = max(most, c);
     }
+    most = wave_max_i(most);
+    if (lane == 0) s_most = most;
   }
   lds_sync();
   for (int j = tid; j < n; j += kLongThreads) {  // ... and its end, the start of row y + 1
@@ -1324,15 +1334,40 @@ __global__ __launch_bounds__(kLongThreads) void render_plan_long_kernel(BandArgs
   lds_sync();
   const int total = rows[H];
   // ---- last write wins: a spot yields to a later one on its pixel ----------
+  // rows of many spots: the latest spot of every pixel, kTile^2 pixels at a time
+  const bool map_rows = s_most > kLongRow;  // uniform
+  for (int y = map_rows ? wid : H; y < H; y += kLongWaves) {
+    const int r0 = rows[y], r1 = rows[y + 1];
+    if (r1 - r0 <= kLongRow) continue;
+    for (int x0 = 0; x0 < W; x0 += kTile * kTile) {
+      int *owner = s_tile[wid];
+#pragma unroll
+      for (int u = 0; u < kTile * kTile / kWave; ++u) owner[lane + u * kWave] = -1;
+      wave_lds_sync();
+      for (int e = r0 + lane; e < r1; e += kWave) {
+        const int k = s_key[e], x = (k >> 16) - x0;
+        if (x >= 0 && x < kTile * kTile) atomicMax(&owner[x], k);
+      }
+      wave_lds_sync();
+      for (int e = r0 + lane; e < r1; e += kWave) {
+        const int k = s_key[e], x = (k >> 16) - x0;
+        if (x >= 0 && x < kTile * kTile && owner[x] != k) s_I[e] = 0.0f;
+      }
+      wave_lds_sync();
+    }
+  }
+  if (map_rows) lds_sync();
   float pm = 0.0f;
   int mine = 0;
   for (int e = tid; e < total; e += kLongThreads) {
     const int k = s_key[e], yi = s_y[e];
-    bool lose = false;
-    for (int o = rows[yi]; o < rows[yi + 1]; ++o) {
-      const int ko = s_key[o];
-      lose |= (ko >> 16) == (k >> 16) && ko > k;
-    }
+    const int r0 = rows[yi], r1 = rows[yi + 1];
+    bool lose = map_rows && s_I[e] == 0.0f;  // a zero adds nothing either way
+    if (!map_rows || r1 - r0 <= kLongRow)
+      for (int o = r0; o < r1; ++o) {
+        const int ko = s_key[o];
+        lose |= (ko >> 16) == (k >> 16) && ko > k;
+      }
     if (lose) {
       s_I[e] = 0.0f;  // contributes nothing
     } else {
@@ -1556,7 +1591,7 @@ __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
       const int2 en = s_ent[q];
       const int yi = en.x >> 16, xi = en.x & 0xffff;
       const int x = xi - R + c;
-      if (x < 0 || x >= W) continue;
+      if (x < 0 || x >= W || (kLong && en.y == 0)) continue;  // (hidden spots are zeros)
       // render_kernel's splat terms: ((I wx) scale) wy, truncated
       const float wx = (xi >= R && xi + R < W) ? s_tp[c > R ? c - R : R - c]
                                                : reflect_weight3(x, xi, W, R, s_tp);

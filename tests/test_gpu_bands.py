@@ -460,3 +460,33 @@ def test_short_lists_of_any_intensity_equal_the_splat_renderer(shape):
     ref, out, st_ref, st, _ = _render_both(spots, cnt, 96, shape, 1.0)
     assert torch.equal(st_ref, st)
     assert torch.equal(out.view(torch.int32), ref.view(torch.int32))
+
+
+@pytest.mark.parametrize("shape", [(130, 600), (200, 255)])
+@pytest.mark.parametrize("length", [63, 64, 65, 128, 700])
+def test_long_lists_gathered_in_a_few_rows(shape, length):
+    """Rows of `length` spots, many of them on the same pixels, either side of the
+    length from which a row's pixels are mapped (64) and over several parts of the
+    map (256 pixels): the latest spot of a pixel is the one that is seen, a zero
+    too.  At most 9 x 1 spots reach a pixel, well inside LONG_TOL's count."""
+    import torch
+    print(f"long lists in rows: {shape}, {length} spots each", flush=True)
+    H, W = shape
+    rng = np.random.default_rng(length)
+    ys = np.arange(4, H, 12)
+    m = len(ys) * length
+    sp = np.zeros((3, max(m, 1100), 4), np.float32)
+    for i in range(3):
+        order = rng.permutation(m)
+        y = np.repeat(ys, length)[order]
+        # the second pattern's rows take few columns, the third's lie at the end
+        x = rng.integers(0, W, m) if i == 0 else rng.integers(0, 20, m) if i == 1 else rng.integers(W - 9, W, m)
+        sp[i, :m, 0] = x + 0.5 - W // 2
+        sp[i, :m, 1] = y + 0.5 - H // 2
+        sp[i, :m, 3] = rng.lognormal(0.0, 1.5, m)
+        sp[i, :m:7, 3] = 0.0
+    spots = torch.from_numpy(sp).cuda()
+    cnt = torch.full((3,), m, dtype=torch.int32, device="cuda")
+    out = _render_long(spots, cnt, spots.shape[1], shape, 1.0).cpu().numpy()
+    for o, r in zip(out, _fp64_patterns(spots, cnt, shape, 1.0, True, range(3))):
+        assert np.abs(o - r).max() <= LONG_TOL
