@@ -67,12 +67,29 @@ def fast_renderer(n: int, height: int, width: int) -> str:
     return "dsx_render_fast_bands"
 
 
+# Fast rendering of long lists (more than dsx_render_max_spots() spots): the plan
+# and band writer (dsx_render_fast_long) cost in proportion to the spots, the
+# windowed renderer (dsx_render_fast_large) to the pixels.  Time of the former
+# over the latter, 1 to 1,500 patterns with taps of radius 1 to 8, lists filled to
+# 60-80 % with |F|^2 of random structures: 0.1-0.5 at a capacity of one spot per
+# 12 pixels; at 1 per 8 0.3-1.0 (129 x 128, 170 x 171) and 0.2-0.8 (256 x 256,
+# 301 x 203); at 1 per 6.7 0.3-1.26 and 0.25-1.0; at 1 per 4 0.6-2.0 and more.
+# (Lists of equal intensities, whose maximum can be anywhere, come out level at
+# 1 per 12 and 1.2-1.9 times slower at 1 per 6.7.)
+LONG_PIXELS_PER_SPOT = 6
+LONG_PIXELS_PER_SPOT_SMALL = 8      # below LONG_SMALL_PIXELS pixels
+LONG_SMALL_PIXELS = 32768
+
+
 def long_renderer(cap: int, height: int, width: int, radius: int) -> bool:
     """Whether ``render_spots`` renders fast lists of more than
     dsx_render_max_spots() spots with dsx_render_fast_long: patterns too large
-    for the dense renderers' LDS, as far as the lists fit its plan."""
+    for the dense renderers' LDS, as far as the lists are sparse enough and fit
+    its plan."""
     L = _lib.load()
-    return (height * width > int(L.dsx_render_dense_max_pixels())
+    pixels = int(height) * int(width)
+    least = LONG_PIXELS_PER_SPOT_SMALL if pixels < LONG_SMALL_PIXELS else LONG_PIXELS_PER_SPOT
+    return (pixels > int(L.dsx_render_dense_max_pixels()) and least * int(cap) <= pixels
             and bool(L.dsx_render_fast_long_fits(int(cap), int(radius), int(height), int(width))))
 
 

@@ -362,6 +362,9 @@ def test_long_lists_dispatch_and_limits():
     assert engine.long_renderer(2000, 256, 256, 4)
     assert not engine.long_renderer(2000, 128, 128, 4)   # the dense renderers
     assert not engine.long_renderer(30000, 256, 256, 4)  # dsx_render_fast_large
+    # dense lists stay with it: a spot per 6 pixels, per 8 of small patterns
+    assert engine.long_renderer(10922, 256, 256, 4) and not engine.long_renderer(10923, 256, 256, 4)
+    assert engine.long_renderer(2064, 129, 128, 8) and not engine.long_renderer(2065, 129, 128, 8)
     # render_spots on both sides of the lists it takes: the same pixels
     spots, cnt = _spot_lists(6, 1500, 200, 160, 1400, seed=2)
     a = engine.render_spots(spots, cnt, 1500, (200, 160), 1.0, 1.0)
@@ -490,3 +493,18 @@ def test_long_lists_gathered_in_a_few_rows(shape, length):
     out = _render_long(spots, cnt, spots.shape[1], shape, 1.0).cpu().numpy()
     for o, r in zip(out, _fp64_patterns(spots, cnt, shape, 1.0, True, range(3))):
         assert np.abs(o - r).max() <= LONG_TOL
+
+
+@pytest.mark.parametrize("shape,cap", [((129, 128), 2064), ((200, 164), 5466)])
+def test_both_sides_of_the_density_line_give_the_same_pixels(shape, cap):
+    # one list either side of the capacity from which the windowed renderer takes it
+    import torch
+    from diffsims_amd import engine
+    print(f"long lists: {shape}, capacity {cap}", flush=True)
+    spots, cnt = _spot_lists(4, cap, *shape, 1300, seed=cap)
+    assert engine.long_renderer(cap, *shape, 4) and not engine.long_renderer(cap + 1, *shape, 4)
+    a = engine.render_spots(spots, cnt, cap, shape, 1.0, 1.0)
+    wide = torch.zeros((4, cap + 1, 4), dtype=torch.float32, device="cuda")
+    wide[:, :cap] = spots
+    b = engine.render_spots(wide, cnt, cap + 1, shape, 1.0, 1.0)
+    assert float((a - b).abs().max()) <= 2 * LONG_TOL
