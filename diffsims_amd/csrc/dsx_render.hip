@@ -790,6 +790,7 @@ struct BandArgs {
   int rec_ints;     // stride of rec
   int p0, m;        // first pattern of the round, patterns in it
   int band_rows, nb;
+  bool wide;        // kBandWide stores per thread (band_wide)
   int ntx, n_tiles;
   int wave_ints;    // LDS words of one plan wave
 };
@@ -1501,18 +1502,11 @@ __global__ __launch_bounds__(kLongThreads) void render_plan_long_kernel(BandArgs
     ent[e] = make_int2((static_cast<int>(s_y[e]) << 16) | (s_key[e] >> 16), __float_as_int(s_I[e]));
 }
 
-// Pixels per band: 2,048 (two 16-byte stores per thread) up to R = 5, 4,096
-// for wider taps.  A band of B rows splats the spots of B + 2R rows, so wide
-// taps make the splat's VALU work, not the stores, bound small bands.
-// Render stage of 12,000 x 232 x 200, 235 spots each, with 2,048 / 4,096
-// pixels: R = 4 402 / 461 us, R = 5 458 / 468, R = 6 589 / 472, R = 7
-// 672 / 533, R = 8 782 / 618.
-__host__ __device__ constexpr int band_vec(int R, bool long_lists = false) {
-  return R <= 5 && !long_lists ? 2 : 4;
-}
-__host__ __device__ constexpr int band_pix(int R, bool long_lists = false) {
-  return 4 * band_vec(R, long_lists) * kBandThreads;
-}
+// Pixels per band: 2,048 (two 16-byte stores per thread) or 4,096.  A band of B
+// rows splats the spots of B + 2R rows, so with wide taps and many spots the
+// splat's VALU work, not the stores, bounds narrow bands: band_wide.
+constexpr int kBandNarrow = 2, kBandWide = 4;  // 16-byte stores per thread
+__host__ __device__ constexpr int band_pix(int vec) { return 4 * vec * kBandThreads; }
 
 // kAligned: every row is a whole number of 16-byte vectors.  Otherwise the
 // band's pixels sit in LDS at the offset their first pixel has within its
@@ -1523,9 +1517,9 @@ __host__ __device__ constexpr int band_pix(int R, bool long_lists = false) {
 // 730 us there; 62 us plan and 425 us writer here, 5.3 TB/s).
 // kLong: lists of any length (render_plan_long_kernel), whose window passes
 // through LDS kPlanMax spots at a time.
-template <int kR, bool kAligned, bool kLong = false>
+template <int kR, bool kAligned, int kVec, bool kLong = false>
 __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
-  constexpr int kVec = band_vec(kR, kLong), kPix = band_pix(kR, kLong);
+  constexpr int kPix = band_pix(kVec);
   // how the rows outside the band are dropped, as measured (render stage, us,
   // row tests / flat index): 16,000 x 256 x 256 with R = 2 667 / 666, R = 4
   // 660 / 646, R = 5 729 / 698, R = 6 701 / 731, R = 7 732 / 710 (231 x 201:
@@ -2510,9 +2504,22 @@ static int render_common(int mode, const float *spot_d, const int *count_d, int 
 
 // ---- band renderer: host side ----------------------------------------------
 
-static void band_shape(int R, int H, int W, int &band_rows, int &nb, bool long_lists = false) {
-  band_rows = std::max(1, std::min(H, band_pix(R, long_lists) / std::max(1, W)));
+static void band_shape(int vec, int H, int W, int &band_rows, int &nb) {
+  band_rows = std::max(1, std::min(H, band_pix(vec) / std::max(1, W)));
   nb = (H + band_rows - 1) / band_rows;
+}
+
+// Wide bands: taps from radius 6 on, more than two of them to a pattern, and a
+// list of at least one spot per 133 pixels.  Time with narrow bands over wide
+// ones, 300 to 12,000 patterns, R = 6 to 8: 512 x 512 with lists of 0.6 to 2.2
+// spots per 1,000 pixels 0.85-1.0, 300 x 256 at 3.2 0.79-1.0, 144 x 145 at 7.3
+// 0.82-1.0, 300 x 256 at 7.7 0.91-1.22, 64 x 1,021 at 9 1.2-1.5, 232 x 200 at 12.7
+// 1.1-1.28 and at 20 1.07-1.27, 64 x 65 0.84-1.0 at any.  Up to R = 5 narrow bands
+// are as fast (12,000 x 232 x 200, 235 spots: R = 4 402 against 461 us).
+constexpr int kWideTaps = 6;
+static bool band_wide(int R, int cap, int H, int W) {
+  const long long pixels = static_cast<long long>(H) * W;
+  return R >= kWideTaps && pixels > 2 * band_pix(kBandWide) && 133ll * cap >= pixels;
 }
 
 // Shapes the plan and the band writer take: tap radius 1..8 below both
@@ -2531,7 +2538,7 @@ static int band_rec_ints(int nb) { return (4 + 2 * nb + 3) & ~3; }
 // rounds) | per pattern of a round: header and each band's window | row-sorted spots.
 static long long band_workspace_ints(int n, int H, int W) {
   int br, nb;
-  band_shape(1, H, W, br, nb);  // the narrowest bands
+  band_shape(kBandNarrow, H, W, br, nb);
   const long long chunk = std::min(std::max(n, 1), kBandChunk);
   return band_list_ints(std::max(n, 1)) + chunk * band_rec_ints(nb) + chunk * kPlanMax * 2;
 }
@@ -2547,7 +2554,7 @@ static int long_chunk(int cap, int n) {
 
 static long long long_workspace_ints(int cap, int n, int H, int W) {
   int br, nb;
-  band_shape(1, H, W, br, nb, true);
+  band_shape(kBandWide, H, W, br, nb);
   const long long chunk = long_chunk(cap, n);
   return chunk * band_rec_ints(nb) + chunk * cap * 2;
 }
@@ -2575,9 +2582,9 @@ static int launch_long_r(const BandArgs &b, size_t lds, hipStream_t st) {
   hipLaunchKernelGGL(render_plan_long_kernel<kR>, dim3(b.m), dim3(kLongThreads), lds, st, b);
   const unsigned blocks = static_cast<unsigned>((b.m + 7) / 8) * 8u * static_cast<unsigned>(b.nb);
   if ((b.r.W & 3) == 0 && (reinterpret_cast<uintptr_t>(b.r.out) & 15) == 0)
-    hipLaunchKernelGGL((render_band_kernel<kR, true, true>), dim3(blocks), dim3(kBandThreads), 0, st, b);
+    hipLaunchKernelGGL((render_band_kernel<kR, true, kBandWide, true>), dim3(blocks), dim3(kBandThreads), 0, st, b);
   else
-    hipLaunchKernelGGL((render_band_kernel<kR, false, true>), dim3(blocks), dim3(kBandThreads), 0, st, b);
+    hipLaunchKernelGGL((render_band_kernel<kR, false, kBandWide, true>), dim3(blocks), dim3(kBandThreads), 0, st, b);
   return DSX_OK;
 }
 
@@ -2590,10 +2597,16 @@ static void launch_bands_r(const BandArgs &b, size_t plan_lds, hipStream_t st) {
   const int plan_blocks = (b.m + 8 * kPlanWaves - 1) / (8 * kPlanWaves) * 8;
   hipLaunchKernelGGL(render_plan_kernel<kR>, dim3(plan_blocks), dim3(kPlanThreads), plan_lds, st, b);
   const unsigned band_blocks = static_cast<unsigned>((b.m + 7) / 8) * 8u * static_cast<unsigned>(b.nb);
-  if ((b.r.W & 3) == 0 && (reinterpret_cast<uintptr_t>(b.r.out) & 15) == 0)
-    hipLaunchKernelGGL((render_band_kernel<kR, true>), dim3(band_blocks), dim3(kBandThreads), 0, st, b);
+  const bool aligned = (b.r.W & 3) == 0 && (reinterpret_cast<uintptr_t>(b.r.out) & 15) == 0;
+  constexpr int kWide = kR >= kWideTaps ? kBandWide : kBandNarrow;
+  if (b.wide && aligned)
+    hipLaunchKernelGGL((render_band_kernel<kR, true, kWide>), dim3(band_blocks), dim3(kBandThreads), 0, st, b);
+  else if (b.wide)
+    hipLaunchKernelGGL((render_band_kernel<kR, false, kWide>), dim3(band_blocks), dim3(kBandThreads), 0, st, b);
+  else if (aligned)
+    hipLaunchKernelGGL((render_band_kernel<kR, true, kBandNarrow>), dim3(band_blocks), dim3(kBandThreads), 0, st, b);
   else
-    hipLaunchKernelGGL((render_band_kernel<kR, false>), dim3(band_blocks), dim3(kBandThreads), 0, st, b);
+    hipLaunchKernelGGL((render_band_kernel<kR, false, kBandNarrow>), dim3(band_blocks), dim3(kBandThreads), 0, st, b);
 }
 
 }  // namespace dsx
@@ -2688,7 +2701,8 @@ extern "C" int dsx_render_fast_bands(const float *spot_d, const int *count_d, in
   }
   BandArgs b;
   b.r = a;
-  band_shape(a.R, a.H, a.W, b.band_rows, b.nb);
+  b.wide = band_wide(a.R, cap, a.H, a.W);
+  band_shape(b.wide ? kBandWide : kBandNarrow, a.H, a.W, b.band_rows, b.nb);
   b.ntx = (a.W + kTile - 1) / kTile;
   b.n_tiles = b.ntx * ((a.H + kTile - 1) / kTile);
   b.wave_ints = plan_wave_ints(a.H, b.n_tiles);
@@ -2767,7 +2781,7 @@ extern "C" int dsx_render_fast_long(const float *spot_d, const int *count_d, int
   a.n = n;
   a.out = out_d;
   a.status = status_d;
-  band_shape(a.R, a.H, a.W, b.band_rows, b.nb, true);
+  band_shape(kBandWide, a.H, a.W, b.band_rows, b.nb);
   b.ntx = (a.W + kTile - 1) / kTile;
   b.n_tiles = b.ntx * ((a.H + kTile - 1) / kTile);
   b.wave_ints = 0;

@@ -508,3 +508,14 @@ def test_both_sides_of_the_density_line_give_the_same_pixels(shape, cap):
     wide[:, :cap] = spots
     b = engine.render_spots(wide, cnt, cap + 1, shape, 1.0, 1.0)
     assert float((a - b).abs().max()) <= 2 * LONG_TOL
+
+
+@pytest.mark.parametrize("shape,sigma,cap", [
+    ((101, 100), 1.75, 75), ((101, 100), 1.75, 76), ((101, 99), 2.0, 75), ((101, 99), 1.5, 76),
+    ((64, 128), 1.5, 96), ((82, 100), 1.5, 96), ((300, 257), 1.75, 579), ((300, 257), 1.75, 580)])
+def test_narrow_and_wide_bands_give_the_same_bits(shape, sigma, cap):
+    # either side of one spot per 133 pixels and of two wide bands, from radius 6 on
+    print(f"bands: {shape}, sigma {sigma}, capacity {cap}", flush=True)
+    spots, cnt = _spot_lists(50, cap, *shape, 0.7 * cap, seed=cap, edge=0.2, dup=0.05, R=8)
+    ref, out, st_ref, st, _ = _render_both(spots, cnt, cap, shape, sigma)
+    _assert_same(ref, out, st_ref, st)
