@@ -58,11 +58,39 @@ SPLAT_MAX_PATTERNS = 768
 SPLAT_MAX_PIXELS = 256 * 256
 
 
-def fast_renderer(n: int, height: int, width: int) -> str:
+# Widths that are not a multiple of 4: the band writer's plan lists patterns
+# whose maximum could be in many tiles for the splat kernel, which then runs
+# behind the writer with most of the GPU idle.  Time with bands over the splat
+# kernel, lists of 65, 146 and 259 spots of the 40-atom cell: 300 patterns 1.05-2.0
+# at any size up to 300 x 257, 800 and more 0.5-0.95 (231 x 201, 300 x 257); taps of
+# radius 7 and 8 on 65 x 67, 101 x 99 and 144 x 145: 800 patterns 1.0-1.6, 1,500
+# 0.9-1.4, from 2,500 on 0.5-0.9 unless a list holds a spot per 8 pixels (65 x 67:
+# 1.2-1.3 at any number); 64 x 1,021 1.3-1.5 up to 1,500.
+ODD_MIN_PATTERNS_WIDE_TAPS = 1536
+ODD_SMALL_PIXELS = 24000
+
+
+def _splat_pays_at_odd_width(n: int, height: int, width: int, cap: int, radius: int) -> bool:
+    if n < SPLAT_MAX_PATTERNS:
+        return True
+    if radius < 6:
+        return False
+    if min(height, width) <= 10 * radius:
+        return n < 2000 or 8 * cap >= height * width
+    return n < ODD_MIN_PATTERNS_WIDE_TAPS and height * width <= ODD_SMALL_PIXELS
+
+
+def fast_renderer(n: int, height: int, width: int, cap: Optional[int] = None,
+                  radius: Optional[int] = None) -> str:
     """Which entry point ``render_spots`` uses for ``n`` fast patterns of at
     most dsx_render_max_spots() spots: "dsx_render_fast" or
-    "dsx_render_fast_bands" (the same output bit for bit)."""
+    "dsx_render_fast_bands" (the same output bit for bit).  With the lists'
+    capacity and the taps' radius the choice is also made for widths that are
+    not a multiple of 4."""
     if n < SPLAT_MAX_PATTERNS and height * width <= SPLAT_MAX_PIXELS:
+        return "dsx_render_fast"
+    if width % 4 and cap is not None and radius is not None and _splat_pays_at_odd_width(
+            n, height, width, cap, radius):
         return "dsx_render_fast"
     return "dsx_render_fast_bands"
 
@@ -579,7 +607,7 @@ def render_spots(spots: torch.Tensor, count: torch.Tensor, cap: int, shape, sigm
             _lib.check(L.dsx_render_fast_large(
                 _lib.ptr(spots), _lib.ptr(count), cap, n, ctypes.byref(p), _lib.ptr(work),
                 work.numel(), _lib.ptr(out), _lib.ptr(status), stream), "dsx_render_fast_large")
-    elif fast and fast_renderer(n, H, W) == "dsx_render_fast":
+    elif fast and fast_renderer(n, H, W, cap, p.radius) == "dsx_render_fast":
         _lib.check(L.dsx_render_fast(_lib.ptr(spots), _lib.ptr(count), cap, n, ctypes.byref(p),
                                      _lib.ptr(out), _lib.ptr(status), stream), "dsx_render_fast")
     elif fast:

@@ -315,6 +315,21 @@ def test_fast_renderer_choice():
     assert fast_renderer(10, 256, 257) == "dsx_render_fast_bands"
 
 
+@pytest.mark.parametrize("n,shape,cap,radius,bands", [
+    (767, (300, 257), 292, 4, False), (768, (300, 257), 292, 4, True),     # few patterns
+    (767, (300, 256), 292, 4, True),                                       # whole 16-byte rows
+    (768, (101, 99), 292, 5, True), (1535, (101, 99), 292, 6, False),      # wide taps, small patterns
+    (1536, (101, 99), 292, 6, True), (768, (231, 201), 292, 8, True),
+    (1999, (1021, 67), 400, 8, False), (2000, (1021, 67), 400, 8, True),   # narrow patterns
+    (12000, (65, 67), 544, 7, True), (12000, (65, 67), 545, 7, False),     # a spot per 8 pixels
+])
+def test_fast_renderer_choice_at_odd_widths(n, shape, cap, radius, bands):
+    from diffsims_amd.engine import fast_renderer
+
+    assert fast_renderer(n, *shape, cap, radius) == ("dsx_render_fast_bands" if bands else "dsx_render_fast")
+
+
+
 # -- bench contract ---------------------------------------------------------------
 
 def test_bench_refuses_more_than_one_gpu():
