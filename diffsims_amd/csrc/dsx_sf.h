@@ -169,32 +169,41 @@ static inline int atom_rows_per_block(int n, int waves, int least) {
   return rows < least ? least : (rows > most ? most : rows);
 }
 
-// Which tables take these kernels.  They cost the same from 1 to 64 atoms, a
-// thread per reflection costs in proportion to the atoms but needs many rows to
-// fill the chip.  Measured in us, thread per reflection | atom per lane:
-//   rows        24 atoms    32         48         64         100          500
-//   1,563,972   115 | 230   145 | 230  182 | 230  229 | 228  -            1225 | 930   forward
-//               568 | 549   568 | 538  592 | 557  727 | 560  -            4393 | 2560  adjoint
-//   195,590     21 | 38     26 | 39    32 | 39    39 | 39                              forward
-//               104 | 126   120 | 129  139 | 131  160 | 129                            adjoint
-//   58,076      15 | 17     18 | 17    23 | 17    28 | 18    40 | 23                   forward
-//               58 | 83     67 | 83    85 | 83    104 | 84   151 | 88                  adjoint
-//   17,332      14 | 11     18 | 11    22 | 11    28 | 11                              forward
-//               44 | 36     55 | 37    72 | 37    91 | 37                              adjoint
-//   4,614       14 | 10     17 | 9     21 | 9     27 | 9     38 | 12                   forward
-//               42 | 20     53 | 20    70 | 20    89 | 20    136 | 25                  adjoint
-// (at 17,332 rows of 16 atoms both take 10 forward and 31 adjoint).
+// Which tables take these kernels.  A lane per atom costs a pass per 64 atoms,
+// full or not, a thread per reflection costs in proportion to the atoms but needs
+// many rows to fill the chip.  Measured in us, thread per reflection | atom per
+// lane (lines of 17 to 40 rows, 4 elements):
+//   rows       24 atoms   32        48        64        65        80        100
+//   1,000,000  55 | 128   65 | 128  87 | 127  108 | 128 107 | 179 128 | 178 156 | 178
+//              341 | 341  376 | 341 390 | 341 427 | 341 440 | 482 496 | 481 606 | 480
+//   400,000    27 | 64    32 | 64   43 | 64   53 | 64   53 | 89   63 | 89   76 | 89
+//              159 | 174  178 | 175 200 | 176 232 | 177 215 | 244 251 | 245 299 | 246
+//   195,590    15 | 30    18 | 30   24 | 30   30 | 30   30 | 41   36 | 41   43 | 41
+//              95 | 92    106 | 92  124 | 92  147 | 94  147 | 118 167 | 119 196 | 119
+//   100,000    12 | 21    15 | 21   20 | 21   25 | 21   25 | 28   30 | 28   36 | 28
+//              62 | 64    70 | 64   88 | 65   105 | 65 106 | 82  122 | 82  144 | 82
+//   58,076     11 | 12    13 | 12   18 | 12   22 | 12   22 | 16   26 | 16   32 | 16
+//              50 | 40    59 | 40   76 | 40   94 | 40   95 | 49   112 | 50  133 | 49
+//   17,332     11 | 8     13 | 8    17 | 8    22 | 8    22 | 12   26 | 12   31 | 12
+//              38 | 28    47 | 28   65 | 28   82 | 28   83 | 37   100 | 37  122 | 37
+//   4,614      10 | 7     12 | 7    17 | 7    21 | 7    22 | 9    26 | 9    31 | 9
+//              35 | 25    44 | 25   62 | 25   80 | 25   81 | 34   98 | 34   120 | 34
+// (first line forward, second adjoint; at 400,000 rows forward 129 atoms 96 | 113,
+// 160 116 | 114, 193 138 | 138, 500 346 | 240, at 195,590 96 atoms 41 | 41 and 129
+// 53 | 52; adjoint 129 atoms 375 | 319 and 500 1,398 | 634.)
 static inline bool atoms_fit(int n_atoms, int n_elem) {
   return n_atoms <= kAtomMax && n_elem >= 1 && n_elem <= kAtomElems;
 }
 
 static inline bool atoms_per_lane(int n, int n_atoms, int n_elem) {
-  const bool few_rows = n <= 24 * 1024 ? n_atoms >= 24 : (n <= 64 * 1024 && n_atoms >= 32);
-  return atoms_fit(n_atoms, n_elem) && (n_atoms > kWave || few_rows);
+  const int least = n <= 24 * 1024 ? 24 : n <= 64 * 1024 ? 32 : n <= 128 * 1024 ? 76 : n <= 256 * 1024 ? 96 : 160;
+  return atoms_fit(n_atoms, n_elem) && n_atoms >= least;
 }
 
 static inline bool atoms_per_lane_adjoint(int n, int n_atoms, int n_elem) {
-  return atoms_fit(n_atoms, n_elem) && (n_atoms >= 48 || (n_atoms >= 24 && n <= 24 * 1024));
+  const int passes = (n_atoms + kWave - 1) / kWave;
+  const int least = n <= 64 * 1024 ? 24 : n <= 256 * 1024 ? 32 : 40 * passes;
+  return atoms_fit(n_atoms, n_elem) && n_atoms >= least;
 }
 
 }  // namespace dsx

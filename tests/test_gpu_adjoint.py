@@ -612,12 +612,15 @@ def test_more_tile_entries_than_are_numbered_are_refused():
 
 
 # rows, atoms, elements, table: either side of the lines between the kernels with
-# a thread per reflection and a lane per atom (23/24, 47/48, 64/65 and 512/513
-# atoms, 20/21 elements, 24,576 and 65,536 rows), and row counts around a wave's 16
+# a thread per reflection and a lane per atom (24 to 160 atoms by the rows, 512/513
+# atoms, 20/21 elements), and row counts around a wave's 16
 SF_SIZES = [(1, 24, 3, "lobato"), (15, 23, 3, "lobato"), (17, 48, 20, "xtables"), (64, 64, 1, None),
             (65, 65, 2, "lobato"), (999, 47, 20, "lobato"), (1000, 100, 21, "xtables"),
             (1003, 512, 20, "lobato"), (700, 513, 5, "lobato"), (24577, 24, 2, "lobato"),
-            (24576, 30, 2, None), (65537, 33, 1, "lobato"), (65536, 32, 1, "lobato"), (33000, 130, 4, "xtables")]
+            (24576, 30, 2, None), (65537, 33, 1, "lobato"), (65536, 32, 1, "lobato"), (33000, 130, 4, "xtables"),
+            (65537, 31, 2, "lobato"), (70001, 75, 2, "lobato"), (70001, 76, 2, "lobato"),
+            (131073, 95, 3, "xtables"), (131073, 96, 3, "xtables"), (262145, 159, 2, "lobato"),
+            (262145, 160, 2, "lobato"), (262145, 79, 2, "lobato"), (262145, 80, 2, "lobato")]
 
 
 @pytest.mark.parametrize("n,n_atoms,n_elem,table", SF_SIZES)
