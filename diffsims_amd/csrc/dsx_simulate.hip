@@ -757,10 +757,25 @@ __global__ __launch_bounds__(kCoopWaves *kWave, 4) void simulate_coop_kernel(Sim
 //   24-atom cell, full sweep of 4,614 rows  512: 11 (8) 29 (1) 45   2,048: 23
 //     (2) 31 (1) 45   4,096: 40 (1) 48   8,192: 76 (1) 52
 //   256 rows  500: 12 (8) 9 (2) 11   4,000: 10 (1) 11   20,000: 21 (1) 16
-// Under precession with long line lists one wave stays ahead (the per-row
-// threshold saves a quarter of the candidates): 20,000 14,622 (1) 20,271.
-static int coop_waves(int n_orient, int n_refl, int n_lines, bool precession) {
-  const int limit = n_lines >= 2048 ? (precession ? 1 << 30 : 16384) : 6144;
+// How many orientations a wave each stays ahead for, time over the wave per
+// four, non-precessed tables of 282 to 7,798 lines: it repeats the work per line
+// that the other shares, so it depends on the candidates per line, c = rows per
+// line (1.5 max_excitation_error / g_max + sin phi).  They cross at 4,600 to 5,000
+// orientations for c <= 0.12, 5,200-6,200 at 0.16, 6,500 at 0.22, 7,800-8,700 at
+// 0.32, 10,500 at 0.46, 11,300-12,000 at 0.54-0.66 and 12,500-14,000 above; 16,384
+// take 1.7-1.9 times as long at 0.12 and 1.1 at 1.  Where precession gives most
+// of the candidates (rows per line times sin phi of 0.3 and more) the per-row
+// threshold saves a quarter of them and one wave is ahead at any number (20,000:
+// 0.66-0.91; 500-atom cell 14,622 us against 20,271).  The full sweep shares each row:
+// they cross at 3,900-4,200 with 6,212 to 28,800 rows, at 5,000-6,100 with 484.
+static int coop_waves(int n_orient, int n_refl, int n_lines, double me, double g_max, double sin_phi) {
+  double limit = n_refl < 1024 ? 5120 : 4096;
+  if (n_lines > 0) {
+    const double rows = static_cast<double>(n_refl) / n_lines;
+    const double c = g_max > 0.0 ? rows * (1.5 * me / g_max + sin_phi) : 0.0;
+    limit = rows * sin_phi >= 0.3 ? 1e10 : std::min(std::max(3000.0 + 15500.0 * c, 4500.0), 12288.0);
+    if (n_lines < 2048) limit = std::min(limit, 6144.0);
+  }
   if (n_orient > limit) return 0;
   int w = n_orient <= 512 ? 8 : (n_orient <= 1280 ? 4 : (n_orient <= 2560 ? 2 : 1));
   while (w > 1 && n_refl < w * 2 * kWave) w /= 2;  // at least two rows per lane
@@ -879,7 +894,8 @@ extern "C" int dsx_simulate(const int *hkl_d, const float *g4_d, const float *F2
   // dominates, and the line state would cost it occupancy
   const bool avg = p->shape_model >= DSX_SF_PRECESSION_AVG;
   const bool use_lines = lines_d && !avg && lines_pay(n_refl, n_lines);
-  const int coop = avg ? 0 : coop_waves(n_orient, n_refl, use_lines ? n_lines : 0, a.precession != 0);
+  const int coop = avg ? 0 : coop_waves(n_orient, n_refl, use_lines ? n_lines : 0, p->max_excitation_error,
+                                        p->g_max, a.precession ? a.sin_phi : 0.0);
   if (coop > 0) {
     if (use_lines)
       launch_coop<true>(coop, a, s);

@@ -368,3 +368,24 @@ def test_lorentzian_of_a_vanishing_width_is_zero(n):
     assert bool((b.maxI == 0).all())
     listed = torch.arange(b.cap, device="cuda")[None] < b.count[:, None]
     assert bool((b.spots[..., 3][listed] == 0).all())
+
+
+def test_long_line_lists_either_side_of_the_limit_for_a_wave_each():
+    """A table of more than 2,048 lines: batches of which each orientation has a wave
+    of its own are leading parts of one that is too large for it."""
+    from diffsims_amd import engine
+    from diffsims_amd.crystallography import PhaseArrays
+
+    rng = np.random.default_rng(4)
+    pa = PhaseArrays((14.0, 15.0, 16.0), (90.0,) * 3, ["Si"] * 3, rng.uniform(0, 1, (3, 3)), np.ones(3),
+                     np.full(3, 0.4), "c")
+    tab = engine.build_phase_table(pa, 1.9, False)
+    assert uses_lines(tab) and tab.n_lines >= 2048
+    st = engine.SimSettings(max_excitation_error=0.01)
+    Rt = engine.rotation_matrices_to_device(rotations(12392, 5))
+    big = engine.simulate(tab, Rt, st, 1.9)
+    for n in (3000, 4500, 8500):
+        print(f"long line lists: {n} of {big.n}", flush=True)
+        part = engine.simulate(tab, Rt[:n].contiguous(), st, 1.9, cap=big.cap)
+        assert_same_batches(part, engine.SpotBatch(tab, big.idx[:n], big.spots[:n], big.count[:n],
+                                                   big.ncand[:n], big.maxI[:n], big.cap))
