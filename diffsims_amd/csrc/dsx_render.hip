@@ -1520,11 +1520,13 @@ __host__ __device__ constexpr int band_pix(int vec) { return 4 * vec * kBandThre
 template <int kR, bool kAligned, int kVec, bool kLong = false>
 __global__ __launch_bounds__(kBandThreads) void render_band_kernel(BandArgs b) {
   constexpr int kPix = band_pix(kVec);
-  // how the rows outside the band are dropped, as measured (render stage, us,
-  // row tests / flat index): 16,000 x 256 x 256 with R = 2 667 / 666, R = 4
-  // 660 / 646, R = 5 729 / 698, R = 6 701 / 731, R = 7 732 / 710 (231 x 201:
-  // 571 / 599), R = 8 909 / 850; long lists of 2,300 521 / 497
-  constexpr bool kFlat = kLong || kR == 4 || kR == 5 || kR == 8;
+  // how the rows outside the band are dropped: one comparison of the flat index
+  // (its terms in registers) or a test per row.  Render stage, time of the former
+  // over the latter, 144 x 144 to 512 x 512 with 65 and 259 spots: aligned rows R = 1
+  // to 3 0.98-1.03, R = 4 0.97-1.02, R = 5 0.95-1.02, R = 6 0.95-1.08, R = 7
+  // 0.93-1.04 (mean 0.98), R = 8 0.93-1.06 (0.95); others 0.97-1.03 up to R = 6, R = 7
+  // 0.94-1.05 (1.01), R = 8 0.93-1.04; long lists of 2,300 497 / 521 us
+  constexpr bool kFlat = kLong || (kAligned && kR >= 4);
   __shared__ __align__(16) racc_t s_acc[kPix + (kAligned ? 0 : 4)];
   __shared__ int2 s_ent[kPlanMax];
   __shared__ float s_tp[kR + 1];
