@@ -539,6 +539,35 @@ def test_long_list_kernel_equals_small_list_kernel(shape, sigma, clip, kw):
     assert torch.equal(fwd, pc)
 
 
+@pytest.mark.parametrize("shape,sigma", [((256, 256), 1.0), ((97, 131), 4.0)])
+def test_long_list_patterns_and_losses_are_the_same_bits_in_every_run(shape, sigma):
+    """Entries are numbered in list order whatever the waves' timing, in one range
+    of tiles and in several; gradients may differ in their last bits."""
+    import torch
+    from diffsims_amd import _lib
+    from diffsims_amd import differentiable as D
+    from tests import parity as P
+
+    print(f"tiles: repeated runs, {shape}, sigma {sigma}", flush=True)
+    spec = P.triclinic(20, 9, edges=(7, 12))
+    from diffsims_amd import engine
+    m = D.RefinementModel(P.to_arrays(spec), 1.6, engine.SimSettings(max_excitation_error=0.02), shape, sigma,
+                          3.2 / min(shape), clip_threshold=1e-2)
+    rng = np.random.default_rng(6)
+    leaves = D.leaf_parameters(P.to_arrays(spec), rng.uniform(0, 2 * np.pi, (600, 3)), requires_grad=False)
+    with torch.no_grad():
+        Rt, rec, xyz, B = D.forward_args(leaves)
+        t = m.tables(rec, xyz, B)
+        b = _copy_lists(m.spots(t, Rt), 1100)
+    target = torch.rand(shape, generator=torch.Generator("cuda").manual_seed(2), device="cuda") * 0.2
+    runs = []
+    for _ in range(5):
+        pat = torch.full((600, *shape), float("nan"), device="cuda")
+        runs.append((m.adjoint(t, Rt, b, _lib.ADJ_L2, target, True, pattern=pat)[0], pat))
+    for loss, pat in runs[1:]:
+        assert torch.equal(pat, runs[0][1]) and torch.equal(loss, runs[0][0])
+
+
 def test_long_lists_without_workspace_report_their_patterns():
     import ctypes
     import torch

@@ -413,26 +413,34 @@ def test_stream_handle_is_the_current_stream():
 @pytest.mark.parametrize("width", [1, 64, 130, 200])
 @pytest.mark.parametrize("axes", [False, True])
 def test_polar_rows_around_a_wave_are_written_to_their_width(width, axes):
-    """Lists of 0 to 130 spots (a wave takes 64 at a time) into buffers that held
-    other values: every entry of a row is its spot's or zero.  r and theta are the
-    FP64 values rounded to FP32, so within one unit of the last place."""
+    """Lists of 0 to 130 spots (a wave takes 64 at a time) into buffers that hold
+    other values: every entry of a row is its spot's or zero, and the number of
+    spots is the kept ones'.  r and theta are the FP64 values rounded to FP32, so
+    within one unit of the last place."""
     import torch
 
-    from diffsims_amd import engine
+    from diffsims_amd import _lib
 
+    L = _lib.load(require_gpu=True)
     counts = [0, 1, 63, 64, 65, 127, 128, 129, 130]
     print("polar rows", width, axes, flush=True)
     rng = np.random.default_rng(width)
     sp = rng.normal(size=(len(counts), 130, 4)).astype(np.float32)
-    dirty = [torch.full((len(counts), width), float("nan"), device="cuda") for _ in range(4)]
-    del dirty
-    kw = {}
+    spots = torch.from_numpy(sp).cuda()
+    count = torch.tensor(counts, dtype=torch.int32, device="cuda")
+    shape = (len(counts), width)
+    I = torch.full(shape, float("nan"), device="cuda")
+    n_out = torch.full((len(counts),), -1, dtype=torch.int32, device="cuda")
     if axes:
         ra, az = np.linspace(0, 3, 40), np.linspace(-np.pi, np.pi, 90)
-        kw = dict(radial_axes=ra, azimuthal_axes=az)
-    r, t, I = engine.polar_templates(torch.from_numpy(sp).cuda(),
-                                     torch.tensor(counts, dtype=torch.int32, device="cuda"), 130,
-                                     width=width, **kw)
+        d_ra, d_az = torch.from_numpy(ra).cuda(), torch.from_numpy(az).cuda()
+        r, t = (torch.full(shape, -1, dtype=torch.int32, device="cuda") for _ in range(2))
+        args = (_lib.ptr(d_ra), len(ra), _lib.ptr(d_az), len(az), None, None, _lib.ptr(r), _lib.ptr(t))
+    else:
+        r, t = (torch.full(shape, float("nan"), device="cuda") for _ in range(2))
+        args = (None, 0, None, 0, _lib.ptr(r), _lib.ptr(t), None, None)
+    _lib.check(L.dsx_polar_templates(_lib.ptr(spots), _lib.ptr(count), 130, len(counts), width, *args,
+                                     _lib.ptr(I), _lib.ptr(n_out), _lib.stream_handle()), "polar")
     r, t, I = r.cpu().numpy(), t.cpu().numpy(), I.cpu().numpy()
 
     def nearest(axis, v):
@@ -448,6 +456,7 @@ def test_polar_rows_around_a_wave_are_written_to_their_width(width, axes):
             er, et = nearest(ra, er), nearest(az, et)
             keep = (er < len(ra) - 1) & (et < len(az) - 1)
             er, et, eI = er[keep], et[keep], eI[keep]
+        assert int(n_out[o]) == len(er)
         m = min(len(er), width)
         for got, want in ((r, er), (t, et), (I, eI)):
             assert np.allclose(got[o, :m], want[:m], rtol=1.2e-7, atol=0)
