@@ -810,9 +810,10 @@ __global__ __launch_bounds__(kTileThreads, 4) void render_tiles_fwd_kernel(AdjAr
 // Chain rule of every spot gathered by the render adjoint: one block per
 // pattern (grid-stride), its spots spread over the block's threads; dL/dRt of
 // the pattern is a block sum, dL/d|F|^2 of the reflections global atomics,
-// dL/drec a per-block partial summed later in a fixed order.  Bound by FP64
-// arithmetic (about 20 % of the time are the atomics, 15 % the reads of the
-// rows): 4,096 patterns of the 500-atom cell under precession 3.50 ms with the
+// dL/drec a per-block partial summed later in a fixed order.  Bound by latency:
+// at 253 registers two waves per SIMD, 82 % of the time waiting, for the rows
+// (15 % of it), the atomics (20 %) and FP64 results, VALU busy 27 %.
+// 4,096 patterns of the 500-atom cell under precession 3.50 ms with the
 // library's roots and quotients, 3.08 with those of dsx_physics.h.  Reading the
 // rows a spot ahead (3.28) and more waves per SIMD (10.9, spills) are slower.
 constexpr int kChainThreads = 256;
@@ -1053,7 +1054,8 @@ __global__ __launch_bounds__(kSfaThreads) void structure_factor_adjoint_kernel(S
 // The same with a lane per atom (dsx_sf.h): runs of 4 rows.  Pass 1 forms F
 // and dF/dq of the run's rows, pass 2 adds every atom's terms in its own lane.
 // 1.56 million reflections of the 500-atom cell: 4.39 ms with a thread per
-// reflection (whose per-atom sums cross the wave 24 times), 2.56 here.
+// reflection (whose per-atom sums cross the wave 24 times), 2.56 here, VALU busy
+// 90 % (five of its registers are in scratch at 128).
 constexpr int kSfaRun = 4;
 
 // FP32 sums of the blocks meet in float atomics, whose rounding grows with the
@@ -1236,8 +1238,10 @@ static void launch_sfa_atoms(const SfAdjArgs &a, hipStream_t s) {
 using namespace dsx;
 
 // Workspace of the long lists' kernel, per block: large_block_ints(cap, H W)
-// ints, filled with the entries' records and rows and the first row of every
-// 64 listed spots (dsx_tiles.h); with gradients the chain-rule hand-over follows the
+// ints, filled with the first row of every 64 listed spots and as many entries'
+// records and rows as the rest holds (dsx_tiles.h): at least one tile's, and with
+// a pattern's pixels besides enough for wide boxes to be taken in few ranges;
+// with gradients the chain-rule hand-over follows the
 // blocks.  Chain-rule hand-over (the small-pattern kernel's whole workspace):
 // float4 gsum[n * cap] | int gcount[n] | (8-byte aligned) double
 // dpart[chain blocks][9].
@@ -1320,7 +1324,9 @@ static int launch_tiles(AdjArgs &a, int *work_d, long long work_ints, hipStream_
     set_error("dsx_render_adjoint: %lld tiles of a %dx%d pattern exceed the LDS", n_tiles, a.H, a.W);
     return DSX_EINVAL;
   }
-  // the widths and heights of the strip kernel that these patterns had before
+  // The shapes that are taken: 256 strips of 8,192 pixels (16,384 for rows above
+  // 8,192).  With sides of at most 32,767 and 2^22 pixels that is at most 16,384
+  // tiles, whose counters always fit above.
   const int strip_rows = std::min(a.H, (a.W <= 8192 ? 8192 : 16384) / a.W);
   if (strip_rows < 1 || (a.H + strip_rows - 1) / strip_rows > kAdjMaxStrips) {
     set_error("dsx_render_adjoint: a %dx%d pattern exceeds the sides taken", a.H, a.W);

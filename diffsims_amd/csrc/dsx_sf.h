@@ -21,10 +21,12 @@ namespace dsx {
 constexpr int kAtomThreads = 256;
 constexpr int kAtomWaves = kAtomThreads / kWave;
 constexpr int kAtomRows = 16;     // rows a wave stages at a time
-constexpr int kAtomMax = 512;     // atoms that fit the block's LDS
-constexpr int kAtomElems = 20;    // elements whose factors of the staged rows fit it
+// atoms and elements whose tables fit the 64 KB of LDS that a block has without
+// further ado; larger cells keep a thread per reflection
+constexpr int kAtomMax = 512;
+constexpr int kAtomElems = 20;
 
-// Sum over the lanes of each of n values, v[i] -> lanes i mod n.  Every step
+// Sum over the lanes of each of 16 values, v[i] -> lanes i mod 16.  Every step
 // halves the values: a lane keeps those with its bit of the index and hands
 // the others to its partner.
 template <int w>
@@ -39,16 +41,12 @@ __device__ __forceinline__ void fold_step(double *v, int lane) {
 }
 
 // (a loop over the widths is not unrolled and would index v at run time)
-template <int n>
-__device__ __forceinline__ double fold(double (&v)[n], int lane) {
-  static_assert(n == 16 || n == 32, "values");
-  if (n == 32) fold_step<(n == 32 ? 16 : 8)>(v, lane);
+__device__ __forceinline__ double fold(double (&v)[16], int lane) {
   fold_step<8>(v, lane);
   fold_step<4>(v, lane);
   fold_step<2>(v, lane);
   fold_step<1>(v, lane);
-  double s = v[0];
-  if (n == 16) s += __shfl_xor(s, 16, kWave);
+  const double s = v[0] + __shfl_xor(v[0], 16, kWave);
   return s + __shfl_xor(s, 32, kWave);
 }
 

@@ -473,6 +473,9 @@ __global__ __launch_bounds__(kSimThreads, sim_min_waves(kAvg, kLines)) void simu
 // With a line index a chunk is a line per thread (row interval, block prefix
 // sum), and its candidates are taken in steps.
 // The rows tested, their order and every value are those of simulate_kernel.
+// Held to 128 registers (four waves per SIMD) the line form keeps 9 of them in
+// scratch with 8 or 4 waves, 8 with 2 and 3 with 1; VALU busy 74 % on 4,096
+// orientations of 14,306 lines.
 // ---------------------------------------------------------------------------
 
 constexpr int kCoopPer = 4;                      // candidates per lane and step

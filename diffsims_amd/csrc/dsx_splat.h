@@ -44,8 +44,9 @@ __device__ __forceinline__ bool subpixel_box(float I, float X, float Y, float pr
 
 // subpixel_box with its logarithm and root in FP32 (about 60 instructions
 // instead of 250), where they decide: the radius is within 2e-5 sigma there,
-// so a box edge can only differ where an edge lies within box_margin of a
-// pixel (one spot in 500) or the box is tiny; those take the FP64 form.
+// so a box edge can only differ where one of the four edges lies within
+// box_margin of a pixel (8 box_margin of the spots: 0.37 % at 256 pixels, 0.57 %
+// at 512, sigma 1) or the box is tiny; those take the FP64 form.
 // Args carries pref, ep, clip, H, W and the host's log2_clip, two_s2_ln2
 // (2 sigma^2 ln 2), tiny_box (0.04 sigma^2) and box_margin.
 template <class Args>
@@ -60,7 +61,7 @@ __device__ __forceinline__ bool subpixel_box_fast(float I, float X, float Y, con
   const float y0 = Y - rad, y1 = Y + rad, x0 = X - rad, x1 = X + rad;
   const float near = fminf(fminf(fabsf(y0 - rintf(y0)), fabsf(y1 - rintf(y1))),
                            fminf(fabsf(x0 - rintf(x0)), fabsf(x1 - rintf(x1))));
-  // !(...) also sends infinities and subnormal amplitudes to the FP64 form
+  // !(...) also sends infinities and very small amplitudes to the FP64 form
   if (!(rad2 > a.tiny_box && rad2 < 1e8f && amp > 1e-30f && near > a.box_margin))
     return subpixel_box(I, X, Y, a.pref, a.ep, a.clip, a.H, a.W, lo, hi, xlo, xhi);
   lo = max(0, static_cast<int>(ceilf(y0)));

@@ -31,13 +31,16 @@
 // atomic per pixel and box, pixels kept in HBM between the maximum and the
 // read-out) took 19.6 ms for 4,096 patterns of 512 x 512 with 28,700 boxes
 // (43,000 listed spots) and their gradients, 11.7 ms here; forward only 9.95
-// and 6.4 ms: count 1.1, scatter 1.8, maximum 0.2 (a few tiles in ten can
-// hold it), tiles 3.2 ms, the gather 3.6 ms more.  Bound by VALU issue (about
-// 60 %): the factors of all 16 rows and columns of a tile are formed for boxes
-// of 5.4; the scatter by its 16-byte writes.  Measured and not kept: four
-// spots' loads in flight per lane in count and scatter (7.7 ms forward,
-// registers), 1,024-thread blocks (7.2), the gather's factors by recurrence
-// along a lane's four rows (no faster).
+// and 6.4 ms then (6.54 since): count 1.1, scatter 1.8, maximum 0.2 (a few tiles in ten can
+// hold it), tiles 3.2 ms, the gather 3.6 ms more.  Bound by VALU issue (78 % of
+// the SIMDs' cycles forward, 74 % with the gather, which keeps 12 registers in
+// scratch at 128): the factors of all 16 rows and columns of a tile are formed
+// for boxes of 5.4; the scatter by its 16-byte writes.  Small frames of few spots
+// in thin tiles (20 x 900, 480 spots) take up to 1.2 times as long as the strip
+// kernel did.  Measured and not kept: four spots' loads in flight per lane in
+// count and scatter (7.7 ms forward, registers), 1,024-thread blocks (7.2), the
+// next tile's records loaded ahead (6.7 and 12.5), the gather's factors by
+// recurrence along a lane's four rows (no faster).
 #pragma once
 
 #include "dsx_splat.h"
@@ -188,8 +191,10 @@ __device__ __forceinline__ void tiles_body(const Args &a, int *s_tiles, TileShar
   const int ntx = (W + kTileEdge - 1) / kTileEdge;
   const int n_tiles = ntx * ((H + kTileEdge - 1) / kTileEdge);
   // The list is split over the first `cw` waves in consecutive parts, each
-  // with counters of its own, so that a tile's entries (and the sums over
-  // them) are in list order whatever the waves' timing.
+  // with counters of its own, so that a tile's entries are in list order whatever
+  // the waves' timing, and patterns and losses the same bits in every run (the
+  // lanes of one LDS atomic are served in order, as on every run so far).  The
+  // gathered sums meet in float atomics and vary in their last bits.
   const int cw = a.count_waves, last = (cw - 1) * n_tiles;
   int *s_start = s_tiles;                // [cw][n_tiles]: first entry of (tile, part), tile-major
   int *s_u = s_tiles + cw * n_tiles;     // [n_tiles] bounds

@@ -103,7 +103,8 @@ int dsx_hkl_points_in_sphere(const int highest[3], const double metric[6], doubl
  *   F2_d[i] = |F|^2,  F_d[i] = {Re F, Im F} (F_d may be NULL).
  * f_e is evaluated and F accumulated in FP64 (the Lobato sums cancel by up to
  * two digits); the Debye-Waller exp is FP32, and so is the per-atom sincos
- * except for larger cells (more than 64 atoms, 24 in short tables: FP64).
+ * except for larger cells (from 24 atoms in short tables to 160 in long ones:
+ * FP64).
  * Atoms: elem_d int32 [n_atoms] (row into coeff_d), occ_d, B_d float
  * [n_atoms]; coeff_d double [n_elem][10] = {a1,b1,...,a5,b5};
  * scatter = DSX_SCATTER_*.
@@ -412,12 +413,15 @@ int dsx_render_fast_ragged(const float *spot_d, const long long *spot_off_d, con
  * cap, n, H, W, gradients) ints (gradients: nonzero when dRt_d is passed).
  * With cap <= dsx_render_max_spots() it is needed only for gradients
  * (per-spot sums handed from the render pass to the chain-rule pass; EINVAL
- * without it) and every status_d entry is 0.  With a larger cap it holds
- * the spots and tile lists of the patterns and their unscaled pixels until the
- * maximum is known when pattern_d is NULL, and with gradients n * cap per-spot
- * sums (EINVAL without it); when it is missing without gradients, or too small
- * for a pattern's lists, that pattern's status_d entry is 1.  At most 2^22
- * pixels per pattern.
+ * without it) and every status_d entry is 0.  With a larger cap it holds, per
+ * block, a record and a row for every tile (16 x 16 pixels) that a spot's box
+ * meets; a pattern with more of them is taken in ranges of tiles.  With
+ * gradients it also holds n * cap per-spot sums (EINVAL without it).  Shorter
+ * than dsx_render_adjoint_workspace_ints it is EINVAL for the call; without
+ * one (and without gradients) every status_d entry is 1 and the patterns are
+ * zeros, as for a single pattern with 2^31 records or more.  At most 2^22
+ * pixels per pattern, and 256 strips of 8,192 pixels (of 16,384 for widths above
+ * 8,192).
  * This entry point also serves as the sub-pixel renderer for such large
  * patterns (mode DSX_ADJ_FORWARD).
  */
