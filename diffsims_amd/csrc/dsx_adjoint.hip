@@ -1059,13 +1059,15 @@ __global__ __launch_bounds__(kSfaThreads) void structure_factor_adjoint_kernel(S
 constexpr int kSfaRun = 4;
 
 // FP32 sums of the blocks meet in float atomics, whose rounding grows with the
-// number of blocks: with 64 rows a block the gradients' error was 1.3 to 2 times
-// that of the thread-per-reflection kernel (256 rows a block) up to 64 k rows
-// (60,000 rows x 48 atoms 2.9e-7 -> 5.1e-7 of the norm).  A block takes at least
-// 256 rows, with as many waves as its LDS holds: 2.9e-7, and 84 -> 44 us there,
-// 17,332 rows x 48 atoms 35 -> 29; 4,614 rows x 24 atoms 1.4e-7 -> 1.9e-7 -> 1.2e-7,
-// where 18.5 us (64 rows) become 25.5 (a thread per reflection: 48).
-constexpr int kSfaAtomRows = 256;
+// number of blocks: with 64 rows a block the gradients' error was 1.1 to 2 times
+// that of the thread-per-reflection kernel (256 rows a block) up to 64 k rows.
+// 60,000 rows x 48 atoms: 2.9e-7 of the norm there, 5.1e-7 with 64 rows and 2.9e-7
+// with 256, as many waves as the block's LDS holds; 84 -> 44 us, 17,332 x 48 35 -> 29.
+// Small tables take fewer rows, where the error stays below that kernel's and
+// more CUs work: 4,614 x 24 1.35e-7 with a thread per reflection; 1.12e-7 with 256
+// rows in 25.5 us, 1.25e-7 with 192 in 21.7, 1.40e-7 with 128 in 18.7; 3,000 x 24
+// 1.38e-7; 1.11e-7, 1.13e-7 and 1.22e-7; 8,000 x 24 1.60e-7; 1.38e-7, 1.49e-7, 1.64e-7.
+static int sfa_atom_rows(int n) { return n <= 4096 ? 128 : n <= 8192 ? 192 : 256; }
 
 template <int kWaves>
 __global__ __launch_bounds__(kWaves *kWave, 4) void structure_factor_adjoint_atoms_kernel(SfAdjArgs a,
@@ -1228,7 +1230,7 @@ static bool sfa_atoms_fit(int n_atoms, int n_elem, int waves) {
 
 template <int kWaves>
 static void launch_sfa_atoms(const SfAdjArgs &a, hipStream_t s) {
-  const int rows = atom_rows_per_block(a.n, kWaves, kSfaAtomRows);
+  const int rows = atom_rows_per_block(a.n, kWaves, sfa_atom_rows(a.n));
   hipLaunchKernelGGL(structure_factor_adjoint_atoms_kernel<kWaves>, dim3((a.n + rows - 1) / rows),
                      dim3(kWaves * kWave), sfa_atoms_lds(a.n_atoms, a.n_elem, kWaves), s, a, rows);
 }
@@ -1631,8 +1633,11 @@ extern "C" int dsx_structure_factor_adjoint(const int *hkl_d, int n, const doubl
   a.dB = dB_d;
   a.drec = drec_d;
   if (atoms_per_lane_adjoint(n, n_atoms, n_elem)) {
-    if (sfa_atoms_fit(n_atoms, n_elem, 16))
+    const int waves = sfa_atom_rows(n) / kAtomRows;  // 8, 12 or 16: a turn of the block's rows
+    if (waves >= 16 && sfa_atoms_fit(n_atoms, n_elem, 16))
       launch_sfa_atoms<16>(a, as_stream(stream));
+    else if (waves >= 12 && sfa_atoms_fit(n_atoms, n_elem, 12))
+      launch_sfa_atoms<12>(a, as_stream(stream));
     else if (sfa_atoms_fit(n_atoms, n_elem, 8))
       launch_sfa_atoms<8>(a, as_stream(stream));
     else

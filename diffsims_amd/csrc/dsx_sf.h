@@ -185,7 +185,7 @@ static inline int atom_rows_per_block(int n, int waves, int least) {
 //   17,332     11 | 8     13 | 8    17 | 8    22 | 8    22 | 12   26 | 12   31 | 12
 //              38 | 28    47 | 28   65 | 28   82 | 28   83 | 37   100 | 37  122 | 37
 //   4,614      10 | 7     12 | 7    17 | 7    21 | 7    22 | 9    26 | 9    31 | 9
-//              35 | 25    44 | 25   62 | 25   80 | 25   81 | 34   98 | 34   120 | 34
+//              35 | 22    44 | 22   62 | 22   80 | 22   81 | 30   98 | 30   120 | 30
 // (first line forward, second adjoint; at 400,000 rows forward 129 atoms 96 | 113,
 // 160 116 | 114, 193 138 | 138, 500 346 | 240, at 195,590 96 atoms 41 | 41 and 129
 // 53 | 52; adjoint 129 atoms 375 | 319 and 500 1,398 | 634.)

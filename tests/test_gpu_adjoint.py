@@ -648,6 +648,7 @@ SF_SIZES = [(1, 24, 3, "lobato"), (15, 23, 3, "lobato"), (17, 48, 20, "xtables")
             (1003, 512, 20, "lobato"), (700, 513, 5, "lobato"), (24577, 24, 2, "lobato"),
             (24576, 30, 2, None), (65537, 33, 1, "lobato"), (65536, 32, 1, "lobato"), (33000, 130, 4, "xtables"),
             (65537, 31, 2, "lobato"), (70001, 75, 2, "lobato"), (70001, 76, 2, "lobato"),
+            (4096, 40, 4, "lobato"), (4097, 64, 20, "lobato"), (8192, 200, 18, None), (8193, 24, 2, "lobato"),
             (131073, 95, 3, "xtables"), (131073, 96, 3, "xtables"), (262145, 159, 2, "lobato"),
             (262145, 160, 2, "lobato"), (262145, 79, 2, "lobato"), (262145, 80, 2, "lobato")]
 
