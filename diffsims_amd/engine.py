@@ -61,23 +61,35 @@ SPLAT_MAX_PIXELS = 256 * 256
 # Widths that are not a multiple of 4: the band writer's plan lists patterns
 # whose maximum could be in many tiles for the splat kernel, which then runs
 # behind the writer with most of the GPU idle.  Time with bands over the splat
-# kernel, lists of 65, 146 and 259 spots of the 40-atom cell: 300 patterns 1.05-2.0
-# at any size up to 300 x 257, 800 and more 0.5-0.95 (231 x 201, 300 x 257); taps of
-# radius 7 and 8 on 65 x 67, 101 x 99 and 144 x 145: 800 patterns 1.0-1.6, 1,500
-# 0.9-1.4, from 2,500 on 0.5-0.9 unless a list holds a spot per 8 pixels (65 x 67:
-# 1.2-1.3 at any number); 64 x 1,021 1.3-1.5 up to 1,500.
+# kernel, lists of 65, 146 and 259 spots of the 40-atom cell, beyond what
+# SPLAT_MAX_PATTERNS decides:
+# up to 700 patterns of more than SPLAT_MAX_PIXELS pixels 0.25-0.95 (247 x 298 to
+# 512 x 510), but with about a pattern per CU, which the splat kernel renders in
+# one turn, 0.9-1.2 (300 patterns of up to 401 x 259); 1,021 x 67 1.1-1.9 with taps
+# of radius 7 and with longer lists, 0.8-1.2 with sparse ones;
+# 800 patterns and more 0.5-0.95 (231 x 201, 300 x 257); taps of radius 7 and 8 on
+# 65 x 67, 101 x 99 and 144 x 145: 800 patterns 1.0-1.6, 1,500 0.9-1.4, from 2,500 on
+# 0.5-0.9 unless a list holds a spot per 8 pixels (65 x 67: 1.2-1.3 at any number);
+# 64 x 1,021 1.3-1.5 up to 1,500, and with a spot per 105 pixels 1.1-1.4 at 2,500 and
+# 5,000 (sparser lists 0.7-1.2).
 ODD_MIN_PATTERNS_WIDE_TAPS = 1536
 ODD_SMALL_PIXELS = 24000
+ODD_NARROW = 80
+ODD_NARROW_PIXELS_PER_SPOT = 165
+ODD_LONG_PIXELS_PER_SPOT = 110
 
 
 def _splat_pays_at_odd_width(n: int, height: int, width: int, cap: int, radius: int) -> bool:
+    pixels, narrow = height * width, min(height, width) <= 10 * radius
     if n < SPLAT_MAX_PATTERNS:
-        return True
+        return (narrow or 192 <= n < 400 and pixels <= 2 * SPLAT_MAX_PIXELS
+                or min(height, width) <= ODD_NARROW and ODD_NARROW_PIXELS_PER_SPOT * cap >= pixels)
     if radius < 6:
         return False
-    if min(height, width) <= 10 * radius:
-        return n < 2000 or 8 * cap >= height * width
-    return n < ODD_MIN_PATTERNS_WIDE_TAPS and height * width <= ODD_SMALL_PIXELS
+    if narrow:
+        return (n < 2000 or 8 * cap >= pixels or n < 6000 and pixels > ODD_SMALL_PIXELS
+                and ODD_LONG_PIXELS_PER_SPOT * cap >= pixels)
+    return n < ODD_MIN_PATTERNS_WIDE_TAPS and pixels <= ODD_SMALL_PIXELS
 
 
 def fast_renderer(n: int, height: int, width: int, cap: Optional[int] = None,

@@ -316,11 +316,16 @@ def test_fast_renderer_choice():
 
 
 @pytest.mark.parametrize("n,shape,cap,radius,bands", [
-    (767, (300, 257), 292, 4, False), (768, (300, 257), 292, 4, True),     # few patterns
-    (767, (300, 256), 292, 4, True),                                       # whole 16-byte rows
+    (191, (300, 257), 292, 4, True), (192, (300, 257), 292, 4, False),     # about one to a CU
+    (399, (300, 257), 292, 4, False), (400, (300, 257), 292, 4, True),
+    (300, (401, 327), 292, 4, True), (5, (512, 510), 648, 7, True),        # large patterns
+    (300, (300, 256), 292, 4, True),                                       # whole 16-byte rows
+    (767, (1021, 67), 415, 2, False), (767, (1021, 67), 414, 2, True),     # narrow, few patterns
+    (767, (1021, 67), 292, 7, False),
     (768, (101, 99), 292, 5, True), (1535, (101, 99), 292, 6, False),      # wide taps, small patterns
     (1536, (101, 99), 292, 6, True), (768, (231, 201), 292, 8, True),
     (1999, (1021, 67), 400, 8, False), (2000, (1021, 67), 400, 8, True),   # narrow patterns
+    (5999, (1021, 67), 622, 8, False), (5999, (1021, 67), 621, 8, True), (6000, (1021, 67), 648, 8, True),
     (12000, (65, 67), 544, 7, True), (12000, (65, 67), 545, 7, False),     # a spot per 8 pixels
 ])
 def test_fast_renderer_choice_at_odd_widths(n, shape, cap, radius, bands):
