@@ -626,8 +626,8 @@ def large_precession_leg(dev, n_chunks):
                      "frac": round(achieved / HBM_PEAK_GBS, 5),
                      "traffic": None,
                      "note": "algorithmic bytes: the spot lists read once and the shared target. "
-                             "The kernel is bound by the matrix and VALU work per spot and the "
-                             "latency of its per-tile lists, not by HBM"},
+                             "The kernel is bound by VALU issue (profiles/cases_counters.md), "
+                             "not by HBM"},
         "cpu_baseline": cpu_baseline_entry(
             1 / cdt, "1 orientation, FP64 NumPy restatement of the reference loop (F of the "
             "intersecting rows, precession shape factor) incl. sub-pixel render, forward only",
