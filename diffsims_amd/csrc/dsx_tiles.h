@@ -108,8 +108,9 @@ __device__ __forceinline__ tile_f4 tile_pixels(TileShared &sh, const float4 *rec
   for (int e = e0; e < e1; e += kWave) {
     tile_stage(sh, rec, erow, e, e1, lane, wid);
     const int m = min(kWave, e1 - e);
+    int k = 0;
 #pragma unroll 2
-    for (int k = 0; k < m; k += 8) {  // records past m have zero amplitude and mask
+    for (; k + 4 < m; k += 8) {  // records past m have zero amplitude and mask
       const float4 v = sh.stage[wid][k + sub], w = sh.stage[wid][k + 4 + sub];
       const int mv = __float_as_int(v.w), mw = __float_as_int(w.w);
       const float av = v.z * tile_factor(fp - v.y, c, mv, pos);
@@ -118,6 +119,12 @@ __device__ __forceinline__ tile_f4 tile_pixels(TileShared &sh, const float4 *rec
       const float bw = tile_factor(fp - w.x, c, mw, 16 + pos);
       acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc, 0, 0, 0);
       odd = __builtin_amdgcn_mfma_f32_16x16x4f32(aw, bw, odd, 0, 0, 0);
+    }
+    if (k < m) {
+      const float4 v = sh.stage[wid][k + sub];
+      const int mv = __float_as_int(v.w);
+      const float av = v.z * tile_factor(fp - v.y, c, mv, pos);
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, tile_factor(fp - v.x, c, mv, 16 + pos), acc, 0, 0, 0);
     }
     if (e1 - e0 > kWave) {  // uniform
 #pragma unroll
