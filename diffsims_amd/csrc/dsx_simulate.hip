@@ -770,9 +770,10 @@ __global__ __launch_bounds__(kCoopWaves *kWave, 4) void simulate_coop_kernel(Sim
 // of the candidates (rows per line times sin phi of 0.3 and more) the per-row
 // threshold saves a quarter of them and one wave is ahead at any number (20,000:
 // 0.66-0.91; 500-atom cell 14,622 us against 20,271).  The full sweep shares each row:
-// they cross at 3,900-4,200 with 6,212 to 28,800 rows, at 5,000-6,100 with 484.
+// they cross at 3,900-4,200 with 6,212 to 28,800 rows, at 5,000-6,100 with 484 and
+// beyond 6,144 with 250 (9.4 us | 12.8 there).
 static int coop_waves(int n_orient, int n_refl, int n_lines, double me, double g_max, double sin_phi) {
-  double limit = n_refl < 1024 ? 5120 : 4096;
+  double limit = n_refl < 384 ? 6144 : n_refl < 1024 ? 5120 : 4096;
   if (n_lines > 0) {
     const double rows = static_cast<double>(n_refl) / n_lines;
     const double c = g_max > 0.0 ? rows * (1.5 * me / g_max + sin_phi) : 0.0;
