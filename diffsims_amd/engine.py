@@ -69,7 +69,8 @@ SPLAT_MAX_PIXELS = 256 * 256
 # of radius 7 and with longer lists, 0.8-1.2 with sparse ones;
 # 800 patterns and more 0.5-0.95 (231 x 201, 300 x 257); taps of radius 7 and 8 on
 # 65 x 67, 101 x 99 and 144 x 145: 800 patterns 1.0-1.6, 1,500 0.9-1.4, from 2,500 on
-# 0.5-0.9 unless a list holds a spot per 8 pixels (65 x 67: 1.2-1.3 at any number);
+# 0.35-1.0 (1.2-1.3 where a list of the cell holds a spot per 7 pixels of 65 x 67,
+# 0.3-0.5 with log-normal intensities there and on 33 x 31);
 # 64 x 1,021 1.3-1.5 up to 1,500, and with a spot per 105 pixels 1.1-1.4 at 2,500 and
 # 5,000 (sparser lists 0.7-1.2).
 ODD_MIN_PATTERNS_WIDE_TAPS = 1536
@@ -87,8 +88,8 @@ def _splat_pays_at_odd_width(n: int, height: int, width: int, cap: int, radius: 
     if radius < 6:
         return False
     if narrow:
-        return (n < 2000 or 8 * cap >= pixels or n < 6000 and pixels > ODD_SMALL_PIXELS
-                and ODD_LONG_PIXELS_PER_SPOT * cap >= pixels)
+        return n < 2000 or (n < 6000 and pixels > ODD_SMALL_PIXELS
+                            and ODD_LONG_PIXELS_PER_SPOT * cap >= pixels)
     return n < ODD_MIN_PATTERNS_WIDE_TAPS and pixels <= ODD_SMALL_PIXELS
 
 
@@ -110,14 +111,16 @@ def fast_renderer(n: int, height: int, width: int, cap: Optional[int] = None,
 # Fast rendering of long lists (more than dsx_render_max_spots() spots): the plan
 # and band writer (dsx_render_fast_long) cost in proportion to the spots, the
 # windowed renderer (dsx_render_fast_large) to the pixels.  Time of the former
-# over the latter, 1 to 1,500 patterns with taps of radius 1 to 8, lists filled to
-# 60-80 % with |F|^2 of random structures: 0.1-0.5 at a capacity of one spot per
-# 12 pixels; at 1 per 8 0.3-1.0 (129 x 128, 170 x 171) and 0.2-0.8 (256 x 256,
-# 301 x 203); at 1 per 6.7 0.3-1.26 and 0.25-1.0; at 1 per 4 0.6-2.0 and more.
-# (Lists of equal intensities, whose maximum can be anywhere, come out level at
-# 1 per 12 and 1.2-1.9 times slower at 1 per 6.7.)
-LONG_PIXELS_PER_SPOT = 6
-LONG_PIXELS_PER_SPOT_SMALL = 8      # below LONG_SMALL_PIXELS pixels
+# over the latter, 1 to 1,500 patterns with taps of radius 2 to 8, by pixels per
+# spot of the capacity.  Lists of real cells (default_cap, filled to 49 % below 4,096
+# expected spots and to 78 % above): 6.1-7.5 0.24-0.75, 5.5 (170 x 171) 0.33-0.61, 4.0
+# (200 x 200) 0.75-1.16, 3.1 (129 x 128) 0.64-1.33, 2.9 (170 x 171) 0.95-1.45, 1.6
+# 2.1-3.0.  Random positions with |F|^2 of random structures, filled to 60-80 %:
+# 0.3-1.26 at 6.7, 0.45-1.4 at 4.8 (256 x 256, 301 x 203) and 0.39-1.7 there on
+# 129 x 128.  Log-normal intensities 0.2-0.5 at 4.7 to 6.4; equal ones, whose
+# maximum can be anywhere, level at 12 and 1.2-1.9 at 6.7.
+LONG_PIXELS_PER_SPOT = 4.5
+LONG_PIXELS_PER_SPOT_SMALL = 5      # below LONG_SMALL_PIXELS pixels
 LONG_SMALL_PIXELS = 32768
 
 

@@ -362,9 +362,9 @@ def test_long_lists_dispatch_and_limits():
     assert engine.long_renderer(2000, 256, 256, 4)
     assert not engine.long_renderer(2000, 128, 128, 4)   # the dense renderers
     assert not engine.long_renderer(30000, 256, 256, 4)  # dsx_render_fast_large
-    # dense lists stay with it: a spot per 6 pixels, per 8 of small patterns
-    assert engine.long_renderer(10922, 256, 256, 4) and not engine.long_renderer(10923, 256, 256, 4)
-    assert engine.long_renderer(2064, 129, 128, 8) and not engine.long_renderer(2065, 129, 128, 8)
+    # dense lists stay with it: a spot per 4.5 pixels, per 5 of small patterns
+    assert engine.long_renderer(7288, 200, 164, 4) and not engine.long_renderer(7289, 200, 164, 4)
+    assert engine.long_renderer(3302, 129, 128, 8) and not engine.long_renderer(3303, 129, 128, 8)
     # render_spots on both sides of the lists it takes: the same pixels
     spots, cnt = _spot_lists(6, 1500, 200, 160, 1400, seed=2)
     a = engine.render_spots(spots, cnt, 1500, (200, 160), 1.0, 1.0)
@@ -495,7 +495,7 @@ def test_long_lists_gathered_in_a_few_rows(shape, length):
         assert np.abs(o - r).max() <= LONG_TOL
 
 
-@pytest.mark.parametrize("shape,cap", [((129, 128), 2064), ((200, 164), 5466)])
+@pytest.mark.parametrize("shape,cap", [((129, 128), 3302), ((200, 164), 7288)])
 def test_both_sides_of_the_density_line_give_the_same_pixels(shape, cap):
     # one list either side of the capacity from which the windowed renderer takes it
     import torch

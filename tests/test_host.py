@@ -326,7 +326,7 @@ def test_fast_renderer_choice():
     (1536, (101, 99), 292, 6, True), (768, (231, 201), 292, 8, True),
     (1999, (1021, 67), 400, 8, False), (2000, (1021, 67), 400, 8, True),   # narrow patterns
     (5999, (1021, 67), 622, 8, False), (5999, (1021, 67), 621, 8, True), (6000, (1021, 67), 648, 8, True),
-    (12000, (65, 67), 544, 7, True), (12000, (65, 67), 545, 7, False),     # a spot per 8 pixels
+    (1999, (33, 31), 248, 7, False), (2000, (33, 31), 248, 7, True),       # dense and narrow
 ])
 def test_fast_renderer_choice_at_odd_widths(n, shape, cap, radius, bands):
     from diffsims_amd.engine import fast_renderer
